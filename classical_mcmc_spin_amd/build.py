@@ -2,7 +2,7 @@
 
 The shared library lands next to this file so it travels with the source tree.
 Run ``python -m classical_mcmc_spin_amd.build`` or call :func:`build`.
-Objects compile in parallel; the persistent kernel is compiled once per
+Objects compile in parallel; the persistent kernels are compiled once per
 sites-per-thread value (-DCSL_SPT=n).
 """
 from __future__ import annotations
@@ -23,7 +23,7 @@ LIB_PATH = os.path.join(HERE, LIB_NAME)
 HIP_UNITS = [("csl_kernels.hip", "", []), ("csl_capi.hip", "", []), ("csl_mixed.hip", "", []), ("csl_adjoint.hip", "", []),
              ("csl_dssf.hip", "", []), ("csl_spectrum.hip", "", []), ("csl_quench.hip", "", []),
              ("csl_dopri5.hip", "", []), ("csl_partition.hip", "", []), ("csl_mixed_persist.hip", "", [])] + [
-    ("csl_persistent.hip", f"_spt{n}", [f"-DCSL_SPT={n}"]) for n in (1, 2, 3, 4, 6)]
+    (src, f"_spt{n}", [f"-DCSL_SPT={n}"]) for src in ("csl_persistent.hip", "csl_trajectory.hip") for n in (1, 2, 3, 4, 6)]
 CXX_UNITS = ["gpu_api_shim.cpp", "mixed_gpu_api_shim.cpp"]
 
 HIPCC_FLAGS = [

@@ -402,20 +402,36 @@ TuneVal pick_persistent(const csl_lattice* h, size_t B, int block_req) {
     auto it = h->tune.find(batch_class(B));
     if (it != h->tune.end()) return it->second;
     // heuristic: two LDS buffers (one barrier per stage) and compile-time
-    // stages, the shape whose busiest SIMD carries the fewest wave-sized
-    // units of sites (a stage ends when that SIMD is done), ties: the fewest
-    // sites per thread
+    // stages.  Atom-major shapes first (24x24, one trajectory: 3.1 us a step
+    // against 5.8 for the best other shape); among them the one whose busiest
+    // SIMD carries the fewest wave-sized units of sites (a stage ends when
+    // that SIMD is done); ties: at most three waves per SIMD, whose larger
+    // VGPR budget holds three and more sites without spills (513
+    // trajectories of 36x36: 768 x 4 6.1 ms, 1024 x 3 6.7 ms per 512 steps),
+    // then the fewest sites per thread.
     const int fl = csl::kPersistDoubleBuffer | csl::kPersistUnrollStages;
     const TuneVal* best = nullptr;
-    int best_share = 0;
+    std::array<int, 4> best_rank{};
+    auto atom_major = [&](const TuneVal& c) {
+        return (csl::persistent_variant(h->L, c.block, c.spt, c.flags) & csl::kVariantAtomMajor) != 0;
+    };
     for (const auto& c : cands) {
         if (c.flags != fl) continue;
-        const int sh = simd_share(h->L, c.block, c.spt, c.flags);
-        if (!best || sh < best_share || (sh == best_share && c.spt < best->spt)) {
+        const std::array<int, 4> rank{atom_major(c) ? 0 : 1, simd_share(h->L, c.block, c.spt, c.flags),
+                                      c.spt >= 3 && c.block > 768 ? 1 : 0, c.spt};
+        if (!best || rank < best_rank) {
             best = &c;
-            best_share = sh;
+            best_rank = rank;
         }
     }
+    // several trajectories per CU: two sites per thread share a wave's
+    // per-step work (records, field rows, barriers); with one trajectory per
+    // CU its latency counts and one site per thread is faster (12x12: 1024
+    // trajectories 1.06 against 1.34 ms per 256 steps, one trajectory 0.53
+    // against 0.44 ms)
+    if (best && best->spt == 1 && best_rank[0] == 0 && B >= 2 * size_t(h->n_cu))
+        for (const auto& c : cands)
+            if (c.flags == fl && c.spt == 2 && atom_major(c)) return c;
     if (best) return *best;
     for (auto& c : cands)
         if (c.flags == csl::kPersistDoubleBuffer) return c;

@@ -352,6 +352,16 @@ size_t persistent_lds_bytes(const LatDev& L, int block, bool dbuf) {
 namespace {
 hipError_t persistent_dispatch(const LatDev& L, const PersistArgs& A, int block, int spt, int flags,
                                hipStream_t st, int* occ) {
+    if (persistent_variant(L, block, spt, flags) & kVariantAtomMajor) {
+        switch (spt) {
+            case 1: return launch_trajectory_spt<1>(L, A, block, st, occ);
+            case 2: return launch_trajectory_spt<2>(L, A, block, st, occ);
+            case 3: return launch_trajectory_spt<3>(L, A, block, st, occ);
+            case 4: return launch_trajectory_spt<4>(L, A, block, st, occ);
+            case 6: return launch_trajectory_spt<6>(L, A, block, st, occ);
+            default: return hipErrorInvalidValue;
+        }
+    }
     const bool dbuf = flags & kPersistDoubleBuffer;
     const size_t lds = persistent_lds_bytes(L, block, dbuf);
     switch (spt) {

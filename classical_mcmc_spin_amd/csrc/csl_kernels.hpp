@@ -290,16 +290,29 @@ __host__ __device__ inline void atom_major_tile(int nwaves, int n_atoms, int U, 
     units = q + int((extra >> i_w) & 1u);
 }
 
+// LDS of the atom-major kernel (csl_trajectory.hip) with its records and
+// pulse envelopes handled `chunk` steps at a time.
+inline size_t trajectory_lds_bytes(const LatDev& L, int block, int chunk) {
+    return sizeof(double) * (6 * size_t(L.NP) + 73 * size_t(L.n_atoms) + size_t(chunk) * (12 + 4 * size_t(block / kWave)));
+}
+constexpr size_t kLdsBytes = 160 * 1024;  // LDS of a CU
+// Steps handled together: the most, up to 8, whose tables fit (0: none).
+inline int trajectory_chunk(const LatDev& L, int block) {
+    for (int c = 8; c >= 1; c >>= 1)
+        if (trajectory_lds_bytes(L, block, c) <= kLdsBytes) return c;
+    return 0;
+}
+
 inline int persistent_variant(const LatDev& L, int block, int spt, int flags) {
     if (flags & kPersistMulti) return 0;
     const bool dbuf = flags & kPersistDoubleBuffer, unroll = flags & kPersistUnrollStages;
     if (!(unroll && dbuf && L.uniform && L.site_uniform && !L.has_onsite && L.full_coord &&
           L.zmax == zmax_bucket(L.zmax)))
         return 0;
-    // atom-major: whole waves per sublattice, each with 1..spt units
+    // atom-major: whole waves per sublattice, each with spt or spt - 1 units
     const int U = L.npad / kWave, wpa = block / (L.n_atoms * kWave);
-    const bool am = L.npad % kWave == 0 && block % (L.n_atoms * kWave) == 0 && wpa * spt >= U && wpa <= U &&
-                    wpa <= 32;
+    const bool am = L.npad % kWave == 0 && block % (L.n_atoms * kWave) == 0 && wpa > 0 && (U + wpa - 1) / wpa == spt &&
+                    wpa <= 32 && trajectory_chunk(L, block) > 0;
     return kVariantFieldOnly | (am ? kVariantAtomMajor : 0);
 }
 
@@ -324,6 +337,16 @@ template <> hipError_t launch_persistent_spt<2>(const LatDev&, const PersistArgs
 template <> hipError_t launch_persistent_spt<3>(const LatDev&, const PersistArgs&, int, int, size_t, hipStream_t, int*);
 template <> hipError_t launch_persistent_spt<4>(const LatDev&, const PersistArgs&, int, int, size_t, hipStream_t, int*);
 template <> hipError_t launch_persistent_spt<6>(const LatDev&, const PersistArgs&, int, int, size_t, hipStream_t, int*);
+
+// The kernel of the atom-major shapes (csl_trajectory.hip, one object per
+// sites-per-thread value).
+template <int SPT>
+hipError_t launch_trajectory_spt(const LatDev& L, const PersistArgs& A, int block, hipStream_t st, int* occupancy);
+template <> hipError_t launch_trajectory_spt<1>(const LatDev&, const PersistArgs&, int, hipStream_t, int*);
+template <> hipError_t launch_trajectory_spt<2>(const LatDev&, const PersistArgs&, int, hipStream_t, int*);
+template <> hipError_t launch_trajectory_spt<3>(const LatDev&, const PersistArgs&, int, hipStream_t, int*);
+template <> hipError_t launch_trajectory_spt<4>(const LatDev&, const PersistArgs&, int, hipStream_t, int*);
+template <> hipError_t launch_trajectory_spt<6>(const LatDev&, const PersistArgs&, int, hipStream_t, int*);
 
 size_t persistent_lds_bytes(const LatDev& L, int block, bool dbuf);
 bool persistent_spt_supported(int spt);

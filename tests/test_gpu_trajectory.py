@@ -1,0 +1,67 @@
+"""The atom-major persistent kernel (k_trajectory) at the edges of its tiles
+and chunks against the oracle: lattices whose last unit of 64 cells is nearly
+empty or exactly full, 3, 6 and 12 bonds per site, 2 and 16 sublattices,
+damping, step counts around the chunk of 8 steps and record intervals below,
+at and above it.
+
+Tolerance: a step rounds each component some thirty times (27 bond products,
+the cross product, the updates), so 41 steps of unit spins stay within
+41 * 30 * 2.2e-16 = 3e-13 of another order of the same sums; 1e-12 allows for
+the growth along the trajectory (less than a factor of two over 0.41 units of
+time).
+"""
+import numpy as np
+import pytest
+
+from classical_mcmc_spin_amd import GPULattice, model
+from helpers import random_state
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+DT = 0.01
+
+
+def _kitaev(**kw):
+    return model.build_kitaev_honeycomb(field_strength=0.1, field_direction=(1.0, 1.0, 1.0), **kw)
+
+
+CELLS = {
+    "z3_5x3": (lambda: _kitaev(), (5, 3, 1)),            # 15 of 64 cells
+    "z3_8x8": (lambda: _kitaev(), (8, 8, 1)),            # one full unit
+    "z3_13x5": (lambda: _kitaev(), (13, 5, 1)),          # 65 cells: a second unit with one cell
+    "z3_23x25": (lambda: _kitaev(), (23, 25, 1)),        # 9 units over uneven waves
+    "z12_6x7": (lambda: _kitaev(J2_A=0.1, J2_B=-0.07, J3=0.05), (6, 7, 1)),
+    "z6_pyro2": (lambda: model.build_pyrochlore_conventional(field_strength=0.1), (2, 2, 2)),
+}
+
+
+@pytest.mark.parametrize("name", sorted(CELLS))
+@pytest.mark.parametrize("steps,every,alpha", [(1, 1, 0.0), (8, 1, 0.03), (41, 1, 0.0), (41, 3, 0.0), (23, 11, 0.03)])
+def test_trajectory_edges(oracle, name, steps, every, alpha):
+    build, dims = CELLS[name]
+    uc = build()
+    lat = model.Lattice(uc, *dims)
+    s = random_state(lat, 77)
+    f = np.zeros((lat.N_atoms, 3))
+    f[:, 0] = 1.0
+    fd = np.einsum("aij,aj->ai", lat.frames, f).reshape(-1)
+    T1 = (steps + 0.5) * DT
+    tp = np.array([[0.0, 0.2], [0.1, 0.0], [0.0, 0.0]])
+    am = np.array([[0.5, 0.25], [0.5, 0.0], [0.0, 0.0]])
+    print(f"[trajectory] {name} steps {steps} every {every} alpha {alpha}", flush=True)
+    with GPULattice(lat) as gl:
+        gl.set_damping(alpha)
+        gl.set_pulse(np.concatenate([fd, fd]), 0.5, 0.1, 3.0, 0.0, 0.0)
+        r = gl.integrate_batched(s, tp, am, 0.0, T1, DT, save_interval=every, tgrid="boost", want_final=True)
+        assert gl.last_launch_config()["atom_major"]
+    o = oracle.OracleLattice(uc, *dims)
+    o.set_alpha(alpha)
+    keep = sorted(set(range(0, steps, every)) | {steps})
+    for b in range(3):
+        o.set_pulse(f * (am[b, 0] / 0.5), tp[b, 0], f * (am[b, 1] / 0.5), tp[b, 1], 0.5, 0.1, 3.0)
+        ref = o.integrate_md(s.reshape(-1), 0.0, T1, DT)
+        assert r["mags"].shape[0] == len(keep)
+        assert np.max(np.abs(r["mags"][:, b] - ref["mags"][keep])) <= TOL
+        assert np.max(np.abs(r["energy"][:, b] - ref["energy"][keep])) <= TOL
+        assert np.max(np.abs(r["final"][b] - ref["final"].reshape(-1, 3))) <= TOL
