@@ -1410,6 +1410,50 @@ std::vector<int> transpose_offsets(const EllHost& e23, const EllHost& e32, size_
     return off;
 }
 
+// The persistent kernels' bond matrices (MixDev::jpad, j32pad): kind 23
+// padded to zm bonds per sublattice, then kind 22 padded to z22, then one
+// zero matrix for the padding slots of kind 32 and, where kind 32 has no
+// twins among kind 23, its own matrices transposed to 3x8.
+struct PaddedMats {
+    std::vector<double> mats;
+    std::vector<int> off32;
+    int j22off = 0, z22 = 6, zm = 4;
+};
+
+PaddedMats pad_mats(const EllHost& e22, const EllHost& e23, const EllHost& e32, const std::vector<int>& twins, int A2,
+                    int A3, bool tt) {
+    PaddedMats P;
+    // lattices with SU(3)-SU(3) bonds have one padded size
+    P.z22 = e22.zmax <= 6 && !tt ? 6 : 8;
+    P.zm = std::max(e23.zmax, e32.zmax) <= 4 && !tt ? 4 : 8;
+    const int s23 = std::max(e23.zmax, 1), s22 = std::max(e22.zmax, 1), s32 = std::max(e32.zmax, 1);
+    P.mats.assign(size_t(A2) * P.zm * 24, 0.0);
+    for (int a = 0; a < A2; ++a)
+        for (int k = 0; k < e23.cnt_atom[a]; ++k)
+            std::copy_n(&e23.mats[size_t(a * s23 + k) * 24], 24, &P.mats[size_t(a * P.zm + k) * 24]);
+    P.j22off = int(P.mats.size());
+    P.mats.resize(P.mats.size() + size_t(A2) * P.z22 * 9, 0.0);
+    for (int a = 0; a < A2; ++a)
+        for (int k = 0; k < e22.cnt_atom[a]; ++k)
+            std::copy_n(&e22.mats[size_t(a * s22 + k) * 9], 9, &P.mats[size_t(P.j22off) + size_t(a * P.z22 + k) * 9]);
+    const int zero = int(P.mats.size());
+    P.mats.resize(P.mats.size() + 24, 0.0);
+    P.off32.assign(size_t(A3) * P.zm, zero);
+    for (int a = 0; a < A3; ++a)
+        for (int k = 0; k < e32.cnt_atom[a]; ++k) {
+            int& o = P.off32[size_t(a) * P.zm + k];
+            if (!twins.empty()) {
+                const int t = twins[size_t(a) * 8 + k] / 24;  // (sublattice * s23 + slot) of the twin
+                o = (t / s23 * P.zm + t % s23) * 24;
+            } else {
+                o = int(P.mats.size());
+                for (int e = 0; e < 3; ++e)
+                    for (int d = 0; d < 8; ++d) P.mats.push_back(e32.mats[size_t(a * s32 + k) * 24 + d * 3 + e]);
+            }
+        }
+    return P;
+}
+
 struct EllDev {
     DBuf<int> col, cnt, cnt_atom;
     DBuf<double> mats;
@@ -1456,7 +1500,7 @@ struct csl_mixed {
     size_t last_split = 0;  // trajectories the persistent kernel ran in two pieces
     double last_persist_ms = 0.0;  // the persistent launch alone
     DBuf<double> pG, ptgrid;
-    DBuf<int> j32off;  // see MixDev::j32off
+    DBuf<unsigned char> ppack;  // packed partner and matrix tables (MixDev::q22 .. j32pad)
     DBuf<csl::MixDev> pM;  // device copy of M for the persistent kernel
     DBuf<unsigned> coop_ctl;  // cooperative kernel: barrier counter, status
     DBuf<int> psched;         // work split of the persistent kernel
@@ -1775,11 +1819,11 @@ bool run_mixed_coop(csl_mixed* h, size_t B, const double* d_tp, const double* d_
 csl::MixPersistShape mixed_persist_shape(const csl_mixed* h) {
     const csl::MixDev& M = h->M;
     if (!(M.e22.uniform && M.e23.uniform && M.e33.uniform && M.e32.uniform && M.site_uniform2 && M.site_uniform3))
-        return {0, 0, false};
+        return {0, 0, false, false};
     if (h->zmax[0] > csl::kMixZ22 || h->zmax[1] > csl::kMixZ23 || h->zmax[2] > csl::kMixZ33 ||
         h->zmax[3] > csl::kMixZ32)
-        return {0, 0, false};
-    return csl::mixed_persist_shape(M.NP2, M.NP3, h->zmax[2] > 0);
+        return {0, 0, false, false};
+    return csl::mixed_persist_shape(M, h->zmax[2] > 0);
 }
 
 // The batch on the persistent kernel (states in h->X, records into h->recs):
@@ -1800,7 +1844,11 @@ bool run_mixed_persist(csl_mixed* h, size_t B, const double* d_tp, const double*
     csl::MixPersistArgs A{};
     int occ = 0;
     h->pM.upload(&h->M, 1, s);
-    if (csl::launch_mixed_persist(h->M, h->pM.p, A, shape, 0, s, &occ) != hipSuccess || occ < 1) {
+    auto launch = [&](int wg, int* o) {
+        return shape.waves ? csl::launch_mixed_waves(h->M, h->pM.p, A, shape, wg, s, o)
+                           : csl::launch_mixed_persist(h->M, h->pM.p, A, shape, wg, s, o);
+    };
+    if (launch(0, &occ) != hipSuccess || occ < 1) {
         (void)hipGetLastError();
         return false;
     }
@@ -1847,7 +1895,7 @@ bool run_mixed_persist(csl_mixed* h, size_t B, const double* d_tp, const double*
     hip_check(hipEventCreate(&e0), "event");
     hip_check(hipEventCreate(&e1), "event");
     hip_check(hipEventRecord(e0, s), "event record");
-    hip_check(csl::launch_mixed_persist(h->M, h->pM.p, A, shape, int(grid_wg), s, nullptr), "k_mixed_persist");
+    hip_check(launch(int(grid_wg), nullptr), "mixed persistent kernel");
     hip_check(hipEventRecord(e1, s), "event record");
     hip_check(hipStreamSynchronize(s), "mixed persistent integration");
     if (A.sched) {
@@ -2058,10 +2106,42 @@ int csl_mixed_create(size_t A2, size_t A3, size_t n_cells, const double* field2,
             h->zmax[2] = e33.zmax;
             h->zmax[3] = e32.zmax;
             const std::vector<int> jo = transpose_offsets(e23, e32, A2, A3, int(n_cells), npad);
-            M.j32off = nullptr;
-            if (!jo.empty()) {
-                h->j32off.upload(jo.data(), jo.size(), s);
-                M.j32off = h->j32off.p;
+            // tables of the persistent kernels, packed into one buffer
+            std::vector<unsigned char> pk;
+            if (M.NP2 <= 2048 && M.NP3 <= 2048 && e22.zmax <= csl::kMixZ22 && e23.zmax <= csl::kMixZ23 &&
+                e33.zmax <= csl::kMixZ33 && e32.zmax <= csl::kMixZ32 && e22.uniform && e23.uniform && e32.uniform) {
+                const PaddedMats P = pad_mats(e22, e23, e32, jo, int(A2), int(A3), e33.zmax > 0);
+                auto put = [&](const void* v, size_t bytes) {
+                    const size_t at = pk.size();
+                    const auto* c = static_cast<const unsigned char*>(v);
+                    pk.insert(pk.end(), c, c + bytes);
+                    pk.resize((pk.size() + 255) / 256 * 256);
+                    return at;
+                };
+                auto partners = [&](const EllHost& e, int NP, int Z, int npart) {
+                    std::vector<unsigned short> q(size_t(NP) * Z);
+                    for (int p = 0; p < NP; ++p)
+                        for (int k = 0; k < Z; ++k)
+                            q[size_t(p) * Z + k] = static_cast<unsigned short>(
+                                k < e.cnt[p] ? e.col[size_t(k) * NP + p] : std::min(p, npart - 1));
+                    return put(q.data(), q.size() * sizeof(unsigned short));
+                };
+                const size_t o22 = partners(e22, M.NP2, csl::kMixZ22, M.NP2);
+                const size_t o23 = partners(e23, M.NP2, csl::kMixZ23, M.NP3);
+                const size_t o32 = partners(e32, M.NP3, csl::kMixZ32, M.NP2);
+                const size_t o33 = partners(e33, M.NP3, csl::kMixZ33, M.NP3);
+                const size_t oj = put(P.mats.data(), P.mats.size() * sizeof(double));
+                const size_t oo = put(P.off32.data(), P.off32.size() * sizeof(int));
+                h->ppack.upload(pk.data(), pk.size(), s);
+                M.q22 = reinterpret_cast<const uint4*>(h->ppack.p + o22);
+                M.q23 = reinterpret_cast<const uint4*>(h->ppack.p + o23);
+                M.q32 = reinterpret_cast<const uint4*>(h->ppack.p + o32);
+                M.q33 = reinterpret_cast<const uint2*>(h->ppack.p + o33);
+                M.jpad = reinterpret_cast<const double*>(h->ppack.p + oj);
+                M.j32pad = reinterpret_cast<const int*>(h->ppack.p + oo);
+                M.j22off = P.j22off;
+                M.jz22 = P.z22;
+                M.jzm = P.zm;
             }
             site_tables<3>(N2, A2, npad, field2, onsite2, h->field2, h->onsite2, M.site_uniform2, M.has_onsite2, s);
             site_tables<8>(N3, A3, npad, field3, onsite3, h->field3, h->onsite3, M.site_uniform3, M.has_onsite3, s);

@@ -38,11 +38,22 @@ struct MixDev {
     double alpha;
     double gamma[8];
     int has_bloch;
-    // [A3][8]: offset (doubles) in e23.mats of the SU(2)->SU(3) matrix whose
-    // transpose is the SU(3)->SU(2) matrix of each (sublattice, slot), or
-    // null when the tables do not pair up that way (the persistent kernel
-    // then reads e32.mats)
-    const int* __restrict__ j32off;
+    // partner indices of the persistent kernels, 16 bits each, one load per
+    // site and bond kind ([NP2] kinds 22 and 23, [NP3] kinds 32 and 33); a
+    // padding slot's partners are itself.  Null when a table does not fit.
+    const uint4* __restrict__ q22;
+    const uint4* __restrict__ q23;
+    const uint4* __restrict__ q32;
+    const uint2* __restrict__ q33;
+    // bond matrices of the persistent kernels, every sublattice padded with
+    // zero matrices to the same number of bonds (no per-bond count tests):
+    // kind 23 [A2][jzm][3][8], kind 22 from j22off [A2][jz22][3][3], and for
+    // each (SU(3) sublattice, slot) the offset j32pad of a 3x8 matrix whose
+    // transpose is the kind 32 one (the kind 23 matrix itself where the
+    // tables pair up)
+    const double* __restrict__ jpad;
+    const int* __restrict__ j32pad;
+    int j22off, jz22, jzm;
 };
 
 constexpr int kRec = CSL_MIXED_RECORD;
@@ -85,7 +96,7 @@ struct MixPersistArgs {
     double dt;
     const double* tgrid;       // [n_steps + 1] step start times
     double* X;                 // [B_rec][3 NP2 + 8 NP3] SoA states: initial in, final out; x during the run
-    double* G;                 // [grid][2 parities][2][NP3] SU(3) components 6, 7 of the stage values
+    double* G;                 // [grid][2 parities][NP3][2] SU(3) components 6, 7 of the stage values
     const double* tp;          // [B_rec][2] SU(2) pulse centres, or null: no drive
     const double* tp3;         // [B_rec][2] SU(3) pulse centres
     const double* scale;       // [B_rec][2] pulse scales, or null (1)
@@ -112,9 +123,16 @@ constexpr int kMixZ22 = 8, kMixZ23 = 8, kMixZ32 = 8, kMixZ33 = 4;
 struct MixPersistShape {
     int block, spt;
     bool tt;
+    bool waves;  // one unit of 64 sites of one species per wave (csl_mixed_waves.hip)
 };
-MixPersistShape mixed_persist_shape(int NP2, int NP3, bool tt);
-size_t mixed_persist_lds_bytes(int NP2, int NP3, int block);
+MixPersistShape mixed_persist_shape(const MixDev& M, bool tt);
+// glds: SU(3) components 6, 7 of the stage values in LDS too
+size_t mixed_persist_lds_bytes(const MixDev& M, int block, bool glds);
+// The one-unit-per-wave kernel: its LDS, and the launcher (arguments as
+// launch_mixed_persist).
+size_t mixed_waves_lds_bytes(const MixDev& M);
+hipError_t launch_mixed_waves(const MixDev& Mh, const MixDev* M, const MixPersistArgs& A, const MixPersistShape& shape,
+                              int grid, hipStream_t st, int* occ);
 // Mh: the lattice description on the host, M: its copy in device memory.
 // With occ non-null: the co-resident workgroups per CU of that instance
 // (nothing is launched).

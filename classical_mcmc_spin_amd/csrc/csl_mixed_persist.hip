@@ -1,624 +1,660 @@
 // csl_mixed_persist.hip — persistent batched RK4 kernel of the mixed
-// SU(2) + SU(3) lattice: one workgroup integrates one trajectory for the
-// whole time grid (mixed_lattice_gpu.cu:278-347 launches one kernel per RK
-// stage instead), so the per-stage state never crosses HBM.
+// SU(2) + SU(3) lattice: one workgroup integrates one trajectory (or a piece
+// of one) for the whole time grid (mixed_lattice_gpu.cu:278-347 launches one
+// kernel per RK stage instead), so the per-stage state never crosses HBM.
+// Lattices of at most 16 units of 64 sites run on csl_mixed_waves.hip.
 //
 // On-chip budget of one trajectory of the 8x8x8 TmFeO3-like cell (2048 SU(2)
 // + 2048 SU(3) sites, 176 KB of stage values): RK4 needs the step-start
 // state x, the accumulator and the stage values.  The stage values are what
-// the neighbours gather, so they go to LDS — the SU(2) planes and SU(3)
-// components 0..5 (144 KB); SU(3) components 6 and 7 (32 KB) go to a
-// per-workgroup global buffer with two parities that stays in L2.  The
+// the neighbours gather, so they go to LDS: the SU(2) sites as records of 24
+// bytes, the SU(3) components 0..5 as records of 48 bytes (three 16-byte
+// loads at one address; the strides spread a wave's records over all banks).
+// SU(3) components 6 and 7 go to LDS too where they fit (GLDS, up to 1536
+// sites of each species) and otherwise to a per-workgroup global buffer with
+// two parities that stays in L2, one 16-byte access per site.  The
 // accumulators of a thread's sites live in VGPRs; x lives in the trajectory's
 // own slot of the global state array (read in stages 1 and 2, written in
-// stage 3: three 176 KB passes per step instead of the stage kernels' sixteen
-// plane passes).
+// stage 3).
 //
-// Per stage (stage values y_s in LDS + G[s&1]):  every thread evaluates its
-// SU(2) and SU(3) sites from y_s, updates the accumulators, writes SU(3)
-// components 6, 7 of y_{s+1} straight to G[(s+1)&1] and keeps the rest of
-// y_{s+1} in VGPRs -> barrier (every read of y_s done) -> y_{s+1} into LDS ->
-// barrier.  Threads own sites p = tid + j*512 of each species (sublattice
-// major, npad a multiple of 64), so a wave covers 64 sites of one sublattice
-// and reads that sublattice's bond matrices, field, onsite matrix, frame and
-// drive directions with scalar loads (translation-invariant tables only).
-// Records (both species' magnetisations and E/(N2+N3), the 34 values of the
-// stage kernels' record) are reduced inside the workgroup and written
-// directly, at stage 0 of every save_interval-th step and after the last step.
+// Per stage without SU(3)-SU(3) bonds: the SU(2) sites from y_s, their next
+// values kept in VGPRs -> barrier -> the SU(3) sites, updated in place (only
+// the owner reads an SU(3) site's own value then) -> barrier -> the SU(2)
+// next values into LDS -> barrier.  With them (TT) both species' next values
+// are held until one barrier.  A wave owns SPT consecutive units of 64 sites
+// of each species; two units of one sublattice are advanced together, so
+// their bond matrices (scalar loads) are fetched once.
+//
+// Field rows, pulse envelopes and records are handled as in
+// csl_trajectory.hip: rows of -(B + drive) from LDS, envelopes of two steps
+// at a time, records from the waves' sums of S and S.H, two at a time.  With
+// every record's 33 wave sums in shuffles, an envelope evaluation per wave
+// and stage, one 4-byte partner load per bond and one 8-byte access per
+// component a stage of the 8x8x8 cell took 36.8 us.
 #include <algorithm>
 #include <type_traits>
 
-#include "csl_device.hpp"
-#include "csl_mixed_device.hpp"
+#include "csl_mixed_lds.hpp"
 
 namespace csl {
 
 namespace {
 
-// a double of lane l of this wave, in every lane
-__device__ __forceinline__ double lane_double(double v, int l) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-    return __hiloint2double(hi, lo);
-}
+constexpr int kChunk = 2;   // steps whose records and envelopes go together
 
-// The lattice description lives in device memory and is read through a
-// pointer laundered by an opaque zero where it is used (once per site and
-// phase): its fields and the table pointers are fetched with scalar loads at
-// the point of use instead of occupying SGPRs for the whole kernel (the
-// description is 416 bytes, more than the SGPR file).
-using MP = cptr<MixDev>;
-__device__ __forceinline__ MP fresh_mix(const MixDev* Mg) { return as_const(Mg) + opaque_zero(); }
-
-// Stage values of one trajectory: SU(2) planes F[3][NP2] and SU(3)
-// components 0..5 TL[6][NP3] in LDS, components 6, 7 in Gc[2][NP3].
-struct MixStageView {
-    const double* F;
-    const double* TL;
-    const double* Gc;
-    int NP2, NP3;
-    __device__ __forceinline__ double tm(int c, int q) const {
-        return c < 6 ? TL[c * NP3 + q] : Gc[(c - 6) * NP3 + q];
+// LDS layout (in doubles)
+struct Lay {
+    int t, t2, f;            // SU(3) [NP3][6] (and [NP3][2] with GLDS), SU(2) [NP2][3]
+    int cst, hin, drv, red;
+    int rows, n2, n3, rec;   // units of each species, doubles per record
+    int total;
+    __host__ __device__ Lay(int NP2, int NP3, int A2, int A3, int nwaves, bool glds) {
+        t = 0;
+        t2 = 6 * NP3;
+        f = t2 + (glds ? 2 * NP3 : 0);
+        rows = 3 * A2 + 8 * A3;
+        cst = f + 3 * NP2;
+        cst += cst & 1;
+        hin = cst + 3 * rows;
+        drv = hin + 8 * rows;
+        red = drv + 2 * kChunk * 12;
+        n2 = NP2 / kWave;
+        n3 = NP3 / kWave;
+        // a record: SU(2) units x 4, SU(3) units x 8 (twice with signed
+        // sums), one energy sum per wave
+        rec = 4 * n2 + ((A3 & 1) ? 16 : 8) * n3 + 4 * nwaves;
+        total = red + kChunk * rec;
     }
-    __device__ __forceinline__ double fe(int c, int q) const { return F[c * NP2 + q]; }
 };
 
-// Undriven local field of SU(2) site p (sublattice a) from the stage values:
-// -B + 2A S + sum J22 S_p + sum J23 l_p, the terms in the order of the stage
-// kernels' field_su2 (uniform tables, per-sublattice field and onsite).
-__device__ __forceinline__ void fe_field(const MixDev* Mg, const MixStageView& V, int a, int p, const double S[3],
-                                         double H[3]) {
-    const MP M = fresh_mix(Mg);
-    const cptr<double> f = as_const(M->field2) + a * 3;
+// Ends a bond: the field values as they are now (the products cannot be put
+// off past this point, with the bond's matrix saved for later).
+template <int N, int D>
+__device__ __forceinline__ void end_bond(double (*H)[D]) {
 #pragma unroll
-    for (int d = 0; d < 3; ++d) H[d] = -f[d];
-    if (M->has_onsite2) {
-        const cptr<double> A2 = as_const(M->onsite2) + a * 9;
+    for (int j = 0; j < N; ++j)
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            double r = 0.0;
-#pragma unroll
-            for (int e = 0; e < 3; ++e) r += A2[d * 3 + e] * S[e];
-            H[d] += r;
-        }
-    }
-    // partner indices of every bond first (independent loads in flight),
-    // then the gathers and products
-    const int c22 = uniform(as_const(M->e22.cnt_atom)[a]);
-    const int c23 = uniform(as_const(M->e23.cnt_atom)[a]);
-    int q22[kMixZ22], q23[kMixZ23];
-#pragma unroll
-    for (int k = 0; k < kMixZ22; ++k)
-        if (k < c22) q22[k] = M->e22.col[size_t(k) * V.NP2 + fresh(p)];
-#pragma unroll
-    for (int k = 0; k < kMixZ23; ++k)
-        if (k < c23) q23[k] = M->e23.col[size_t(k) * V.NP2 + fresh(p)];
-#pragma unroll
-    for (int k = 0; k < kMixZ22; ++k) {
-        if (k < c22) {
-            double s[3];
-#pragma unroll
-            for (int e = 0; e < 3; ++e) s[e] = V.fe(e, q22[k]);
-            const cptr<double> J = as_const(M->e22.mats) + (a * M->e22.zmax + k) * 9;
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-#pragma unroll
-                for (int e = 0; e < 3; ++e) H[d] = fma(J[d * 3 + e], s[e], H[d]);
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < kMixZ23; ++k) {
-        if (k < c23) {
-            double s[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) s[e] = V.tm(e, q23[k]);
-            const cptr<double> J = as_const(M->e23.mats) + (a * M->e23.zmax + k) * 24;
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) H[d] = fma(J[d * 8 + e], s[e], H[d]);
-        }
-    }
+        for (int d = 0; d < D; ++d) asm volatile("" : "+v"(H[j][d]));
 }
 
-// The same for an SU(3) site: -B + 2A l + sum J33 l_p + sum J32 S_p
-// (field_su3); TT: the lattice has SU(3)-SU(3) bonds.
-template <bool TT>
-__device__ __forceinline__ void tm_field(const MixDev* Mg, const MixStageView& V, int a, int p, const double S[8],
-                                         double H[8]) {
-    const MP M = fresh_mix(Mg);
-    const cptr<double> f = as_const(M->field3) + a * 8;
+template <int Z22, int ZM, bool GLDS>
+struct Field {
+    const MixDev* Mg;
+    const double* smem;
+    const Lay& Y;
+    const double2* g;        // components 6, 7 of the stage (global), !GLDS
+
+    __device__ __forceinline__ void tm(int q, double v[8]) const {
+        const double2* r = reinterpret_cast<const double2*>(smem + Y.t + 6 * q);
 #pragma unroll
-    for (int d = 0; d < 8; ++d) H[d] = -f[d];
-    if (M->has_onsite3) {
-        const cptr<double> A3 = as_const(M->onsite3) + a * 64;
-#pragma unroll
-        for (int d = 0; d < 8; ++d) {
-            double r = 0.0;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) r += A3[d * 8 + e] * S[e];
-            H[d] += r;
+        for (int i = 0; i < 3; ++i) {
+            const double2 a = r[i];
+            v[2 * i] = a.x;
+            v[2 * i + 1] = a.y;
         }
+        const double2 a = GLDS ? *reinterpret_cast<const double2*>(smem + Y.t2 + 2 * q) : g[q];
+        v[6] = a.x;
+        v[7] = a.y;
     }
-    const int c33 = TT ? uniform(as_const(M->e33.cnt_atom)[a]) : 0;
-    const int c32 = uniform(as_const(M->e32.cnt_atom)[a]);
-    int q33[TT ? kMixZ33 : 1], q32[kMixZ32];
-    if constexpr (TT) {
+
+    // fields of N units of SU(2) sublattice a at sites p, p + 64, ...  The
+    // bonds are kept apart (an opaque address each, end_bond):
+    // the compiler otherwise loads every bond's matrix at once and spills them
+    template <int N>
+    __device__ __forceinline__ void fe(int a, int p, const double (*S)[3], double (*H)[3]) const {
+        const cptr<MixDev> M = as_const(Mg) + opaque_zero();
+        int q22[N][8], q23[N][8];
 #pragma unroll
-        for (int k = 0; k < kMixZ33; ++k)
-            if (k < c33) q33[k] = M->e33.col[size_t(k) * V.NP3 + fresh(p)];
-    }
-#pragma unroll
-    for (int k = 0; k < kMixZ32; ++k)
-        if (k < c32) q32[k] = M->e32.col[size_t(k) * V.NP3 + fresh(p)];
-    if constexpr (TT) {
-#pragma unroll
-        for (int k = 0; k < kMixZ33; ++k) {
-            if (k < c33) {
-                double s[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) s[e] = V.tm(e, q33[k]);
-                const cptr<double> J = as_const(M->e33.mats) + (a * M->e33.zmax + k) * 64;
-#pragma unroll
-                for (int d = 0; d < 8; ++d)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) H[d] = fma(J[d * 8 + e], s[e], H[d]);
-            }
+        for (int j = 0; j < N; ++j) {
+            unpack8(M->q22[p + j * kWave], q22[j]);
+            unpack8(M->q23[p + j * kWave], q23[j]);
         }
-    }
-    // the SU(3)->SU(2) matrices as transposes of the SU(2)->SU(3) ones when
-    // the tables pair up (half the bond-matrix footprint in the scalar
-    // cache: the SU(2) sites read the same matrices); same values, same order
-    const int* jo = M->j32off;
-    if (jo) {
-        int off[kMixZ32];
+        if (M->has_onsite2) {
+            const cptr<double> A2 = as_const(M->onsite2) + a * 9;
 #pragma unroll
-        for (int k = 0; k < kMixZ32; ++k) off[k] = as_const(jo)[a * 8 + k];
+            for (int j = 0; j < N; ++j)
 #pragma unroll
-        for (int k = 0; k < kMixZ32; ++k) {
-            if (k < c32) {
+                for (int d = 0; d < 3; ++d)
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) H[j][d] = fma(A2[d * 3 + e], S[j][e], H[j][d]);
+        }
+        // components 6 and 7 of the SU(3) partners from global memory: in
+        // flight while the SU(2) bonds run
+        double2 gl[GLDS ? 1 : N][GLDS ? 1 : ZM];
+        if constexpr (!GLDS) {
+#pragma unroll
+            for (int j = 0; j < N; ++j)
+#pragma unroll
+                for (int k = 0; k < ZM; ++k) gl[j][k] = g[q23[j][k]];
+        }
+        const cptr<double> jp = as_const(M->jpad);
+        const int j2 = M->j22off + a * (Z22 * 9), j3 = a * (ZM * 24);
+#pragma unroll
+        for (int k = 0; k < Z22; ++k) {
+            const cptr<double> J2 = jp + j2 + k * 9 + opaque_zero();
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
                 double s[3];
+                ld3(smem + Y.f + 3 * q22[j][k], s);
 #pragma unroll
-                for (int e = 0; e < 3; ++e) s[e] = V.fe(e, q32[k]);
-                const cptr<double> J = as_const(M->e23.mats) + uniform(off[k]);
+                for (int e = 0; e < 3; ++e)
 #pragma unroll
-                for (int d = 0; d < 8; ++d)
+                    for (int d = 0; d < 3; ++d) H[j][d] = fma(J2[d * 3 + e], s[e], H[j][d]);
+            }
+            end_bond<N, 3>(H);
+        }
 #pragma unroll
-                    for (int e = 0; e < 3; ++e) H[d] = fma(J[e * 8 + d], s[e], H[d]);
+        for (int k = 0; k < ZM; ++k) {
+            const cptr<double> J3 = jp + j3 + k * 24 + opaque_zero();
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                const int q = q23[j][k];
+                double s[8];
+                const double2* r = reinterpret_cast<const double2*>(smem + Y.t + 6 * q);
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    const double2 v = r[i];
+                    s[2 * i] = v.x;
+                    s[2 * i + 1] = v.y;
+                }
+                const double2 v = GLDS ? *reinterpret_cast<const double2*>(smem + Y.t2 + 2 * q) : gl[GLDS ? 0 : j][GLDS ? 0 : k];
+                s[6] = v.x;
+                s[7] = v.y;
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) H[j][d] = fma(J3[d * 8 + e], s[e], H[j][d]);
+            }
+            end_bond<N, 3>(H);
+        }
+    }
+
+    // bond fields of N units of SU(3) sublattice a (the on-site part apart)
+    template <int N, bool TT>
+    __device__ __forceinline__ void tm_bonds(int a, int p, double (*H)[8]) const {
+        const cptr<MixDev> M = as_const(Mg) + opaque_zero();
+        int q32[N][8];
+#pragma unroll
+        for (int j = 0; j < N; ++j) unpack8(M->q32[p + j * kWave], q32[j]);
+        if constexpr (TT) {
+            const int c33 = uniform(as_const(M->e33.cnt_atom)[a]);
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                const uint2 v = M->q33[p + j * kWave];
+                const int q33[4] = {lo16(v.x), hi16(v.x), lo16(v.y), hi16(v.y)};
+#pragma unroll
+                for (int k = 0; k < kMixZ33; ++k) {
+                    if (k < c33) {
+                        double s[8];
+                        tm(q33[k], s);
+                        const cptr<double> J = as_const(M->e33.mats) + (a * M->e33.zmax + k) * 64;
+#pragma unroll
+                        for (int d = 0; d < 8; ++d)
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) H[j][d] = fma(J[d * 8 + e], s[e], H[j][d]);
+                    }
+                }
             }
         }
-        return;
-    }
+        const cptr<int> off = as_const(M->j32pad) + a * ZM;
+        const cptr<double> jp = as_const(M->jpad);
 #pragma unroll
-    for (int k = 0; k < kMixZ32; ++k) {
-        if (k < c32) {
-            double s[3];
+        for (int k = 0; k < ZM; ++k) {
+            const cptr<double> J = jp + uniform(off[k]) + opaque_zero();
 #pragma unroll
-            for (int e = 0; e < 3; ++e) s[e] = V.fe(e, q32[k]);
-            const cptr<double> J = as_const(M->e32.mats) + (a * M->e32.zmax + k) * 24;
+            for (int j = 0; j < N; ++j) {
+                double s[3];
+                ld3(smem + Y.f + 3 * q32[j][k], s);
 #pragma unroll
-            for (int d = 0; d < 8; ++d)
+                for (int e = 0; e < 3; ++e)
 #pragma unroll
-                for (int e = 0; e < 3; ++e) H[d] = fma(J[d * 3 + e], s[e], H[d]);
+                    for (int d = 0; d < 8; ++d) H[j][d] = fma(J[e * 8 + d], s[e], H[j][d]);
+            }
+            end_bond<N, 8>(H);
         }
     }
-}
-
-// 0.5 S.(H - B) of a site: its share of the energy (H undriven)
-template <int D>
-__device__ __forceinline__ double site_energy_mixed(const double* field, int a, const double* S, const double* H) {
-    const cptr<double> B = as_const(field) + a * D;
-    double e = 0.0;
-#pragma unroll
-    for (int mu = 0; mu < D; ++mu) e += S[mu] * (H[mu] - B[mu]);
-    return 0.5 * e;
-}
-
-// Magnetisation sums (record entries 0..32) of the stage values of this
-// thread's sites, summed over the wave into red[wave][0..32].
-template <int SPT, int T>
-__device__ __forceinline__ void observe(MP M, const MixStageView& V, int tid, int lane, int wave,
-                                        const int* at2, const int* at3, unsigned act2, unsigned act3, double* red) {
-    double pt[33];
-#pragma unroll
-    for (int i = 0; i < 33; ++i) pt[i] = 0.0;
-#pragma unroll
-    for (int j = 0; j < SPT; ++j) {
-        if (!((act2 >> j) & 1u)) continue;
-        const int p = fresh(tid + j * T), a = at2[j];
-        const double S[3] = {V.fe(0, p), V.fe(1, p), V.fe(2, p)};
-        const cptr<double> R = as_const(M->frames2) + a * 9;
-        const double sg = as_const(M->afm2)[a];
-#pragma unroll
-        for (int mu = 0; mu < 3; ++mu) {
-            const double g = R[mu * 3] * S[0] + R[mu * 3 + 1] * S[1] + R[mu * 3 + 2] * S[2];
-            pt[mu] += sg * g;
-            pt[3 + mu] += S[mu];
-            pt[6 + mu] += g;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < SPT; ++j) {
-        if (!((act3 >> j) & 1u)) continue;
-        const int p = fresh(tid + j * T), a = at3[j];
-        const int cell = p - a * M->npad;
-        double S[8];
-#pragma unroll
-        for (int c = 0; c < 8; ++c) S[c] = V.tm(c, p);
-        const cptr<double> R = as_const(M->frames3) + a * 64;
-        const double sg = ((cell * M->A3 + a) & 1) ? -1.0 : 1.0;
-#pragma unroll
-        for (int mu = 0; mu < 8; ++mu) {
-            double g = 0.0;
-#pragma unroll
-            for (int nu = 0; nu < 8; ++nu) g += R[mu * 8 + nu] * S[nu];
-            pt[9 + mu] += sg * S[mu];
-            pt[17 + mu] += S[mu];
-            pt[25 + mu] += g;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 33; ++i) {
-        const double v = wave_sum(pt[i]);
-        if (lane == 0) red[wave * kRec + i] = v;
-    }
-}
+};
 
 }  // namespace
 
-template <int SPT, int T, bool TT>
-__global__ void __launch_bounds__(T) k_mixed_persist(const MixDev* __restrict__ Mg, MixPersistArgs A) {
-    const MP M0 = fresh_mix(Mg);
+template <int SPT, int T, int Z22, int ZM, bool TT, bool GLDS>
+__global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
     extern __shared__ double smem[];
     constexpr int nwaves = T / kWave;
+    constexpr int NP_ = (SPT % 2 == 0 && !TT) ? 2 : 1;   // units advanced together where their sublattice agrees
+    const MixDev* const Mg = K.M;
+    const cptr<MixDev> M0 = as_const(Mg);
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = uniform(tid >> 6);
-    const int NP2 = M0->NP2, NP3 = M0->NP3;
-    double* F = smem;                        // [3][NP2] SU(2) stage values
-    double* TL = F + 3 * size_t(NP2);        // [6][NP3] SU(3) stage values, components 0..5
-    double* red = TL + 6 * size_t(NP3);      // [nwaves][kRec] record sums of the waves
-    double* Gw = A.G + size_t(blockIdx.x) * 4 * size_t(NP3);  // [2 parities][2][NP3]
+    const int NP2 = M0->NP2, NP3 = M0->NP3, A2 = M0->A2, A3 = M0->A3, npad = M0->npad, n_cells = M0->n_cells;
+    const Lay Y(NP2, NP3, A2, A3, nwaves, GLDS);
+    const MixTables Q{smem + Y.cst, smem + Y.hin, smem + Y.drv, smem + Y.red, Y.rows};
+    const int R = Y.rows;
+    double2* const Gw = GLDS ? nullptr : reinterpret_cast<double2*>(K.A.G) + size_t(blockIdx.x) * 2 * size_t(NP3);
     const size_t SZ = 3 * size_t(NP2) + 8 * size_t(NP3);
     const size_t o3 = 3 * size_t(NP2);
-    const double dt = A.dt;
-    const double b16 = (1.0 / 6.0) * dt, b13 = (1.0 / 3.0) * dt;
+    const double dt = K.A.dt;
+    const bool drive = K.A.tp != nullptr;
+    const int u0 = wave * SPT;                       // first unit of the wave (both species)
+    const int p0 = u0 * kWave + lane;
+    const int m2 = min(max(Y.n2 - u0, 0), SPT), m3 = min(max(Y.n3 - u0, 0), SPT);  // its units
+    auto atom = [&](int j) { return uniform((u0 + j) * kWave / npad); };
+    auto real = [&](int j) { const int p = p0 + j * kWave; return p - p / npad * npad < n_cells; };
 
-    // own sites of each species: p = tid + j*T, sublattice p / npad
-    int at2[SPT], at3[SPT];
-    unsigned act2 = 0, act3 = 0;
-#pragma unroll
-    for (int j = 0; j < SPT; ++j) {
-        const int pw = wave * kWave + j * T;
-        at2[j] = uniform(min(pw, NP2 - 1) / M0->npad);
-        at3[j] = uniform(min(pw, NP3 - 1) / M0->npad);
-        const int p = tid + j * T;
-        if (p < NP2 && p - at2[j] * M0->npad < M0->n_cells) act2 |= 1u << j;
-        if (p < NP3 && p - at3[j] * M0->npad < M0->n_cells) act3 |= 1u << j;
-    }
-
-    for (int piece = 0;; ++piece) {
-        // this workgroup's next trajectory (steps [s_begin, s_end))
-        int b = int(blockIdx.x) + piece * int(gridDim.x), s_begin = 0, s_end = A.n_steps, wait = -1, post = -1;
-        if (A.sched) {
-            if (piece >= A.max_pieces) break;
-            const int* r = A.sched + (size_t(blockIdx.x) * A.max_pieces + piece) * 5;
-            b = r[0];
-            s_begin = r[1];
-            s_end = r[2];
-            wait = r[3];
-            post = r[4];
-            if (b < 0) break;  // unused rows come last
-        } else if (b >= A.B) {
-            break;
-        }
-        b += A.b0;
-        double* X = A.X + size_t(b) * SZ;
-        const bool drive = A.tp != nullptr;
-        const double tpa = drive ? A.tp[2 * size_t(b)] : 0.0, tpb = drive ? A.tp[2 * size_t(b) + 1] : 0.0;
-        const double tqa = drive ? A.tp3[2 * size_t(b)] : 0.0, tqb = drive ? A.tp3[2 * size_t(b) + 1] : 0.0;
-        const double sca = (drive && A.scale) ? A.scale[2 * size_t(b)] : 1.0;
-        const double scb = (drive && A.scale) ? A.scale[2 * size_t(b) + 1] : 1.0;
-
-        if (wait >= 0) {
-            // the state at s_begin, stored in X by the workgroup that ran
-            // the trajectory's first steps as its first piece; a bounded
-            // wait that gives up flags the launch
-            if (tid == 0) {
-                unsigned ok = 0;
-                for (long it = 0; it < (1L << 24); ++it) {
-                    ok = __hip_atomic_load(A.flags + wait, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-                    if (ok) break;
-                    __builtin_amdgcn_s_sleep(8);
-                }
-                if (!ok) __hip_atomic_store(A.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            __syncthreads();
-            __atomic_thread_fence(__ATOMIC_ACQUIRE);
-        }
-        // initial state: the stage values of stage 0 (LDS and G[0])
-        __syncthreads();  // the previous trajectory is done with LDS and G
+    MixPiece P;
+    for (int piece = 0; mix_piece(K.A, piece, P); ++piece) {
+        const int b = P.b, s_begin = P.s_begin, s_end = P.s_end;
+        double* const X = K.A.X + size_t(b) * SZ;
+        if (P.wait >= 0) mix_wait_seam(K.A, P.wait, tid);
+        __syncthreads();  // the previous piece is done with LDS and G
+        // initial state: the stage values of stage 0; padding lanes hold
+        // zeros and gather themselves, so their derivative is zero
 #pragma unroll
         for (int j = 0; j < SPT; ++j) {
-            const int p = tid + j * T;
-            if ((act2 >> j) & 1u)
+            const int p = p0 + j * kWave;
+            if (j < m2) {
+                double* r = smem + Y.f + 3 * p;
+                const bool ok = real(j);
 #pragma unroll
-                for (int c = 0; c < 3; ++c) F[c * NP2 + p] = X[size_t(c) * NP2 + p];
-            if ((act3 >> j) & 1u) {
+                for (int c = 0; c < 3; ++c) r[c] = ok ? X[size_t(c) * NP2 + p] : 0.0;
+            }
+            if (j < m3) {
+                const bool ok = real(j);
+                double v[8];
 #pragma unroll
-                for (int c = 0; c < 6; ++c) TL[c * NP3 + p] = X[o3 + size_t(c) * NP3 + p];
-                Gw[p] = X[o3 + size_t(6) * NP3 + p];
-                Gw[NP3 + p] = X[o3 + size_t(7) * NP3 + p];
+                for (int c = 0; c < 8; ++c) v[c] = ok ? X[o3 + size_t(c) * NP3 + p] : 0.0;
+                double2* r = reinterpret_cast<double2*>(smem + Y.t + 6 * p);
+#pragma unroll
+                for (int i = 0; i < 3; ++i) r[i] = make_double2(v[2 * i], v[2 * i + 1]);
+                if constexpr (GLDS) *reinterpret_cast<double2*>(smem + Y.t2 + 2 * p) = make_double2(v[6], v[7]);
+                else Gw[p] = make_double2(v[6], v[7]);
             }
         }
+        mix_fill_tables(M0, Q, tid, T);
         __syncthreads();
+        auto write_drive = [&](int n0, int cp) {
+            if (drive && wave == nwaves - 1) mix_write_drive(Q, b, n0, s_end, cp, kChunk, lane);
+        };
+        auto write_hin = [&](const double* f, int par) {
+            if (drive) mix_write_hin(Q, f, par, 3 * A2, tid, T);
+        };
+        write_drive(s_begin, 0);
+        lds_barrier();
+        write_hin(Q.drv, 0);
+        lds_barrier();
+
+        auto publish = [&](int ri0, int cnt) {
+            for (int k = wave; k < cnt; k += nwaves) {
+                const double *r2 = Q.red + k * Y.rec, *r3 = r2 + 4 * Y.n2, *ra = r3 + 8 * Y.n3;
+                const double* re = r2 + Y.rec - 4 * nwaves;
+                mix_publish(
+                    b, ri0 + k, lane, [&](int w, int c) { return r2[w * 4 + c]; },
+                    [&](int w, int c) { return r3[w * 8 + c]; }, [&](int w, int c) { return ra[w * 8 + c]; },
+                    [&] {
+                        double e = 0.0;
+                        for (int w = 0; w < nwaves; ++w) e += re[w * 4];
+                        return e;
+                    });
+            }
+        };
+        // sums of an SU(2) / SU(3) unit's stage values into record `slot`
+        auto sums2 = [&](int slot, int j, const double S[3]) {
+            wave_sum4(S[0], S[1], S[2], 0.0, lane, Q.red + slot * Y.rec + 4 * (u0 + j));
+        };
+        auto sums3 = [&](int slot, int j, const double S[8]) {
+            double* r = Q.red + slot * Y.rec + 4 * Y.n2 + 8 * (u0 + j);
+            wave_sum4(S[0], S[1], S[2], S[3], lane, r);
+            wave_sum4(S[4], S[5], S[6], S[7], lane, r + 4);
+            if (A3 & 1) {
+                const int p = p0 + j * kWave, a = atom(j);
+                const double sg = (((p - a * npad) * A3 + a) & 1) ? -1.0 : 1.0;
+                r += 8 * Y.n3;
+                wave_sum4(sg * S[0], sg * S[1], sg * S[2], sg * S[3], lane, r);
+                wave_sum4(sg * S[4], sg * S[5], sg * S[6], sg * S[7], lane, r + 4);
+            }
+        };
+        auto sum_e = [&](int slot, double e) {
+            wave_sum4(e, 0.0, 0.0, 0.0, lane, Q.red + slot * Y.rec + (Y.rec - 4 * nwaves) + 4 * wave);
+        };
 
         double acc2[SPT][3], acc3[SPT][8];
-        for (int n = s_begin; n < s_end; ++n) {
-            const bool rec = (n % A.save_interval) == 0;
-            const int ri = n / A.save_interval;
-            const double tn = A.tgrid[n];
-            // RK4 stages at t, t + dt/2, t + dt/2, t + dt
+        // One RK4 stage (runtime index s).  slot >= 0 in stage 0 of a
+        // recorded step.
+        auto stage = [&](int s, int par, int slot) __attribute__((always_inline)) {
+            const double cdt = s == 2 ? dt : 0.5 * dt;
+            const double bdt = (s == 0 || s == 3) ? (1.0 / 6.0) * dt : (1.0 / 3.0) * dt;
+            const double* hrow = Q.hin + (par * 4 + (s == 0 ? 0 : (s == 3 ? 2 : 1))) * R;
+            const double* wrow = Q.hin + (par * 4 + 3) * R;
+            const Field<Z22, ZM, GLDS> F{Mg, smem, Y, GLDS ? nullptr : Gw + (s & 1) * NP3};
+            double2* const Gn = GLDS ? nullptr : Gw + (1 - (s & 1)) * NP3;
+            double e = 0.0;
+            double y2[SPT][3];
+            auto fe_units = [&](auto n_, int j0) __attribute__((always_inline)) {
+                constexpr int N = decltype(n_)::value;
+                const int a = atom(j0);
+                double S[N][3], H[N][3];
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const MP M = fresh_mix(Mg);
-                const MixStageView V{F, TL, Gw + (s & 1) * 2 * NP3, NP2, NP3};  // y_s
-                double* Gn = Gw + (1 - (s & 1)) * 2 * NP3;                      // components 6, 7 of y_{s+1}
-                const double cdt = (s == 2) ? 1.0 * dt : 0.5 * dt;
-                const double bdt = (s == 0 || s == 3) ? b16 : b13;
-                const bool obs = (s == 0) && rec;
-                // drive factors of this stage time (lanes 0..3: species x pulse)
-                double f21 = 0.0, f22 = 0.0, f31 = 0.0, f32 = 0.0;
-                if (drive) {
-                    const double ts = tn + (s == 0 ? 0.0 : (s == 3 ? 1.0 * dt : 0.5 * dt));
-                    double v = 0.0;
-                    if (lane < 4) {
-                        const int sp = lane >> 1, kk = lane & 1;
-                        const double amp = sp ? M->amp3 : M->amp2;
-                        if (amp != 0.0) {
-                            const double tc = sp ? (kk ? tqb : tqa) : (kk ? tpb : tpa);
-                            v = drive_factor(amp, ts, tc, sp ? M->width3 : M->width2, sp ? M->freq3 : M->freq2);
-                            v *= kk ? scb : sca;
-                        }
-                    }
-                    f21 = lane_double(v, 0);
-                    f22 = lane_double(v, 1);
-                    f31 = lane_double(v, 2);
-                    f32 = lane_double(v, 3);
+                for (int j = 0; j < N; ++j) {
+                    ld3(smem + Y.f + 3 * (p0 + (j0 + j) * kWave), S[j]);
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) H[j][d] = hrow[3 * a + d];
                 }
-                if (obs) observe<SPT, T>(M, V, tid, lane, wave, at2, at3, act2, act3, red);
-                double e_acc = 0.0;
-
-                // SU(3) sites: field from y_s, RK4 update; the new stage
-                // values go to LDS / G once nothing reads y_s any more
-                double y3[TT ? SPT : 1][6];
-                auto tm_sites = [&](auto in_place) {
+                F.template fe<N>(a, p0 + j0 * kWave, S, H);
+                const cptr<MixDev> M = as_const(Mg) + opaque_zero();
 #pragma unroll
-                    for (int j = 0; j < SPT; ++j) {
-                        if (!((act3 >> j) & 1u)) continue;
-                        const int p = fresh(tid + j * T), a = at3[j];
-                        const MP M = fresh_mix(Mg);
-                        double S[8];
+                for (int j = 0; j < N; ++j) {
+                    const int p = p0 + (j0 + j) * kWave;
+                    if (slot >= 0) {
 #pragma unroll
-                        for (int c = 0; c < 8; ++c) S[c] = V.tm(c, p);
-                        double H[8];
-                        tm_field<TT>(Mg, V, a, p, S, H);
-                        if (obs) e_acc += site_energy_mixed<8>(M->field3, a, S, H);
-                        if (f31 != 0.0 || f32 != 0.0) {
-                            const cptr<double> d0 = as_const(M->fdrive3) + a * 8;
-                            const cptr<double> d1 = as_const(M->fdrive3) + (M->A3 + a) * 8;
-#pragma unroll
-                            for (int d = 0; d < 8; ++d) H[d] -= d0[d] * f31 + d1[d] * f32;
-                        }
-                        double k[8];
-                        su3_cross(H, S, k);
-                        if (M->has_bloch) {  // mixed_lattice_md.cpp:596-605
-#pragma unroll
-                            for (int d = 0; d < 8; ++d)
-                                if (M->gamma[d] != 0.0) k[d] -= M->gamma[d] * (S[d] - M->eq3[size_t(d) * NP3 + p]);
-                        }
-#pragma unroll
-                        for (int d = 0; d < 8; ++d) {
-                            const size_t q = o3 + size_t(d) * NP3 + p;
-                            double y;
-                            if (s == 0) {
-                                acc3[j][d] = S[d] + bdt * k[d];
-                                y = S[d] + cdt * k[d];
-                            } else if (s < 3) {
-                                acc3[j][d] = acc3[j][d] + bdt * k[d];
-                                y = X[q] + cdt * k[d];
-                            } else {
-                                y = acc3[j][d] + bdt * k[d];
-                                X[q] = y;
-                            }
-                            if (d >= 6) Gn[(d - 6) * NP3 + p] = y;
-                            else if constexpr (decltype(in_place)::value) TL[d * NP3 + p] = y;
-                            else y3[TT ? j : 0][d] = y;
-                        }
+                        for (int d = 0; d < 3; ++d) e = fma(S[j][d], H[j][d] - wrow[3 * a + d], e);
+                        sums2(slot, j0 + j, S[j]);
                     }
-                };
-
-                // SU(2) sites: field from y_s, RK4 update into y2
-                double y2[SPT][3];
+                    double xv[3] = {S[j][0], S[j][1], S[j][2]};
+                    if (s == 1 || s == 2) {
 #pragma unroll
-                for (int j = 0; j < SPT; ++j) {
-                    if (!((act2 >> j) & 1u)) continue;
-                    const int p = fresh(tid + j * T), a = at2[j];
-                    const MP M = fresh_mix(Mg);
-                    const double S[3] = {V.fe(0, p), V.fe(1, p), V.fe(2, p)};
-                    double H[3];
-                    fe_field(Mg, V, a, p, S, H);
-                    if (obs) e_acc += site_energy_mixed<3>(M->field2, a, S, H);
-                    if (f21 != 0.0 || f22 != 0.0) {
-                        const cptr<double> d0 = as_const(M->fdrive2) + a * 3;
-                        const cptr<double> d1 = as_const(M->fdrive2) + (M->A2 + a) * 3;
-#pragma unroll
-                        for (int d = 0; d < 3; ++d) H[d] -= d0[d] * f21 + d1[d] * f22;
+                        for (int d = 0; d < 3; ++d) xv[d] = X[size_t(d) * NP2 + p];
                     }
-                    double k[3] = {H[1] * S[2] - H[2] * S[1], H[2] * S[0] - H[0] * S[2],
-                                   H[0] * S[1] - H[1] * S[0]};
+                    double k[3] = {H[j][1] * S[j][2] - H[j][2] * S[j][1], H[j][2] * S[j][0] - H[j][0] * S[j][2],
+                                   H[j][0] * S[j][1] - H[j][1] * S[j][0]};
                     if (M->alpha != 0.0) {  // mixed_lattice_md.cpp:570-578
-                        const double S2 = S[0] * S[0] + S[1] * S[1] + S[2] * S[2];
-                        const double SH = S[0] * H[0] + S[1] * H[1] + S[2] * H[2];
+                        const double S2 = S[j][0] * S[j][0] + S[j][1] * S[j][1] + S[j][2] * S[j][2];
+                        const double SH = S[j][0] * H[j][0] + S[j][1] * H[j][1] + S[j][2] * H[j][2];
                         const double g = (S2 > 0.0) ? M->alpha / sqrt(S2) : 0.0;
 #pragma unroll
-                        for (int d = 0; d < 3; ++d) k[d] += g * (S[d] * SH - H[d] * S2);
+                        for (int d = 0; d < 3; ++d) k[d] += g * (S[j][d] * SH - H[j][d] * S2);
                     }
+                    // static slot numbers keep the accumulators in VGPRs
 #pragma unroll
-                    for (int d = 0; d < 3; ++d) {
-                        const size_t q = size_t(d) * NP2 + p;
-                        if (s == 0) {
-                            acc2[j][d] = S[d] + bdt * k[d];
-                            y2[j][d] = S[d] + cdt * k[d];
-                        } else if (s < 3) {
-                            acc2[j][d] = acc2[j][d] + bdt * k[d];
-                            y2[j][d] = X[q] + cdt * k[d];
-                        } else {
-                            const double xn = acc2[j][d] + bdt * k[d];
-                            X[q] = xn;
-                            y2[j][d] = xn;
+                    for (int i = 0; i < SPT; ++i)
+                        if (i == j0 + j) {
+#pragma unroll
+                            for (int d = 0; d < 3; ++d) {
+                                acc2[i][d] = (s == 0 ? S[j][d] : acc2[i][d]) + bdt * k[d];
+                                y2[i][d] = s < 3 ? xv[d] + cdt * k[d] : acc2[i][d];
+                            }
+                            if (s == 3 && real(i)) {
+#pragma unroll
+                                for (int d = 0; d < 3; ++d) X[size_t(d) * NP2 + p] = y2[i][d];
+                            }
                         }
+                }
+            };
+            double y3[TT ? SPT : 1][8];
+            auto tm_units = [&](auto n_, int j0) __attribute__((always_inline)) {
+                constexpr int N = decltype(n_)::value;
+                const int a = atom(j0);
+                const double* hr = hrow + 3 * A2 + 8 * a;
+                double H[N][8];
+#pragma unroll
+                for (int j = 0; j < N; ++j)
+#pragma unroll
+                    for (int d = 0; d < 8; ++d) H[j][d] = hr[d];
+                F.template tm_bonds<N, TT>(a, p0 + j0 * kWave, H);
+                const cptr<MixDev> M = as_const(Mg) + opaque_zero();
+#pragma unroll
+                for (int j = 0; j < N; ++j) {
+                    const int p = p0 + (j0 + j) * kWave;
+                    double S[8];
+                    F.tm(p, S);
+                    double xv[8];
+#pragma unroll
+                    for (int d = 0; d < 8; ++d) xv[d] = S[d];
+                    if (s == 1 || s == 2) {
+#pragma unroll
+                        for (int d = 0; d < 8; ++d) xv[d] = X[o3 + size_t(d) * NP3 + p];
+                    }
+                    if (M->has_onsite3) {
+                        const cptr<double> A3m = as_const(M->onsite3) + a * 64;
+#pragma unroll
+                        for (int d = 0; d < 8; ++d)
+#pragma unroll
+                            for (int c = 0; c < 8; ++c) H[j][d] = fma(A3m[d * 8 + c], S[c], H[j][d]);
+                    }
+                    if (slot >= 0) {
+                        const double* w = wrow + 3 * A2 + 8 * a;
+#pragma unroll
+                        for (int d = 0; d < 8; ++d) e = fma(S[d], H[j][d] - w[d], e);
+                        sums3(slot, j0 + j, S);
+                    }
+                    double k[8];
+                    su3_cross(H[j], S, k);
+                    if (M->has_bloch && real(j0 + j)) {  // mixed_lattice_md.cpp:596-605
+#pragma unroll
+                        for (int d = 0; d < 8; ++d)
+                            if (M->gamma[d] != 0.0) k[d] -= M->gamma[d] * (S[d] - M->eq3[size_t(d) * NP3 + p]);
+                    }
+#pragma unroll
+                    for (int i = 0; i < SPT; ++i)
+                        if (i == j0 + j) {
+                            double y[8];
+#pragma unroll
+                            for (int d = 0; d < 8; ++d) {
+                                acc3[i][d] = (s == 0 ? S[d] : acc3[i][d]) + bdt * k[d];
+                                y[d] = s < 3 ? xv[d] + cdt * k[d] : acc3[i][d];
+                            }
+                            if (s == 3 && real(i)) {
+#pragma unroll
+                                for (int d = 0; d < 8; ++d) X[o3 + size_t(d) * NP3 + p] = y[d];
+                            }
+                            if constexpr (!GLDS) Gn[p] = make_double2(y[6], y[7]);
+                            if constexpr (TT) {
+#pragma unroll
+                                for (int d = 0; d < 8; ++d) y3[i][d] = y[d];
+                            } else {
+                                double2* r = reinterpret_cast<double2*>(smem + Y.t + 6 * p);
+#pragma unroll
+                                for (int c = 0; c < 3; ++c) r[c] = make_double2(y[2 * c], y[2 * c + 1]);
+                                if constexpr (GLDS)
+                                    *reinterpret_cast<double2*>(smem + Y.t2 + 2 * p) = make_double2(y[6], y[7]);
+                            }
+                        }
+                }
+            };
+            // units one by one, or pairs of one sublattice together
+            auto each = [&](auto&& f, int m) __attribute__((always_inline)) {
+#pragma unroll
+                for (int j0 = 0; j0 < SPT; j0 += NP_) {
+                    if (j0 >= m) break;
+                    if constexpr (NP_ == 2) {
+                        if (j0 + 1 < m && atom(j0) == atom(j0 + 1)) {
+                            f(std::integral_constant<int, 2>{}, j0);
+                        } else {
+                            f(std::integral_constant<int, 1>{}, j0);
+                            if (j0 + 1 < m) f(std::integral_constant<int, 1>{}, j0 + 1);
+                        }
+                    } else {
+                        f(std::integral_constant<int, 1>{}, j0);
                     }
                 }
-                if constexpr (TT) {
-                    // SU(3) sites read each other's stage values: every site
-                    // of both species before any new value is stored
-                    tm_sites(std::false_type{});
-                    if (obs) {
-                        const double v = wave_sum(e_acc);
-                        if (lane == 0) red[wave * kRec + 33] = v;
-                    }
-                    __syncthreads();  // every read of y_s is done
-#pragma unroll
-                    for (int j = 0; j < SPT; ++j) {
-                        const int p = fresh(tid + j * T);
-                        if ((act3 >> j) & 1u)
-#pragma unroll
-                            for (int d = 0; d < 6; ++d) TL[d * NP3 + p] = y3[j][d];
-                    }
-                } else {
-                    // no SU(3)-SU(3) bonds: an SU(3) site's own stage value
-                    // is read only by its thread, so once the SU(2) sites
-                    // are done with y_s the SU(3) sites update in place
-                    __syncthreads();  // the SU(2) sites' reads of y_s are done
-                    tm_sites(std::true_type{});
-                    if (obs) {
-                        const double v = wave_sum(e_acc);
-                        if (lane == 0) red[wave * kRec + 33] = v;
-                    }
-                    __syncthreads();  // the SU(3) sites' reads of the SU(2) stage values are done
-                }
+            };
+            each(fe_units, m2);
+            if constexpr (TT) {
+                each(tm_units, m3);
+                if (slot >= 0) sum_e(slot, e);
+                __syncthreads();  // every read of y_s is done
 #pragma unroll
                 for (int j = 0; j < SPT; ++j) {
-                    const int p = fresh(tid + j * T);
-                    if ((act2 >> j) & 1u)
+                    const int p = p0 + j * kWave;
+                    if (j >= m3) break;
+                    double2* r = reinterpret_cast<double2*>(smem + Y.t + 6 * p);
 #pragma unroll
-                        for (int d = 0; d < 3; ++d) F[d * NP2 + p] = y2[j][d];
+                    for (int c = 0; c < 3; ++c) r[c] = make_double2(y3[j][2 * c], y3[j][2 * c + 1]);
+                    if constexpr (GLDS)
+                        *reinterpret_cast<double2*>(smem + Y.t2 + 2 * p) = make_double2(y3[j][6], y3[j][7]);
                 }
-                if (obs && wave == 0 && lane < kRec) {
-                    double t = 0.0;
-                    for (int w = 0; w < nwaves; ++w) t += red[w * kRec + lane];
-                    const double sc = lane < 9 ? A.inv2 : (lane < 33 ? A.inv3 : A.invE);
-                    A.recs[(size_t(ri) * A.B_rec + b) * kRec + lane] = t * sc;
+            } else {
+                lds_barrier();  // the SU(2) sites' reads of y_s are done
+                each(tm_units, m3);
+                if (slot >= 0) sum_e(slot, e);
+                lds_barrier();  // the SU(3) sites' reads of the SU(2) stage values are done
+            }
+#pragma unroll
+            for (int j = 0; j < SPT; ++j) {
+                if (j >= m2) break;
+                double* r = smem + Y.f + 3 * (p0 + j * kWave);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) r[d] = y2[j][d];
+            }
+            // y_{s+1} complete; its components 6, 7 in global memory too
+            if constexpr (GLDS) lds_barrier();
+            else __syncthreads();
+        };
+
+        const int si = K.A.save_interval;
+        int ri = (s_begin + si - 1) / si, next_rec = ri * si;
+        for (int n0 = s_begin, cp = 0; n0 < s_end; n0 += kChunk, cp ^= 1) {
+            const int n1 = min(n0 + kChunk, s_end);
+            const int ri0 = ri;
+            write_drive(n1, cp ^ 1);
+            for (int n = n0; n < n1; ++n) {
+                const int par = (n - s_begin) & 1;
+                int slot = -1;
+                if (n == next_rec) {
+                    slot = ri - ri0;
+                    ++ri;
+                    next_rec += si;
                 }
-                __syncthreads();  // y_{s+1} complete (LDS and G)
+                const int q = n + 1 - n0;
+#pragma unroll 1
+                for (int s = 0; s < 4; ++s) {
+                    // rows of the next step: this parity's were last read a
+                    // step ago; the next chunk's envelopes are complete since
+                    // stage 0
+                    if (s == 2 && n + 1 < s_end)
+                        write_hin(q < kChunk ? Q.drv + (cp * kChunk + q) * 12 : Q.drv + (cp ^ 1) * kChunk * 12, par ^ 1);
+                    stage(s, par, s == 0 ? slot : -1);
+                    if (s == 0 && n + 1 == n1 && ri > ri0) publish(ri0, ri - ri0);
+                }
             }
         }
-        if (post >= 0) {
+
+        const MixArgsP G = mix_kern_args();
+        if (P.post >= 0) {
             // hand the state at s_end (in X since the last step's stage 3)
             // to the workgroup that continues the trajectory
             __threadfence();
             __syncthreads();
-            if (tid == 0) __hip_atomic_store(A.flags + post, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+            if (tid == 0) __hip_atomic_store(G->A.flags + P.post, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
         }
         // final record: the state after the last step (the stage values of
-        // the next step's stage 0: LDS and G[0])
-        if (s_end == A.n_steps) {
-            const MP M = fresh_mix(Mg);
-            const MixStageView V{F, TL, Gw, NP2, NP3};
-            observe<SPT, T>(M, V, tid, lane, wave, at2, at3, act2, act3, red);
-            double e_acc = 0.0;
+        // the next step's stage 0), undriven
+        if (s_end == G->A.n_steps) {
+            const Field<Z22, ZM, GLDS> F{Mg, smem, Y, GLDS ? nullptr : Gw};
+            double e = 0.0;
+#pragma unroll 1
+            for (int j = 0; j < m2; ++j) {
+                const int p = p0 + j * kWave, a = atom(j);
+                double S[1][3], H[1][3];
+                ld3(smem + Y.f + 3 * p, S[0]);
 #pragma unroll
-            for (int j = 0; j < SPT; ++j) {
-                if (!((act2 >> j) & 1u)) continue;
-                const int p = fresh(tid + j * T), a = at2[j];
-                const double S[3] = {V.fe(0, p), V.fe(1, p), V.fe(2, p)};
-                double H[3];
-                fe_field(Mg, V, a, p, S, H);
-                e_acc += site_energy_mixed<3>(M->field2, a, S, H);
-            }
+                for (int d = 0; d < 3; ++d) H[0][d] = -Q.cst[3 * (3 * a + d)];
+                F.template fe<1>(a, p, S, H);
 #pragma unroll
-            for (int j = 0; j < SPT; ++j) {
-                if (!((act3 >> j) & 1u)) continue;
-                const int p = fresh(tid + j * T), a = at3[j];
-                double S[8];
+                for (int d = 0; d < 3; ++d) e = fma(S[0][d], H[0][d] - Q.cst[3 * (3 * a + d)], e);
+                sums2(0, j, S[0]);
+            }
+#pragma unroll 1
+            for (int j = 0; j < m3; ++j) {
+                const int p = p0 + j * kWave, a = atom(j);
+                const double* c3 = Q.cst + 3 * (3 * A2 + 8 * a);
+                double S[8], H[1][8];
+                F.tm(p, S);
 #pragma unroll
-                for (int c = 0; c < 8; ++c) S[c] = V.tm(c, p);
-                double H[8];
-                tm_field<TT>(Mg, V, a, p, S, H);
-                e_acc += site_energy_mixed<8>(M->field3, a, S, H);
+                for (int d = 0; d < 8; ++d) H[0][d] = -c3[3 * d];
+                F.template tm_bonds<1, TT>(a, p, H);
+                if (M0->has_onsite3) {
+                    const cptr<double> A3m = as_const(M0->onsite3) + a * 64;
+#pragma unroll
+                    for (int d = 0; d < 8; ++d)
+#pragma unroll
+                        for (int c = 0; c < 8; ++c) H[0][d] = fma(A3m[d * 8 + c], S[c], H[0][d]);
+                }
+#pragma unroll
+                for (int d = 0; d < 8; ++d) e = fma(S[d], H[0][d] - c3[3 * d], e);
+                sums3(0, j, S);
             }
-            const double v = wave_sum(e_acc);
-            if (lane == 0) red[wave * kRec + 33] = v;
-            __syncthreads();
-            if (wave == 0 && lane < kRec) {
-                double t = 0.0;
-                for (int w = 0; w < nwaves; ++w) t += red[w * kRec + lane];
-                const double sc = lane < 9 ? A.inv2 : (lane < 33 ? A.inv3 : A.invE);
-                A.recs[(size_t(A.n_rec - 1) * A.B_rec + b) * kRec + lane] = t * sc;
-            }
+            sum_e(0, e);
+            lds_barrier();
+            publish(G->A.n_rec - 1, 1);
         }
     }
 }
 
 namespace {
 
-template <int SPT, int T, bool TT>
+template <int SPT, int T, int Z22, int ZM, bool TT, bool GLDS>
 hipError_t launch_mp(const MixDev* M, const MixPersistArgs& A, int grid, size_t lds, hipStream_t st, int* occ) {
-    auto kern = k_mixed_persist<SPT, T, TT>;
+    auto kern = k_mixed_persist<SPT, T, Z22, ZM, TT, GLDS>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
     if (occ) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, kern, T, lds);
-    hipLaunchKernelGGL(kern, dim3(unsigned(grid)), dim3(T), lds, st, M, A);
+    const MixKernArgs K{M, A};
+    hipLaunchKernelGGL(kern, dim3(unsigned(grid)), dim3(T), lds, st, K);
     return hipGetLastError();
+}
+
+// components 6 and 7 in LDS where they fit: always up to 1024 sites of each
+// species (two units per wave of 512 threads, one of 1024)
+template <int SPT, int T, int Z22, int ZM, bool TT>
+hipError_t launch_mp_g(const MixDev& Mh, const MixDev* M, const MixPersistArgs& A, int grid, hipStream_t st, int* occ) {
+    const size_t in_lds = mixed_persist_lds_bytes(Mh, T, true);
+    if (in_lds <= 160 * 1024) return launch_mp<SPT, T, Z22, ZM, TT, true>(M, A, grid, in_lds, st, occ);
+    if constexpr (SPT * T > 1024)
+        return launch_mp<SPT, T, Z22, ZM, TT, false>(M, A, grid, mixed_persist_lds_bytes(Mh, T, false), st, occ);
+    return hipErrorInvalidValue;
+}
+
+template <int SPT>
+hipError_t launch_mp_z(const MixDev& Mh, const MixDev* M, const MixPersistArgs& A, int grid, hipStream_t st, int* occ) {
+    if (Mh.jzm == 4) {
+        return Mh.jz22 == 6 ? launch_mp_g<SPT, 1024, 6, 4, false>(Mh, M, A, grid, st, occ)
+                            : launch_mp_g<SPT, 1024, 8, 4, false>(Mh, M, A, grid, st, occ);
+    }
+    return Mh.jz22 == 6 ? launch_mp_g<SPT, 1024, 6, 8, false>(Mh, M, A, grid, st, occ)
+                        : launch_mp_g<SPT, 1024, 8, 8, false>(Mh, M, A, grid, st, occ);
 }
 
 }  // namespace
 
 // Without SU(3)-SU(3) bonds: 1024 threads (4 waves per SIMD) and up to two
-// sites of each species per thread — the SU(3) sites update in place, so a
+// units of each species per wave — the SU(3) sites update in place, so a
 // thread holds only its accumulators and its SU(2) sites' next values.  With
-// them: 512 threads and up to four sites (the SU(3) next values are held too).
-MixPersistShape mixed_persist_shape(int NP2, int NP3, bool tt) {
-    const int np = std::max(NP2, NP3);
+// them: 512 threads and up to four units (the SU(3) next values are held
+// too).  Lattices of at most 16 units (both species together) whose stage
+// values fit LDS twice take the one-unit-per-wave kernel.
+MixPersistShape mixed_persist_shape(const MixDev& M, bool tt) {
+    const int units = (M.NP2 + M.NP3) / kWave, np = std::max(M.NP2, M.NP3);
+    if (!M.jpad) return {0, 0, tt, false};
+    if (units <= 16 && mixed_waves_lds_bytes(M) <= 160 * 1024) return {units * kWave, 1, tt, true};
+    MixPersistShape sh{0, 0, tt, false};
     if (!tt) {
-        if (np <= 1024) return {1024, 1, false};
-        if (np <= 2048) return {1024, 2, false};
-        return {0, 0, false};
+        if (np <= 2048) sh = {1024, np <= 1024 ? 1 : 2, false, false};
+    } else {
+        const int spt = (np + 511) / 512;
+        if (spt <= 4) sh = {512, spt, true, false};
     }
-    const int spt = (np + 511) / 512;
-    if (spt <= 4) return {512, spt, true};
-    return {0, 0, true};
+    if (sh.block && mixed_persist_lds_bytes(M, sh.block, false) > 160 * 1024) sh = {0, 0, tt, false};
+    return sh;
 }
 
-size_t mixed_persist_lds_bytes(int NP2, int NP3, int block) {
-    return sizeof(double) * (3 * size_t(NP2) + 6 * size_t(NP3) + size_t(block / kWave) * kRec);
+size_t mixed_persist_lds_bytes(const MixDev& M, int block, bool glds) {
+    return sizeof(double) * size_t(Lay(M.NP2, M.NP3, M.A2, M.A3, block / kWave, glds).total);
 }
 
 hipError_t launch_mixed_persist(const MixDev& Mh, const MixDev* M, const MixPersistArgs& A, const MixPersistShape& sh,
                                 int grid, hipStream_t st, int* occ) {
-    const size_t lds = mixed_persist_lds_bytes(Mh.NP2, Mh.NP3, sh.block);
     if (!sh.tt && sh.block == 1024) {
-        if (sh.spt == 1) return launch_mp<1, 1024, false>(M, A, grid, lds, st, occ);
-        if (sh.spt == 2) return launch_mp<2, 1024, false>(M, A, grid, lds, st, occ);
+        if (sh.spt == 1) return launch_mp_z<1>(Mh, M, A, grid, st, occ);
+        if (sh.spt == 2) return launch_mp_z<2>(Mh, M, A, grid, st, occ);
     }
-    if (sh.tt && sh.block == 512) {
+    if (sh.tt && sh.block == 512 && Mh.jz22 == 8 && Mh.jzm == 8) {
         switch (sh.spt) {
-            case 1: return launch_mp<1, 512, true>(M, A, grid, lds, st, occ);
-            case 2: return launch_mp<2, 512, true>(M, A, grid, lds, st, occ);
-            case 3: return launch_mp<3, 512, true>(M, A, grid, lds, st, occ);
-            case 4: return launch_mp<4, 512, true>(M, A, grid, lds, st, occ);
+            case 1: return launch_mp_g<1, 512, 8, 8, true>(Mh, M, A, grid, st, occ);
+            case 2: return launch_mp_g<2, 512, 8, 8, true>(Mh, M, A, grid, st, occ);
+            case 3: return launch_mp_g<3, 512, 8, 8, true>(Mh, M, A, grid, st, occ);
+            case 4: return launch_mp_g<4, 512, 8, 8, true>(Mh, M, A, grid, st, occ);
             default: break;
         }
     }

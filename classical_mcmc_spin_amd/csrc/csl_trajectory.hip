@@ -22,7 +22,7 @@
 //     act on those sums, for a chunk of records at once and one wave per
 //     record.
 #include "csl_device.hpp"
-#include "csl_lds.hpp"
+#include "csl_record.hpp"
 
 #ifndef CSL_SPT
 #error "CSL_SPT (sites per thread) must be defined by the build"
@@ -31,38 +31,6 @@
 namespace csl {
 
 namespace {
-
-// Orders the LDS accesses of the workgroup: what __syncthreads does without
-// waiting for global stores (the records' own stores stay in flight).
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// v + w with the upper half of the wave taken from the partner operand:
-// lanes 0..31 hold v summed over the two halves, lanes 32..63 w.
-__device__ __forceinline__ double fold_halves(double v, double w) {
-    auto lo = __builtin_amdgcn_permlane32_swap(unsigned(__double2loint(v)), unsigned(__double2loint(w)), false, false);
-    auto hi = __builtin_amdgcn_permlane32_swap(unsigned(__double2hiint(v)), unsigned(__double2hiint(w)), false, false);
-    return __hiloint2double(int(hi[0]), int(lo[0])) + __hiloint2double(int(hi[1]), int(lo[1]));
-}
-
-// The same between neighbouring rows of 16 lanes: even rows v, odd rows w.
-__device__ __forceinline__ double fold_rows(double v, double w) {
-    auto lo = __builtin_amdgcn_permlane16_swap(unsigned(__double2loint(v)), unsigned(__double2loint(w)), false, false);
-    auto hi = __builtin_amdgcn_permlane16_swap(unsigned(__double2hiint(v)), unsigned(__double2hiint(w)), false, false);
-    return __hiloint2double(int(hi[0]), int(lo[0])) + __hiloint2double(int(hi[1]), int(lo[1]));
-}
-
-// Sum over the 16 lanes of a row, in every lane of the row.
-__device__ __forceinline__ double row_sum(double v) {
-    v += dpp_f64<0xB1, 0xf>(v);   // quad_perm [1,0,3,2]
-    v += dpp_f64<0x4E, 0xf>(v);   // quad_perm [2,3,0,1]
-    v += dpp_f64<0x124, 0xf>(v);  // row_ror:4
-    v += dpp_f64<0x128, 0xf>(v);  // row_ror:8
-    return v;
-}
 
 // The kernel's argument block, read back from the kernel argument segment
 // where it is used: the compiler cannot carry the scalars of rarely taken
@@ -240,12 +208,7 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
 
         // four sums of the wave (S and e) into red[slot][wave]
         auto reduce_obs = [&](int slot, const double s[3], double e) {
-            const double v = row_sum(fold_rows(fold_halves(s[0], s[1]), fold_halves(s[2], e)));
-            // rows hold Sx, Sz, Sy, e
-            if ((lane & 15) == 0) {
-                const int r = lane >> 4;
-                red[(slot * nwaves + wave) * 4 + ((r & 1) << 1 | r >> 1)] = v;
-            }
+            wave_sum4(s[0], s[1], s[2], e, lane, red + (slot * nwaves + wave) * 4);
         };
         // records ri0 .. ri0 + cnt - 1 from red[0 .. cnt-1], one wave each
         auto publish = [&](int ri0, int cnt) {
