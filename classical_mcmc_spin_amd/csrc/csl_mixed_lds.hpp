@@ -54,6 +54,14 @@ __device__ __forceinline__ void st8(double* r6, double* r2, const double v[8]) {
     *reinterpret_cast<double2*>(r2) = make_double2(v[6], v[7]);
 }
 
+// Ends a bond: the field values as they are now (the products cannot be put
+// off past this point, with the bond's matrix saved for later).
+template <int D>
+__device__ __forceinline__ void end_bond(double (&H)[D]) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) asm volatile("" : "+v"(H[d]));
+}
+
 // The small LDS tables of a trajectory, `chunk` steps' envelopes and records
 // at a time.
 struct MixTables {

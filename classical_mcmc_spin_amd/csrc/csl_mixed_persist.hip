@@ -22,15 +22,17 @@
 // the owner reads an SU(3) site's own value then) -> barrier -> the SU(2)
 // next values into LDS -> barrier.  With them (TT) both species' next values
 // are held until one barrier.  A wave owns SPT consecutive units of 64 sites
-// of each species; two units of one sublattice are advanced together, so
-// their bond matrices (scalar loads) are fetched once.
+// of each species and advances them one by one (two of one sublattice
+// together, their bond matrices fetched once, spilled: 33.5 against 28.5 us
+// a stage of the 8x8x8 cell).
 //
 // Field rows, pulse envelopes and records are handled as in
 // csl_trajectory.hip: rows of -(B + drive) from LDS, envelopes of two steps
 // at a time, records from the waves' sums of S and S.H, two at a time.  With
 // every record's 33 wave sums in shuffles, an envelope evaluation per wave
 // and stage, one 4-byte partner load per bond and one 8-byte access per
-// component a stage of the 8x8x8 cell took 36.8 us.
+// component a stage of the 8x8x8 cell took 36.8 us; it takes 28 (a third of
+// the cycles issue FP64 work; x from global memory costs 3.6 of them).
 #include <algorithm>
 #include <type_traits>
 
@@ -67,16 +69,6 @@ struct Lay {
     }
 };
 
-// Ends a bond: the field values as they are now (the products cannot be put
-// off past this point, with the bond's matrix saved for later).
-template <int N, int D>
-__device__ __forceinline__ void end_bond(double (*H)[D]) {
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-#pragma unroll
-        for (int d = 0; d < D; ++d) asm volatile("" : "+v"(H[j][d]));
-}
-
 template <int Z22, int ZM, bool GLDS>
 struct Field {
     const MixDev* Mg;
@@ -97,120 +89,102 @@ struct Field {
         v[7] = a.y;
     }
 
-    // fields of N units of SU(2) sublattice a at sites p, p + 64, ...  The
-    // bonds are kept apart (an opaque address each, end_bond):
-    // the compiler otherwise loads every bond's matrix at once and spills them
-    template <int N>
-    __device__ __forceinline__ void fe(int a, int p, const double (*S)[3], double (*H)[3]) const {
+    // field of SU(2) site p of sublattice a.  The bonds are kept apart (an
+    // opaque address each, end_bond): the compiler otherwise loads every
+    // bond's matrix at once and spills them
+    __device__ __forceinline__ void fe(int a, int p, const double S[3], double (&H)[3]) const {
         const cptr<MixDev> M = as_const(Mg) + opaque_zero();
-        int q22[N][8], q23[N][8];
+        int q22[8], q23[8];
+        unpack8(M->q23[p], q23);
+        unpack8(M->q22[p], q22);
+        // components 6 and 7 of the next kAhead SU(3) partners are on their
+        // way from global memory (L2), the first ones while the SU(2) bonds run
+        constexpr int kAhead = GLDS ? 1 : 4;
+        double2 gl[kAhead];
+        if constexpr (!GLDS) {
 #pragma unroll
-        for (int j = 0; j < N; ++j) {
-            unpack8(M->q22[p + j * kWave], q22[j]);
-            unpack8(M->q23[p + j * kWave], q23[j]);
+            for (int k = 0; k < kAhead; ++k) gl[k] = g[q23[k]];
         }
         if (M->has_onsite2) {
             const cptr<double> A2 = as_const(M->onsite2) + a * 9;
 #pragma unroll
-            for (int j = 0; j < N; ++j)
+            for (int d = 0; d < 3; ++d)
 #pragma unroll
-                for (int d = 0; d < 3; ++d)
-#pragma unroll
-                    for (int e = 0; e < 3; ++e) H[j][d] = fma(A2[d * 3 + e], S[j][e], H[j][d]);
-        }
-        // components 6 and 7 of the SU(3) partners from global memory: in
-        // flight while the SU(2) bonds run
-        double2 gl[GLDS ? 1 : N][GLDS ? 1 : ZM];
-        if constexpr (!GLDS) {
-#pragma unroll
-            for (int j = 0; j < N; ++j)
-#pragma unroll
-                for (int k = 0; k < ZM; ++k) gl[j][k] = g[q23[j][k]];
+                for (int e = 0; e < 3; ++e) H[d] = fma(A2[d * 3 + e], S[e], H[d]);
         }
         const cptr<double> jp = as_const(M->jpad);
         const int j2 = M->j22off + a * (Z22 * 9), j3 = a * (ZM * 24);
 #pragma unroll
         for (int k = 0; k < Z22; ++k) {
-            const cptr<double> J2 = jp + j2 + k * 9 + opaque_zero();
+            const cptr<double> J = jp + j2 + k * 9 + opaque_zero();
+            double s[3];
+            ld3(smem + Y.f + 3 * q22[k], s);
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                double s[3];
-                ld3(smem + Y.f + 3 * q22[j][k], s);
+            for (int e = 0; e < 3; ++e)
 #pragma unroll
-                for (int e = 0; e < 3; ++e)
-#pragma unroll
-                    for (int d = 0; d < 3; ++d) H[j][d] = fma(J2[d * 3 + e], s[e], H[j][d]);
-            }
-            end_bond<N, 3>(H);
+                for (int d = 0; d < 3; ++d) H[d] = fma(J[d * 3 + e], s[e], H[d]);
+            end_bond(H);
         }
 #pragma unroll
         for (int k = 0; k < ZM; ++k) {
-            const cptr<double> J3 = jp + j3 + k * 24 + opaque_zero();
+            const cptr<double> J = jp + j3 + k * 24 + opaque_zero();
+            double s[8];
+            const double2* r = reinterpret_cast<const double2*>(smem + Y.t + 6 * q23[k]);
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                const int q = q23[j][k];
-                double s[8];
-                const double2* r = reinterpret_cast<const double2*>(smem + Y.t + 6 * q);
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    const double2 v = r[i];
-                    s[2 * i] = v.x;
-                    s[2 * i + 1] = v.y;
-                }
-                const double2 v = GLDS ? *reinterpret_cast<const double2*>(smem + Y.t2 + 2 * q) : gl[GLDS ? 0 : j][GLDS ? 0 : k];
-                s[6] = v.x;
-                s[7] = v.y;
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-#pragma unroll
-                    for (int d = 0; d < 3; ++d) H[j][d] = fma(J3[d * 8 + e], s[e], H[j][d]);
+            for (int i = 0; i < 3; ++i) {
+                const double2 v = r[i];
+                s[2 * i] = v.x;
+                s[2 * i + 1] = v.y;
             }
-            end_bond<N, 3>(H);
+            const double2 v = GLDS ? *reinterpret_cast<const double2*>(smem + Y.t2 + 2 * q23[k]) : gl[GLDS ? 0 : k % kAhead];
+            if constexpr (!GLDS)
+                if (k + kAhead < ZM) gl[k % kAhead] = g[q23[k + kAhead]];
+            s[6] = v.x;
+            s[7] = v.y;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) H[d] = fma(J[d * 8 + e], s[e], H[d]);
+            end_bond(H);
         }
     }
 
-    // bond fields of N units of SU(3) sublattice a (the on-site part apart)
-    template <int N, bool TT>
-    __device__ __forceinline__ void tm_bonds(int a, int p, double (*H)[8]) const {
+    // bond field of SU(3) site p of sublattice a (the on-site part apart)
+    template <bool TT>
+    __device__ __forceinline__ void tm_bonds(int a, int p, double (&H)[8]) const {
         const cptr<MixDev> M = as_const(Mg) + opaque_zero();
-        int q32[N][8];
+        int q32[8], off[ZM];
+        unpack8(M->q32[p], q32);
 #pragma unroll
-        for (int j = 0; j < N; ++j) unpack8(M->q32[p + j * kWave], q32[j]);
+        for (int k = 0; k < ZM; ++k) off[k] = (as_const(M->j32pad) + a * ZM)[k];
+        const cptr<double> jp = as_const(M->jpad);
         if constexpr (TT) {
             const int c33 = uniform(as_const(M->e33.cnt_atom)[a]);
+            const uint2 v = M->q33[p];
+            const int q33[4] = {lo16(v.x), hi16(v.x), lo16(v.y), hi16(v.y)};
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                const uint2 v = M->q33[p + j * kWave];
-                const int q33[4] = {lo16(v.x), hi16(v.x), lo16(v.y), hi16(v.y)};
+            for (int k = 0; k < kMixZ33; ++k) {
+                if (k < c33) {
+                    double s[8];
+                    tm(q33[k], s);
+                    const cptr<double> J = as_const(M->e33.mats) + (a * M->e33.zmax + k) * 64;
 #pragma unroll
-                for (int k = 0; k < kMixZ33; ++k) {
-                    if (k < c33) {
-                        double s[8];
-                        tm(q33[k], s);
-                        const cptr<double> J = as_const(M->e33.mats) + (a * M->e33.zmax + k) * 64;
+                    for (int d = 0; d < 8; ++d)
 #pragma unroll
-                        for (int d = 0; d < 8; ++d)
-#pragma unroll
-                            for (int e = 0; e < 8; ++e) H[j][d] = fma(J[d * 8 + e], s[e], H[j][d]);
-                    }
+                        for (int e = 0; e < 8; ++e) H[d] = fma(J[d * 8 + e], s[e], H[d]);
                 }
             }
         }
-        const cptr<int> off = as_const(M->j32pad) + a * ZM;
-        const cptr<double> jp = as_const(M->jpad);
 #pragma unroll
         for (int k = 0; k < ZM; ++k) {
             const cptr<double> J = jp + uniform(off[k]) + opaque_zero();
+            double s[3];
+            ld3(smem + Y.f + 3 * q32[k], s);
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                double s[3];
-                ld3(smem + Y.f + 3 * q32[j][k], s);
+            for (int e = 0; e < 3; ++e)
 #pragma unroll
-                for (int e = 0; e < 3; ++e)
-#pragma unroll
-                    for (int d = 0; d < 8; ++d) H[j][d] = fma(J[e * 8 + d], s[e], H[j][d]);
-            }
-            end_bond<N, 8>(H);
+                for (int d = 0; d < 8; ++d) H[d] = fma(J[e * 8 + d], s[e], H[d]);
+            end_bond(H);
         }
     }
 };
@@ -221,7 +195,6 @@ template <int SPT, int T, int Z22, int ZM, bool TT, bool GLDS>
 __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
     extern __shared__ double smem[];
     constexpr int nwaves = T / kWave;
-    constexpr int NP_ = (SPT % 2 == 0 && !TT) ? 2 : 1;   // units advanced together where their sublattice agrees
     const MixDev* const Mg = K.M;
     const cptr<MixDev> M0 = as_const(Mg);
     const int tid = threadIdx.x;
@@ -330,147 +303,103 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
             double2* const Gn = GLDS ? nullptr : Gw + (1 - (s & 1)) * NP3;
             double e = 0.0;
             double y2[SPT][3];
-            auto fe_units = [&](auto n_, int j0) __attribute__((always_inline)) {
-                constexpr int N = decltype(n_)::value;
-                const int a = atom(j0);
-                double S[N][3], H[N][3];
-#pragma unroll
-                for (int j = 0; j < N; ++j) {
-                    ld3(smem + Y.f + 3 * (p0 + (j0 + j) * kWave), S[j]);
-#pragma unroll
-                    for (int d = 0; d < 3; ++d) H[j][d] = hrow[3 * a + d];
-                }
-                F.template fe<N>(a, p0 + j0 * kWave, S, H);
+            auto fe_unit = [&](int j) __attribute__((always_inline)) {
+                const int p = p0 + j * kWave, a = atom(j);
                 const cptr<MixDev> M = as_const(Mg) + opaque_zero();
+                double S[3], H[3], xv[3];
+                ld3(smem + Y.f + 3 * p, S);
 #pragma unroll
-                for (int j = 0; j < N; ++j) {
-                    const int p = p0 + (j0 + j) * kWave;
-                    if (slot >= 0) {
+                for (int d = 0; d < 3; ++d) {
+                    H[d] = hrow[3 * a + d];
+                    // x in flight while the bonds run
+                    xv[d] = (s == 1 || s == 2) ? X[size_t(d) * NP2 + p] : S[d];
+                }
+                F.fe(a, p, S, H);
+                if (slot >= 0) {
 #pragma unroll
-                        for (int d = 0; d < 3; ++d) e = fma(S[j][d], H[j][d] - wrow[3 * a + d], e);
-                        sums2(slot, j0 + j, S[j]);
-                    }
-                    double xv[3] = {S[j][0], S[j][1], S[j][2]};
-                    if (s == 1 || s == 2) {
+                    for (int d = 0; d < 3; ++d) e = fma(S[d], H[d] - wrow[3 * a + d], e);
+                    sums2(slot, j, S);
+                }
+                double k[3] = {H[1] * S[2] - H[2] * S[1], H[2] * S[0] - H[0] * S[2], H[0] * S[1] - H[1] * S[0]};
+                if (M->alpha != 0.0) {  // mixed_lattice_md.cpp:570-578
+                    const double S2 = S[0] * S[0] + S[1] * S[1] + S[2] * S[2];
+                    const double SH = S[0] * H[0] + S[1] * H[1] + S[2] * H[2];
+                    const double g = (S2 > 0.0) ? M->alpha / sqrt(S2) : 0.0;
 #pragma unroll
-                        for (int d = 0; d < 3; ++d) xv[d] = X[size_t(d) * NP2 + p];
-                    }
-                    double k[3] = {H[j][1] * S[j][2] - H[j][2] * S[j][1], H[j][2] * S[j][0] - H[j][0] * S[j][2],
-                                   H[j][0] * S[j][1] - H[j][1] * S[j][0]};
-                    if (M->alpha != 0.0) {  // mixed_lattice_md.cpp:570-578
-                        const double S2 = S[j][0] * S[j][0] + S[j][1] * S[j][1] + S[j][2] * S[j][2];
-                        const double SH = S[j][0] * H[j][0] + S[j][1] * H[j][1] + S[j][2] * H[j][2];
-                        const double g = (S2 > 0.0) ? M->alpha / sqrt(S2) : 0.0;
+                    for (int d = 0; d < 3; ++d) k[d] += g * (S[d] * SH - H[d] * S2);
+                }
 #pragma unroll
-                        for (int d = 0; d < 3; ++d) k[d] += g * (S[j][d] * SH - H[j][d] * S2);
-                    }
-                    // static slot numbers keep the accumulators in VGPRs
+                for (int d = 0; d < 3; ++d) {
+                    acc2[j][d] = (s == 0 ? S[d] : acc2[j][d]) + bdt * k[d];
+                    y2[j][d] = s < 3 ? xv[d] + cdt * k[d] : acc2[j][d];
+                }
+                if (s == 3 && real(j)) {
 #pragma unroll
-                    for (int i = 0; i < SPT; ++i)
-                        if (i == j0 + j) {
-#pragma unroll
-                            for (int d = 0; d < 3; ++d) {
-                                acc2[i][d] = (s == 0 ? S[j][d] : acc2[i][d]) + bdt * k[d];
-                                y2[i][d] = s < 3 ? xv[d] + cdt * k[d] : acc2[i][d];
-                            }
-                            if (s == 3 && real(i)) {
-#pragma unroll
-                                for (int d = 0; d < 3; ++d) X[size_t(d) * NP2 + p] = y2[i][d];
-                            }
-                        }
+                    for (int d = 0; d < 3; ++d) X[size_t(d) * NP2 + p] = y2[j][d];
                 }
             };
             double y3[TT ? SPT : 1][8];
-            auto tm_units = [&](auto n_, int j0) __attribute__((always_inline)) {
-                constexpr int N = decltype(n_)::value;
-                const int a = atom(j0);
-                const double* hr = hrow + 3 * A2 + 8 * a;
-                double H[N][8];
-#pragma unroll
-                for (int j = 0; j < N; ++j)
-#pragma unroll
-                    for (int d = 0; d < 8; ++d) H[j][d] = hr[d];
-                F.template tm_bonds<N, TT>(a, p0 + j0 * kWave, H);
+            auto tm_unit = [&](int j) __attribute__((always_inline)) {
+                const int p = p0 + j * kWave, a = atom(j);
                 const cptr<MixDev> M = as_const(Mg) + opaque_zero();
+                const double* hr = hrow + 3 * A2 + 8 * a;
+                double H[8], xv[8];
 #pragma unroll
-                for (int j = 0; j < N; ++j) {
-                    const int p = p0 + (j0 + j) * kWave;
-                    double S[8];
-                    F.tm(p, S);
-                    double xv[8];
+                for (int d = 0; d < 8; ++d) {
+                    H[d] = hr[d];
+                    xv[d] = (s == 1 || s == 2) ? X[o3 + size_t(d) * NP3 + p] : 0.0;
+                }
+                F.template tm_bonds<TT>(a, p, H);
+                double S[8];
+                F.tm(p, S);
+                if (M->has_onsite3) {
+                    const cptr<double> A3m = as_const(M->onsite3) + a * 64;
 #pragma unroll
-                    for (int d = 0; d < 8; ++d) xv[d] = S[d];
-                    if (s == 1 || s == 2) {
+                    for (int d = 0; d < 8; ++d)
 #pragma unroll
-                        for (int d = 0; d < 8; ++d) xv[d] = X[o3 + size_t(d) * NP3 + p];
-                    }
-                    if (M->has_onsite3) {
-                        const cptr<double> A3m = as_const(M->onsite3) + a * 64;
+                        for (int c = 0; c < 8; ++c) H[d] = fma(A3m[d * 8 + c], S[c], H[d]);
+                }
+                if (slot >= 0) {
+                    const double* w = wrow + 3 * A2 + 8 * a;
 #pragma unroll
-                        for (int d = 0; d < 8; ++d)
+                    for (int d = 0; d < 8; ++d) e = fma(S[d], H[d] - w[d], e);
+                    sums3(slot, j, S);
+                }
+                double k[8];
+                su3_cross(H, S, k);
+                if (M->has_bloch && real(j)) {  // mixed_lattice_md.cpp:596-605
 #pragma unroll
-                            for (int c = 0; c < 8; ++c) H[j][d] = fma(A3m[d * 8 + c], S[c], H[j][d]);
-                    }
-                    if (slot >= 0) {
-                        const double* w = wrow + 3 * A2 + 8 * a;
+                    for (int d = 0; d < 8; ++d)
+                        if (M->gamma[d] != 0.0) k[d] -= M->gamma[d] * (S[d] - M->eq3[size_t(d) * NP3 + p]);
+                }
+                double y[8];
 #pragma unroll
-                        for (int d = 0; d < 8; ++d) e = fma(S[d], H[j][d] - w[d], e);
-                        sums3(slot, j0 + j, S);
-                    }
-                    double k[8];
-                    su3_cross(H[j], S, k);
-                    if (M->has_bloch && real(j0 + j)) {  // mixed_lattice_md.cpp:596-605
+                for (int d = 0; d < 8; ++d) {
+                    acc3[j][d] = (s == 0 ? S[d] : acc3[j][d]) + bdt * k[d];
+                    y[d] = s < 3 ? (s == 0 ? S[d] : xv[d]) + cdt * k[d] : acc3[j][d];
+                }
+                if (s == 3 && real(j)) {
 #pragma unroll
-                        for (int d = 0; d < 8; ++d)
-                            if (M->gamma[d] != 0.0) k[d] -= M->gamma[d] * (S[d] - M->eq3[size_t(d) * NP3 + p]);
-                    }
+                    for (int d = 0; d < 8; ++d) X[o3 + size_t(d) * NP3 + p] = y[d];
+                }
+                if constexpr (!GLDS) Gn[p] = make_double2(y[6], y[7]);
+                if constexpr (TT) {
 #pragma unroll
-                    for (int i = 0; i < SPT; ++i)
-                        if (i == j0 + j) {
-                            double y[8];
+                    for (int d = 0; d < 8; ++d) y3[j][d] = y[d];
+                } else {
+                    double2* r = reinterpret_cast<double2*>(smem + Y.t + 6 * p);
 #pragma unroll
-                            for (int d = 0; d < 8; ++d) {
-                                acc3[i][d] = (s == 0 ? S[d] : acc3[i][d]) + bdt * k[d];
-                                y[d] = s < 3 ? xv[d] + cdt * k[d] : acc3[i][d];
-                            }
-                            if (s == 3 && real(i)) {
-#pragma unroll
-                                for (int d = 0; d < 8; ++d) X[o3 + size_t(d) * NP3 + p] = y[d];
-                            }
-                            if constexpr (!GLDS) Gn[p] = make_double2(y[6], y[7]);
-                            if constexpr (TT) {
-#pragma unroll
-                                for (int d = 0; d < 8; ++d) y3[i][d] = y[d];
-                            } else {
-                                double2* r = reinterpret_cast<double2*>(smem + Y.t + 6 * p);
-#pragma unroll
-                                for (int c = 0; c < 3; ++c) r[c] = make_double2(y[2 * c], y[2 * c + 1]);
-                                if constexpr (GLDS)
-                                    *reinterpret_cast<double2*>(smem + Y.t2 + 2 * p) = make_double2(y[6], y[7]);
-                            }
-                        }
+                    for (int c = 0; c < 3; ++c) r[c] = make_double2(y[2 * c], y[2 * c + 1]);
+                    if constexpr (GLDS) *reinterpret_cast<double2*>(smem + Y.t2 + 2 * p) = make_double2(y[6], y[7]);
                 }
             };
-            // units one by one, or pairs of one sublattice together
-            auto each = [&](auto&& f, int m) __attribute__((always_inline)) {
 #pragma unroll
-                for (int j0 = 0; j0 < SPT; j0 += NP_) {
-                    if (j0 >= m) break;
-                    if constexpr (NP_ == 2) {
-                        if (j0 + 1 < m && atom(j0) == atom(j0 + 1)) {
-                            f(std::integral_constant<int, 2>{}, j0);
-                        } else {
-                            f(std::integral_constant<int, 1>{}, j0);
-                            if (j0 + 1 < m) f(std::integral_constant<int, 1>{}, j0 + 1);
-                        }
-                    } else {
-                        f(std::integral_constant<int, 1>{}, j0);
-                    }
-                }
-            };
-            each(fe_units, m2);
+            for (int j = 0; j < SPT; ++j)
+                if (j < m2) fe_unit(j);
             if constexpr (TT) {
-                each(tm_units, m3);
+#pragma unroll
+                for (int j = 0; j < SPT; ++j)
+                    if (j < m3) tm_unit(j);
                 if (slot >= 0) sum_e(slot, e);
                 __syncthreads();  // every read of y_s is done
 #pragma unroll
@@ -485,7 +414,9 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
                 }
             } else {
                 lds_barrier();  // the SU(2) sites' reads of y_s are done
-                each(tm_units, m3);
+#pragma unroll
+                for (int j = 0; j < SPT; ++j)
+                    if (j < m3) tm_unit(j);
                 if (slot >= 0) sum_e(slot, e);
                 lds_barrier();  // the SU(3) sites' reads of the SU(2) stage values are done
             }
@@ -545,33 +476,33 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
 #pragma unroll 1
             for (int j = 0; j < m2; ++j) {
                 const int p = p0 + j * kWave, a = atom(j);
-                double S[1][3], H[1][3];
-                ld3(smem + Y.f + 3 * p, S[0]);
+                double S[3], H[3];
+                ld3(smem + Y.f + 3 * p, S);
 #pragma unroll
-                for (int d = 0; d < 3; ++d) H[0][d] = -Q.cst[3 * (3 * a + d)];
-                F.template fe<1>(a, p, S, H);
+                for (int d = 0; d < 3; ++d) H[d] = -Q.cst[3 * (3 * a + d)];
+                F.fe(a, p, S, H);
 #pragma unroll
-                for (int d = 0; d < 3; ++d) e = fma(S[0][d], H[0][d] - Q.cst[3 * (3 * a + d)], e);
-                sums2(0, j, S[0]);
+                for (int d = 0; d < 3; ++d) e = fma(S[d], H[d] - Q.cst[3 * (3 * a + d)], e);
+                sums2(0, j, S);
             }
 #pragma unroll 1
             for (int j = 0; j < m3; ++j) {
                 const int p = p0 + j * kWave, a = atom(j);
                 const double* c3 = Q.cst + 3 * (3 * A2 + 8 * a);
-                double S[8], H[1][8];
+                double S[8], H[8];
                 F.tm(p, S);
 #pragma unroll
-                for (int d = 0; d < 8; ++d) H[0][d] = -c3[3 * d];
-                F.template tm_bonds<1, TT>(a, p, H);
+                for (int d = 0; d < 8; ++d) H[d] = -c3[3 * d];
+                F.template tm_bonds<TT>(a, p, H);
                 if (M0->has_onsite3) {
                     const cptr<double> A3m = as_const(M0->onsite3) + a * 64;
 #pragma unroll
                     for (int d = 0; d < 8; ++d)
 #pragma unroll
-                        for (int c = 0; c < 8; ++c) H[0][d] = fma(A3m[d * 8 + c], S[c], H[0][d]);
+                        for (int c = 0; c < 8; ++c) H[d] = fma(A3m[d * 8 + c], S[c], H[d]);
                 }
 #pragma unroll
-                for (int d = 0; d < 8; ++d) e = fma(S[d], H[0][d] - c3[3 * d], e);
+                for (int d = 0; d < 8; ++d) e = fma(S[d], H[d] - c3[3 * d], e);
                 sums3(0, j, S);
             }
             sum_e(0, e);

@@ -12,7 +12,8 @@
 // one phase on all four SIMDs instead of two phases of four waves each.
 //
 // What bounds it: the chain of one wave's stage (about 290 FP64 instructions
-// of an SU(3) site with eight Fe-Tm bonds) with two to four waves per SIMD.
+// of an SU(3) site with eight Fe-Tm bonds) with two to four waves per SIMD:
+// 2.2 us a stage of that cell, 13.5 on the other kernel before.
 // The constant part of the fields, the pulse envelopes and the records are
 // handled as in csl_trajectory.hip, kChunk steps at a time.
 #include <algorithm>
