@@ -94,6 +94,8 @@ struct csl_lattice {
     DBuf<double> X, ACC, Y1, Y2, partials, fac, tgrid, rec_mags, rec_energy, rec_states, aux;
     DBuf<double> KS;              // stage derivatives of the generic fixed-step engine [S][3][NP]
     DBuf<double> bt_init, bt_tp, bt_amp, bt_final;
+    DBuf<double> pp_recs;         // pump-probe records, trajectory by trajectory
+    DBuf<int> pp_keep;
     DBuf<double> dp_times;        // Dormand-Prince records: times [B][max_rec]
     // persistent-kernel work split (batches larger than the co-resident workgroups)
     DBuf<int> ps_sched;
@@ -2072,10 +2074,9 @@ int csl_pump_probe_ex(csl_lattice* h, const double* ground, const double* field_
             auto g = make_grid(T0, T1, T_step, CSL_TGRID_BOOST);
             const size_t n_rec = records_for(g.size() - 1, 1);
             tt.resize(n_rec);
-            mg.resize(n_rec * B * 9);
             size_t nr = 0;
             rc2 = csl_integrate_batched(h, B, ground, 0, tp.data(), am.data(), T0, T1, T_step, 1, "rk4",
-                                        CSL_TGRID_BOOST, 0, n_rec, tt.data(), mg.data(), nullptr, nullptr, &nr);
+                                        CSL_TGRID_BOOST, 0, n_rec, tt.data(), nullptr, nullptr, nullptr, &nr);
             if (rc2 == CSL_OK) keep = gate(tt.data(), nr);
         }
         // reset the pulse as the reference drivers do (lattice_md.cpp:578-583)
@@ -2084,16 +2085,49 @@ int csl_pump_probe_ex(csl_lattice* h, const double* ground, const double* field_
         const size_t nk = keep.size();
         if (n_rec_out) *n_rec_out = nk;
         if (nk > max_rec) fail(CSL_ERR_CAPACITY, "max_rec is smaller than the number of records");
-        for (size_t j = 0; j < nk; ++j) {
-            const size_t r = keep[j];
-            if (times) times[j] = tt[r];
-            if (M0) std::memcpy(M0 + j * 9, &mg[(r * B + 0) * 9], 9 * sizeof(double));
-            for (size_t i = 0; i < n_tau; ++i) {
-                if (M1 && !w1)
-                    std::memcpy(M1 + (i * max_rec + j) * 9, &mg[(r * B + 1 + i) * 9], 9 * sizeof(double));
-                if (M01)
-                    std::memcpy(M01 + (i * max_rec + j) * 9, &mg[(r * B + 1 + n1 + i) * 9], 9 * sizeof(double));
+        for (size_t j = 0; j < nk; ++j)
+            if (times) times[j] = tt[keep[j]];
+        std::vector<double> m0(w1 ? nk * 9 : 0);  // M0's gated records (synthesis of M1)
+        if (dp5) {
+            for (size_t j = 0; j < nk; ++j) {
+                const size_t r = keep[j];
+                if (M0) std::memcpy(M0 + j * 9, &mg[(r * B + 0) * 9], 9 * sizeof(double));
+                if (w1) std::memcpy(&m0[j * 9], &mg[(r * B + 0) * 9], 9 * sizeof(double));
+                for (size_t i = 0; i < n_tau; ++i) {
+                    if (M1 && !w1)
+                        std::memcpy(M1 + (i * max_rec + j) * 9, &mg[(r * B + 1 + i) * 9], 9 * sizeof(double));
+                    if (M01)
+                        std::memcpy(M01 + (i * max_rec + j) * 9, &mg[(r * B + 1 + n1 + i) * 9], 9 * sizeof(double));
+                }
             }
+        } else if (nk > 0) {
+            // gated and put trajectory by trajectory on the device, then
+            // copied straight into the outputs
+            hipStream_t s = h->stream;
+            const bool run = keep.back() - keep.front() + 1 == nk;
+            if (!run) {
+                const std::vector<int> ki(keep.begin(), keep.end());
+                h->pp_keep.upload(ki.data(), ki.size(), s);
+                hip_check(hipStreamSynchronize(s), "upload");
+            }
+            h->pp_recs.ensure(B * nk * 9);
+            hip_check(csl::launch_gather_records(h->rec_mags.p, int(B), int(nk), int(keep.front()),
+                                                 run ? nullptr : h->pp_keep.p, h->pp_recs.p, s),
+                      "k_gather_records");
+            auto rows = [&](double* host, size_t b0, size_t n) {
+                const double* dev = h->pp_recs.p + b0 * nk * 9;
+                if (!host || !n) return;
+                if (max_rec == nk || n == 1) {
+                    copy_back(host, dev, n * nk * 9, s);
+                } else {
+                    for (size_t i = 0; i < n; ++i) copy_back(host + i * max_rec * 9, dev + i * nk * 9, nk * 9, s);
+                }
+            };
+            rows(M0, 0, 1);
+            if (w1) rows(m0.data(), 0, 1);
+            else rows(M1, 1, n_tau);
+            rows(M01, 1 + n1, n_tau);
+            hip_check(hipStreamSynchronize(s), "pump-probe records");
         }
         if (w1 && M1 && nk > 0) {
             // synthesize_M1_from_M0 (lattice_md.cpp:283-317): M1(t_i) = M_ground
@@ -2125,7 +2159,7 @@ int csl_pump_probe_ex(csl_lattice* h, const double* ground, const double* field_
                         long long idx = std::llround((ti - taus[i] - t_first) / T_step);
                         if (idx < 0) idx = 0;
                         if (idx >= (long long)nk) idx = (long long)nk - 1;
-                        src = &mg[(keep[size_t(idx)] * B + 0) * 9];
+                        src = &m0[size_t(idx) * 9];
                     }
                     std::memcpy(M1 + (i * max_rec + j) * 9, src, 9 * sizeof(double));
                 }

@@ -358,6 +358,10 @@ hipError_t launch_persistent(const LatDev& L, const PersistArgs& A, int block, i
                              hipStream_t st);
 int stage_blocks(const LatDev& L);
 hipError_t launch_stage(const LatDev& L, const StageArgs& A, hipStream_t st);
+// out[b][j] = record keep[j] (r0 + j when keep is null) of trajectory b, 9
+// doubles each, from mags [..][B][9].
+hipError_t launch_gather_records(const double* mags, int B, int nk, int r0, const int* keep, double* out,
+                                 hipStream_t st);
 hipError_t launch_observe(const LatDev& L, const double* y, double* partials, int B,
                           hipStream_t st);
 hipError_t launch_reduce_obs(const double* partials, int nblk, int B, int ri, double inv_n,

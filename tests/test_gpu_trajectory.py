@@ -65,3 +65,32 @@ def test_trajectory_edges(oracle, name, steps, every, alpha):
         assert np.max(np.abs(r["mags"][:, b] - ref["mags"][keep])) <= TOL
         assert np.max(np.abs(r["energy"][:, b] - ref["energy"][keep])) <= TOL
         assert np.max(np.abs(r["final"][b] - ref["final"].reshape(-1, 3))) <= TOL
+
+
+@pytest.mark.parametrize("n_tau,steps", [(1, 1), (7, 15), (8, 16), (17, 33)])
+def test_pump_probe_rows(n_tau, steps):
+    """Trajectory-major pump-probe records (tiles of 16 records x 16
+    trajectories) are the batch's own records, the start sample dropped."""
+    lat = model.Lattice(_kitaev(), 5, 4, 1)
+    s = random_state(lat, 3)
+    f = np.zeros((2, 3))
+    f[:, 0] = 1.0
+    T1 = -0.1 + (steps + 0.5) * DT
+    print(f"[pump] n_tau {n_tau} steps {steps}", flush=True)
+    with GPULattice(lat) as gl:
+        r = gl.pump_probe(s, f, 0.5, 0.1, 0.0, 0.0, 0.02 * (n_tau - 0.5), 0.02, -0.1, T1, DT)
+        fd = np.einsum("aij,aj->ai", lat.frames, f).reshape(-1)
+        gl.set_pulse(np.concatenate([fd, fd]), 0.5, 0.1, 0.0, 0.0, 0.0)
+        taus = 0.02 * np.arange(n_tau)
+        B = 1 + 2 * n_tau
+        tp, am = np.zeros((B, 2)), np.zeros((B, 2))
+        am[0, 0] = 0.5
+        tp[1:1 + n_tau, 0], am[1:1 + n_tau, 0] = taus, 0.5
+        tp[1 + n_tau:, 1], am[1 + n_tau:] = taus, 0.5
+        b = gl.integrate_batched(s, tp, am, -0.1, T1, DT, tgrid="boost")
+    m = b["mags"][1:]
+    assert r["M0"].shape == (steps, 3, 3) and r["M1"].shape == r["M01"].shape == (n_tau, steps, 3, 3)
+    assert np.array_equal(r["times"], b["times"][1:])
+    assert np.array_equal(r["M0"], m[:, 0])
+    assert np.array_equal(r["M1"], np.swapaxes(m[:, 1:1 + n_tau], 0, 1))
+    assert np.array_equal(r["M01"], np.swapaxes(m[:, 1 + n_tau:], 0, 1))
