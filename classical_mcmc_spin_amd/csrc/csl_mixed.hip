@@ -26,7 +26,7 @@
 #include "csl_host.hpp"
 #include "csl_internal.hpp"
 #include "csl_kernels.hpp"
-#include "csl_mixed_device.hpp"
+#include "csl_mixed_lds.hpp"
 #include "csl_tableau.hpp"
 
 namespace csl {
@@ -94,6 +94,73 @@ __device__ __forceinline__ void gather_bonds(const Ell& E, const double* __restr
             for (int a = 0; a < DA; ++a)
 #pragma unroll
                 for (int e = 0; e < DB; ++e) H[a] = fma(J[a * DB + e], s[e], H[a]);
+        }
+    }
+}
+
+// The bond terms of a field and of its tangent in one pass over a site's
+// bonds: H += J s_p, dH += J ds_p, and with THETA (the kinds the scale theta
+// multiplies) dH += J s_p as well.
+template <int DA, int DB, bool THETA>
+__device__ __forceinline__ void gather_bonds_tl(const Ell& E, const double* __restrict__ src,
+                                                const double* __restrict__ zsrc, int NPsrc, int NPpart, int atom, int p,
+                                                double* H, double* dH) {
+    const int c = E.uniform ? E.cnt_atom[atom] : E.cnt[p];
+    for (int k = 0; k < c; ++k) {
+        const int q = E.col[size_t(k) * NPsrc + p];
+        double s[DB], ds[DB];
+#pragma unroll
+        for (int e = 0; e < DB; ++e) {
+            s[e] = src[size_t(e) * NPpart + q];
+            ds[e] = zsrc[size_t(e) * NPpart + q] + (THETA ? s[e] : 0.0);
+        }
+        auto add = [&](auto J) {
+#pragma unroll
+            for (int a = 0; a < DA; ++a)
+#pragma unroll
+                for (int e = 0; e < DB; ++e) {
+                    H[a] = fma(J[a * DB + e], s[e], H[a]);
+                    dH[a] = fma(J[a * DB + e], ds[e], dH[a]);
+                }
+        };
+        if (E.uniform) add(as_const(E.mats) + (size_t(atom) * E.zmax + k) * (DA * DB));
+        else add(E.mats + (size_t(k) * NPsrc + p) * (DA * DB));
+    }
+}
+
+// The same over Z padded bonds whose partners are known (MixDev::q22 ..
+// jpad): no dependent partner loads and no bond count, so the gathers of all
+// bonds are in flight together.  J(k) is the k-th 3 x DX matrix; TR: its
+// transpose is applied (SU(3) sites).
+template <int DA, int DB, int Z, bool THETA, bool TR, class JF>
+__device__ __forceinline__ void gather_padded_tl(JF J, const int* q, const double* __restrict__ src,
+                                                 const double* __restrict__ zsrc, int NPpart, double (&H)[DA], double (&dH)[DA]) {
+    constexpr int G = DB == 8 ? 4 : Z;   // bonds in flight together
+#pragma unroll
+    for (int k0 = 0; k0 < Z; k0 += G) {
+        double s[G][DB], ds[G][DB];
+#pragma unroll
+        for (int k = 0; k < G; ++k)
+#pragma unroll
+            for (int e = 0; e < DB; ++e) {
+                s[k][e] = src[size_t(e) * NPpart + q[k0 + k]];
+                ds[k][e] = zsrc[size_t(e) * NPpart + q[k0 + k]];
+            }
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+            const cptr<double> Jk = J(k0 + k) + opaque_zero();
+#pragma unroll
+            for (int e = 0; e < DB; ++e) {
+                const double dv = ds[k][e] + (THETA ? s[k][e] : 0.0);
+#pragma unroll
+                for (int a = 0; a < DA; ++a) {
+                    const double j = TR ? Jk[e * DA + a] : Jk[a * DB + e];
+                    H[a] = fma(j, s[k][e], H[a]);
+                    dH[a] = fma(j, dv, dH[a]);
+                }
+            }
+            end_bond(H);
+            end_bond(dH);
         }
     }
 }
@@ -220,9 +287,12 @@ __device__ __forceinline__ void rk_update(int s, size_t q, double Sd, double kd,
 // with COH the values other workgroups read (next stage values, the state
 // written in stage 3, record partials) are stored and gathered at agent
 // scope, for the cooperative kernel that runs all stages in one launch.
-template <bool TL, bool COH>
+// Z22, ZM: padded bonds per site of the kinds 22 and 23 / 32 (tangent runs of
+// lattices with MixDev::jpad), 0: the tables' own counts.
+constexpr int kRawRec = 40;   // raw sums of a wave: own at 0, energy at 16, tangent at 20
+template <bool TL, bool COH, int Z22 = 0, int ZM = 0>
 __device__ __forceinline__ void mixed_stage_wg(const MixDev& M, const MixStageArgs& A, int bx, int b, double* fac,
-                                               double (*red)[kRec]) {
+                                               double (*red)[kRawRec]) {
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = uniform(tid >> 6);
@@ -250,9 +320,11 @@ __device__ __forceinline__ void mixed_stage_wg(const MixDev& M, const MixStageAr
     const double dt = A.dt;
     const double cdt = (s == 2) ? 1.0 * dt : 0.5 * dt;
     const double bdt = (s == 0 || s == 3) ? (1.0 / 6.0) * dt : (1.0 / 3.0) * dt;
-    double part[kRec], tpart[kRec];
+    // values of this thread's site whose sums make the record: the
+    // components, the tangent's, twice the energy share, the staggered sign
+    double own[8], town[8], e2 = 0.0, sgn = 1.0;
 #pragma unroll
-    for (int j = 0; j < kRec; ++j) part[j] = tpart[j] = 0.0;
+    for (int j = 0; j < 8; ++j) own[j] = town[j] = 0.0;
     const double* zc = TL ? A.zcur + off : nullptr;
     if (!is3) {
         const int p = bx * 256 + tid;
@@ -261,22 +333,37 @@ __device__ __forceinline__ void mixed_stage_wg(const MixDev& M, const MixStageAr
         if (p < M.NP2 && (p - atom * M.npad) < M.n_cells) {
             const int NP = M.NP2;
             const double S[3] = {cur[p], cur[NP + p], cur[2 * NP + p]};
-            double H[3];
-            field_su2<COH>(M, cur, atom, p, S, H);
+            double H[3], dS[3] = {0.0, 0.0, 0.0}, dH[3] = {0.0, 0.0, 0.0};
+            if constexpr (TL) {
+                const size_t o3 = size_t(3) * M.NP2;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) dS[d] = zc[size_t(d) * NP + p];
+                field_onsite<3>(M.field2, M.onsite2, M.site_uniform2, M.has_onsite2, atom, p, S, H);
+                onsite_lin<3>(M.onsite2, M.site_uniform2, M.has_onsite2, atom, p, dS, dH);
+                if constexpr (Z22 > 0) {
+                    int q22[8], q23[8];
+                    unpack8(M.q22[p], q22);
+                    unpack8(M.q23[p], q23);
+                    const cptr<double> jp = as_const(M.jpad);
+                    gather_padded_tl<3, 3, Z22, false, false>(
+                        [&](int k) { return jp + M.j22off + (atom * Z22 + k) * 9; }, q22, cur, zc, M.NP2, H, dH);
+                    gather_padded_tl<3, 8, ZM, true, false>([&](int k) { return jp + (atom * ZM + k) * 24; }, q23,
+                                                            cur + o3, zc + o3, M.NP3, H, dH);
+                } else {
+                    gather_bonds_tl<3, 3, false>(M.e22, cur, zc, M.NP2, M.NP2, atom, p, H, dH);
+                    gather_bonds_tl<3, 8, true>(M.e23, cur + o3, zc + o3, M.NP2, M.NP3, atom, p, H, dH);
+                }
+            } else {
+                field_su2<COH>(M, cur, atom, p, S, H);
+            }
             if (A.rec) {
-                const cptr<double> R = as_const(M.frames2) + size_t(atom) * 9;
-                const double sg = M.afm2[atom];
-                const double B0 = M.site_uniform2 ? M.field2[atom * 3 + 0] : M.field2[size_t(p) * 3 + 0];
-                const double B1 = M.site_uniform2 ? M.field2[atom * 3 + 1] : M.field2[size_t(p) * 3 + 1];
-                const double B2 = M.site_uniform2 ? M.field2[atom * 3 + 2] : M.field2[size_t(p) * 3 + 2];
 #pragma unroll
                 for (int mu = 0; mu < 3; ++mu) {
-                    const double g = R[mu * 3] * S[0] + R[mu * 3 + 1] * S[1] + R[mu * 3 + 2] * S[2];
-                    part[mu] = sg * g;
-                    part[3 + mu] = S[mu];
-                    part[6 + mu] = g;
+                    const double Bm = M.site_uniform2 ? M.field2[atom * 3 + mu] : M.field2[size_t(p) * 3 + mu];
+                    own[mu] = S[mu];
+                    town[mu] = dS[mu];
+                    e2 += S[mu] * (H[mu] - Bm);
                 }
-                part[33] = 0.5 * (S[0] * (H[0] - B0) + S[1] * (H[1] - B1) + S[2] * (H[2] - B2));
             }
             if (A.tp) {
                 const double f1 = fac[0], f2 = fac[1];
@@ -284,24 +371,12 @@ __device__ __forceinline__ void mixed_stage_wg(const MixDev& M, const MixStageAr
                     const cptr<double> d0 = as_const(M.fdrive2) + size_t(atom) * 3;
                     const cptr<double> d1 = as_const(M.fdrive2) + size_t(M.A2 + atom) * 3;
 #pragma unroll
-                    for (int a = 0; a < 3; ++a) H[a] -= d0[a] * f1 + d1[a] * f2;
+                    for (int a = 0; a < 3; ++a) H[a] -= fma(d0[a], f1, d1[a] * f2);
                 }
             }
-            double k[3] = {H[1] * S[2] - H[2] * S[1], H[2] * S[0] - H[0] * S[2], H[0] * S[1] - H[1] * S[0]};
-            if (M.alpha != 0.0) {  // mixed_lattice_md.cpp:570-578
-                const double S2 = S[0] * S[0] + S[1] * S[1] + S[2] * S[2];
-                const double SH = S[0] * H[0] + S[1] * H[1] + S[2] * H[2];
-                const double g = (S2 > 0.0) ? M.alpha / sqrt(S2) : 0.0;
-#pragma unroll
-                for (int a = 0; a < 3; ++a) k[a] += g * (S[a] * SH - H[a] * S2);
-            }
+            double k[3];
+            ll_mixed_su2(H, S, M.alpha, k);
             if (TL) {
-                const double dS[3] = {zc[p], zc[NP + p], zc[2 * NP + p]};
-                double dH[3] = {0.0, 0.0, 0.0};
-                onsite_lin<3>(M.onsite2, M.site_uniform2, M.has_onsite2, atom, p, dS, dH);
-                gather_bonds<3, 3>(M.e22, zc, M.NP2, M.NP2, atom, p, dH);
-                gather_bonds<3, 8>(M.e23, zc + size_t(3) * M.NP2, M.NP2, M.NP3, atom, p, dH);
-                gather_bonds<3, 8>(M.e23, cur + size_t(3) * M.NP2, M.NP2, M.NP3, atom, p, dH);  // d H / d theta
                 double dk[3] = {dH[1] * S[2] - dH[2] * S[1] + (H[1] * dS[2] - H[2] * dS[1]),
                                 dH[2] * S[0] - dH[0] * S[2] + (H[2] * dS[0] - H[0] * dS[2]),
                                 dH[0] * S[1] - dH[1] * S[0] + (H[0] * dS[1] - H[1] * dS[0])};
@@ -324,17 +399,6 @@ __device__ __forceinline__ void mixed_stage_wg(const MixDev& M, const MixStageAr
                 for (int d = 0; d < 3; ++d)
                     rk_update(s, size_t(d) * NP + p, dS[d], dk[d], bdt, cdt, A.zx + off, A.zacc + off,
                               A.znext + off);
-                if (A.rec) {
-                    const cptr<double> R = as_const(M.frames2) + size_t(atom) * 9;
-                    const double sg = M.afm2[atom];
-#pragma unroll
-                    for (int mu = 0; mu < 3; ++mu) {
-                        const double g = R[mu * 3] * dS[0] + R[mu * 3 + 1] * dS[1] + R[mu * 3 + 2] * dS[2];
-                        tpart[mu] = sg * g;
-                        tpart[3 + mu] = dS[mu];
-                        tpart[6 + mu] = g;
-                    }
-                }
             }
             if (s == 0) {
 #pragma unroll
@@ -370,24 +434,37 @@ __device__ __forceinline__ void mixed_stage_wg(const MixDev& M, const MixStageAr
             double S[8];
 #pragma unroll
             for (int a = 0; a < 8; ++a) S[a] = cur[o3 + size_t(a) * NP + p];
-            double H[8];
-            field_su3<COH>(M, cur, atom, p, S, H);
+            double H[8], dl[8], dH[8];
+#pragma unroll
+            for (int a = 0; a < 8; ++a) dl[a] = dH[a] = 0.0;
+            if constexpr (TL) {
+#pragma unroll
+                for (int a = 0; a < 8; ++a) dl[a] = zc[o3 + size_t(a) * NP + p];
+                field_onsite<8>(M.field3, M.onsite3, M.site_uniform3, M.has_onsite3, atom, p, S, H);
+                onsite_lin<8>(M.onsite3, M.site_uniform3, M.has_onsite3, atom, p, dl, dH);
+                gather_bonds_tl<8, 8, false>(M.e33, cur + o3, zc + o3, M.NP3, M.NP3, atom, p, H, dH);
+                if constexpr (Z22 > 0) {
+                    int q32[8];
+                    unpack8(M.q32[p], q32);
+                    const cptr<double> jp = as_const(M.jpad);
+                    const cptr<int> jo = as_const(M.j32pad) + atom * ZM;
+                    gather_padded_tl<8, 3, ZM, true, true>([&](int k) { return jp + uniform(jo[k]); }, q32, cur, zc, M.NP2,
+                                                           H, dH);
+                } else {
+                    gather_bonds_tl<8, 3, true>(M.e32, cur, zc, M.NP3, M.NP2, atom, p, H, dH);
+                }
+            } else {
+                field_su3<COH>(M, cur, atom, p, S, H);
+            }
             if (A.rec) {
-                const cptr<double> R = as_const(M.frames3) + size_t(atom) * 64;
-                const double sg = ((cell * M.A3 + atom) & 1) ? -1.0 : 1.0;
-                double e = 0.0;
+                sgn = ((cell * M.A3 + atom) & 1) ? -1.0 : 1.0;
 #pragma unroll
                 for (int mu = 0; mu < 8; ++mu) {
-                    double g = 0.0;
-#pragma unroll
-                    for (int nu = 0; nu < 8; ++nu) g += R[mu * 8 + nu] * S[nu];
-                    part[9 + mu] = sg * S[mu];
-                    part[17 + mu] = S[mu];
-                    part[25 + mu] = g;
                     const double Bm = M.site_uniform3 ? M.field3[atom * 8 + mu] : M.field3[size_t(p) * 8 + mu];
-                    e += S[mu] * (H[mu] - Bm);
+                    own[mu] = S[mu];
+                    town[mu] = dl[mu];
+                    e2 += S[mu] * (H[mu] - Bm);
                 }
-                part[33] = 0.5 * e;
             }
             if (A.tp) {
                 const double f1 = fac[2], f2 = fac[3];
@@ -395,7 +472,7 @@ __device__ __forceinline__ void mixed_stage_wg(const MixDev& M, const MixStageAr
                     const cptr<double> d0 = as_const(M.fdrive3) + size_t(atom) * 8;
                     const cptr<double> d1 = as_const(M.fdrive3) + size_t(M.A3 + atom) * 8;
 #pragma unroll
-                    for (int a = 0; a < 8; ++a) H[a] -= d0[a] * f1 + d1[a] * f2;
+                    for (int a = 0; a < 8; ++a) H[a] -= fma(d0[a], f1, d1[a] * f2);
                 }
             }
             double k[8];
@@ -403,19 +480,9 @@ __device__ __forceinline__ void mixed_stage_wg(const MixDev& M, const MixStageAr
             if (M.has_bloch) {  // mixed_lattice_md.cpp:596-605
 #pragma unroll
                 for (int a = 0; a < 8; ++a)
-                    if (M.gamma[a] != 0.0) k[a] -= M.gamma[a] * (S[a] - M.eq3[size_t(a) * NP + p]);
+                    if (M.gamma[a] != 0.0) k[a] = fma(-M.gamma[a], S[a] - M.eq3[size_t(a) * NP + p], k[a]);
             }
             if (TL) {
-                double dl[8];
-#pragma unroll
-                for (int a = 0; a < 8; ++a) dl[a] = zc[o3 + size_t(a) * NP + p];
-                double dH[8];
-#pragma unroll
-                for (int a = 0; a < 8; ++a) dH[a] = 0.0;
-                onsite_lin<8>(M.onsite3, M.site_uniform3, M.has_onsite3, atom, p, dl, dH);
-                gather_bonds<8, 8>(M.e33, zc + o3, M.NP3, M.NP3, atom, p, dH);
-                gather_bonds<8, 3>(M.e32, zc, M.NP3, M.NP2, atom, p, dH);
-                gather_bonds<8, 3>(M.e32, cur, M.NP3, M.NP2, atom, p, dH);  // d H / d theta
                 double dk[8], t2[8];
                 su3_cross(dH, S, dk);
                 su3_cross(H, dl, t2);
@@ -429,19 +496,6 @@ __device__ __forceinline__ void mixed_stage_wg(const MixDev& M, const MixStageAr
                 for (int d = 0; d < 8; ++d)
                     rk_update(s, o3 + size_t(d) * NP + p, dl[d], dk[d], bdt, cdt, A.zx + off, A.zacc + off,
                               A.znext + off);
-                if (A.rec) {
-                    const cptr<double> R = as_const(M.frames3) + size_t(atom) * 64;
-                    const double sg = ((cell * M.A3 + atom) & 1) ? -1.0 : 1.0;
-#pragma unroll
-                    for (int mu = 0; mu < 8; ++mu) {
-                        double g = 0.0;
-#pragma unroll
-                        for (int nu = 0; nu < 8; ++nu) g += R[mu * 8 + nu] * dl[nu];
-                        tpart[9 + mu] = sg * dl[mu];
-                        tpart[17 + mu] = dl[mu];
-                        tpart[25 + mu] = g;
-                    }
-                }
             }
             if (s == 0) {
 #pragma unroll
@@ -468,48 +522,73 @@ __device__ __forceinline__ void mixed_stage_wg(const MixDev& M, const MixStageAr
         }
     }
     if (A.rec) {
-        // SU(2) workgroups own record entries 0..8 and 33, SU(3) ones 9..33
-        const int j0 = is3 ? 9 : 0, j1 = is3 ? 33 : 9;
-#pragma unroll
-        for (int j = 0; j < kRec; ++j) {
-            if ((j >= j0 && j < j1) || j == 33) {
-                const double v = wave_sum(part[j]);
-                if (lane == 0) red[wave][j] = v;
+        // Wave sums of the components (21 instructions per four, against 72
+        // each for sums of the 34 record entries); a wave's sites are of one
+        // sublattice, so its frame and sign act on the sums.  SU(2)
+        // workgroups own record entries 0..8 and 33, SU(3) ones 9..33.
+        double* r = red[wave];
+        wave_sum4(own[0], own[1], own[2], own[3], lane, r);
+        wave_sum4(e2, 0.0, 0.0, 0.0, lane, r + 16);
+        if (TL) wave_sum4(town[0], town[1], town[2], town[3], lane, r + 20);
+        if (is3) {
+            wave_sum4(own[4], own[5], own[6], own[7], lane, r + 4);
+            wave_sum4(sgn * own[0], sgn * own[1], sgn * own[2], sgn * own[3], lane, r + 8);
+            wave_sum4(sgn * own[4], sgn * own[5], sgn * own[6], sgn * own[7], lane, r + 12);
+            if (TL) {
+                wave_sum4(town[4], town[5], town[6], town[7], lane, r + 24);
+                wave_sum4(sgn * town[0], sgn * town[1], sgn * town[2], sgn * town[3], lane, r + 28);
+                wave_sum4(sgn * town[4], sgn * town[5], sgn * town[6], sgn * town[7], lane, r + 32);
             }
         }
         __syncthreads();
-        if (tid < kRec) {
-            const bool mine = (tid >= j0 && tid < j1) || tid == 33;
-            const double v = mine ? (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]) : 0.0;
-            st_x<COH>(A.partials + (size_t(b) * gridDim.x + bx) * kRec + tid, v);
-        }
-        if (TL) {
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < kRec; ++j) {
-                if (j >= j0 && j < j1) {
-                    const double v = wave_sum(tpart[j]);
-                    if (lane == 0) red[wave][j] = v;
+        const int NPs = is3 ? M.NP3 : M.NP2, pw0 = (is3 ? bx - A.nblk2 : bx) * 256;
+        auto entry = [&](int j, const double* raw) {   // record entry j of the four waves' sums at raw
+            double v = 0.0;
+            for (int w = 0; w < 4; ++w) {
+                const int pw = pw0 + w * kWave;
+                if (pw >= NPs) break;
+                const int a = pw / M.npad;
+                const double* q = raw + w * kRawRec;
+                if (!is3 && j < 9) {
+                    const int d = j % 3;
+                    const double* R = M.frames2 + size_t(a) * 9 + d * 3;
+                    const double g = R[0] * q[0] + R[1] * q[1] + R[2] * q[2];
+                    v += j < 3 ? M.afm2[a] * g : (j < 6 ? q[d] : g);
+                } else if (is3 && j >= 9 && j < 33) {
+                    const int d = (j - 9) & 7;
+                    if (j < 17) {
+                        v += q[8 + d];
+                    } else if (j < 25) {
+                        v += q[d];
+                    } else {
+                        const double* R = M.frames3 + size_t(a) * 64 + d * 8;
+                        double g = 0.0;
+                        for (int c = 0; c < 8; ++c) g += R[c] * q[c];
+                        v += g;
+                    }
                 }
             }
-            __syncthreads();
-            if (tid < kRec) {
-                const bool mine = tid >= j0 && tid < j1;
-                const double v = mine ? (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]) : 0.0;
-                A.tpartials[(size_t(b) * gridDim.x + bx) * kRec + tid] = v;
-            }
+            return v;
+        };
+        if (tid < kRec) {
+            double v = entry(tid, &red[0][0]);
+            if (tid == 33) v = 0.5 * ((red[0][16] + red[1][16]) + (red[2][16] + red[3][16]));
+            st_x<COH>(A.partials + (size_t(b) * gridDim.x + bx) * kRec + tid, v);
+        }
+        if (TL && tid >= kWave && tid < kWave + kRec) {
+            const int j = tid - kWave;
+            A.tpartials[(size_t(b) * gridDim.x + bx) * kRec + j] = entry(j, &red[0][20]);
         }
     }
 }
 
-
-template <bool TL>
+template <bool TL, int Z22 = 0, int ZM = 0>
 __global__ void __launch_bounds__(256) k_mixed_stage(MixDev M, MixStageArgs A) {
     __shared__ double fac[4];
-    __shared__ double red[4][kRec];
+    __shared__ double red[4][kRawRec];
     int bx, b;
     mix_block(bx, b);
-    mixed_stage_wg<TL, false>(M, A, bx, b, fac, red);
+    mixed_stage_wg<TL, false, Z22, ZM>(M, A, bx, b, fac, red);
 }
 
 // Cooperative form of the stage kernels for a small batch of a large
@@ -537,7 +616,7 @@ constexpr int kCoopSpin = 1 << 22;
 
 __global__ void __launch_bounds__(256) k_mixed_coop(MixDev M, MixCoopArgs C) {
     __shared__ double fac[4];
-    __shared__ double red[4][kRec];
+    __shared__ double red[4][kRawRec];
     __shared__ int ok;
     int bx, b;
     mix_block(bx, b);
@@ -647,31 +726,29 @@ __global__ void __launch_bounds__(256) k_mixed_loss_grad(const double* __restric
     }
 }
 
-// One workgroup per trajectory: partials -> record ri
-__global__ void __launch_bounds__(256) k_mixed_reduce(const double* __restrict__ partials, int nblk, int B,
-                                                      int ri, double inv2, double inv3, double invE,
-                                                      double* __restrict__ recs, int rec_stride) {
-    __shared__ double red[kRec][4];
-    const int b = blockIdx.x;
-    const int t = threadIdx.x;
-    double v[kRec];
-#pragma unroll
-    for (int j = 0; j < kRec; ++j) v[j] = 0.0;
-    for (int k = t; k < nblk; k += 256) {
-        const double* q = partials + (size_t(b) * nblk + k) * kRec;
-#pragma unroll
-        for (int j = 0; j < kRec; ++j) v[j] += q[j];
+// One workgroup per trajectory: partials -> record ri; blockIdx.y = 1 the
+// tangent's.  Seven groups of 34 threads, a thread per record entry, take
+// the workgroups' partials in turn (no wave sums of mostly empty lanes).
+__global__ void __launch_bounds__(256) k_mixed_reduce(const double* __restrict__ partials,
+                                                      const double* __restrict__ tpartials, int nblk, int B, int ri,
+                                                      double inv2, double inv3, double invE, double* __restrict__ recs,
+                                                      double* __restrict__ trecs, int rec_stride) {
+    constexpr int G = 256 / kRec;
+    __shared__ double red[G][kRec];
+    const bool tan = blockIdx.y == 1;
+    const double* part = tan ? tpartials : partials;
+    const int b = blockIdx.x, g = int(threadIdx.x) / kRec, j = int(threadIdx.x) % kRec;
+    if (g < G) {
+        double v = 0.0;
+        for (int k = g; k < nblk; k += G) v += part[(size_t(b) * nblk + k) * kRec + j];
+        red[g][j] = v;
     }
-#pragma unroll
-    for (int j = 0; j < kRec; ++j) v[j] = wave_sum(v[j]);
-    if ((t & (kWave - 1)) == 0)
-#pragma unroll
-        for (int j = 0; j < kRec; ++j) red[j][t >> 6] = v[j];
     __syncthreads();
-    if (t < kRec) {
-        const double tot = (red[t][0] + red[t][1]) + (red[t][2] + red[t][3]);
-        const double sc = t < 9 ? inv2 : (t < 33 ? inv3 : invE);
-        recs[(size_t(ri) * rec_stride + b) * kRec + t] = tot * sc;
+    if (g == 0) {
+        double tot = 0.0;
+        for (int i = 0; i < G; ++i) tot += red[i][j];
+        const double sc = j < 9 ? inv2 : (j < 33 ? inv3 : invE);
+        (tan ? trecs : recs)[(size_t(ri) * (tan ? B : rec_stride) + b) * kRec + j] = tot * sc;
     }
 }
 
@@ -1619,6 +1696,13 @@ void run_mixed(csl_mixed* h, size_t B, const double* d_tp, const double* d_tp3, 
     hip_check(hipEventCreate(&e1), "event");
     size_t launches = 0;
     const dim3 grid_dim{unsigned(nblk), unsigned(B), 1u};
+    // tangent runs: the padded tables where the lattice has them
+    const int padded = h->M.jpad ? h->M.jz22 * 10 + h->M.jzm : 0;
+    auto* const tl_kernel = padded == 64   ? csl::k_mixed_stage<true, 6, 4>
+                            : padded == 68 ? csl::k_mixed_stage<true, 6, 8>
+                            : padded == 84 ? csl::k_mixed_stage<true, 8, 4>
+                            : padded == 88 ? csl::k_mixed_stage<true, 8, 8>
+                                           : csl::k_mixed_stage<true>;
     auto stage = [&](int st, double t, int rec) {
         csl::MixStageArgs A{};
         A.stage = st;
@@ -1640,7 +1724,7 @@ void run_mixed(csl_mixed* h, size_t B, const double* d_tp, const double* d_tp3, 
             A.zcur = st == 0 ? h->ZX.p : (st == 2 ? h->ZY2.p : h->ZY1.p);
             A.znext = st == 0 ? h->ZY1.p : (st == 1 ? h->ZY2.p : (st == 2 ? h->ZY1.p : h->ZY2.p));
             A.tpartials = h->tpartials.p;
-            hipLaunchKernelGGL(csl::k_mixed_stage<true>, grid_dim, dim3(256), 0, s, h->M, A);
+            hipLaunchKernelGGL(tl_kernel, grid_dim, dim3(256), 0, s, h->M, A);
         } else {
             hipLaunchKernelGGL(csl::k_mixed_stage<false>, grid_dim, dim3(256), 0, s, h->M, A);
         }
@@ -1648,14 +1732,10 @@ void run_mixed(csl_mixed* h, size_t B, const double* d_tp, const double* d_tp3, 
         ++launches;
     };
     auto reduce = [&](size_t ri) {
-        hipLaunchKernelGGL(csl::k_mixed_reduce, dim3(unsigned(B)), dim3(256), 0, s, h->partials.p, nblk, int(B),
-                           int(ri), inv2, inv3, invE, Rp, RS);
+        hipLaunchKernelGGL(csl::k_mixed_reduce, dim3(unsigned(B), tl ? 2u : 1u), dim3(256), 0, s, h->partials.p,
+                           tl ? h->tpartials.p : nullptr, nblk, int(B), int(ri), inv2, inv3, invE, Rp,
+                           tl ? h->trecs.p : nullptr, RS);
         hip_check(hipGetLastError(), "k_mixed_reduce");
-        if (tl) {
-            hipLaunchKernelGGL(csl::k_mixed_reduce, dim3(unsigned(B)), dim3(256), 0, s, h->tpartials.p, nblk,
-                               int(B), int(ri), inv2, inv3, invE, h->trecs.p, int(B));
-            hip_check(hipGetLastError(), "k_mixed_reduce");
-        }
     };
     // The whole launch sequence; with use_graph it is captured once into a
     // hipGraph and replayed while the key (shapes, time grid, device
@@ -1695,7 +1775,7 @@ void run_mixed(csl_mixed* h, size_t B, const double* d_tp, const double* d_tp3, 
             A.zcur = h->ZX.p;
             A.znext = h->zaux.p;
             A.tpartials = h->tpartials.p;
-            hipLaunchKernelGGL(csl::k_mixed_stage<true>, grid_dim, dim3(256), 0, s, h->M, A);
+            hipLaunchKernelGGL(tl_kernel, grid_dim, dim3(256), 0, s, h->M, A);
         } else {
             hipLaunchKernelGGL(csl::k_mixed_stage<false>, grid_dim, dim3(256), 0, s, h->M, A);
         }
@@ -2016,8 +2096,8 @@ void run_mixed_tableau(csl_mixed* h, const Tableau& T, const std::vector<double>
         A.partials = h->partials.p;
         hipLaunchKernelGGL(csl::k_mixed_stage<false>, dim3(unsigned(nblk), 1u, 1u), dim3(256), 0, s, M, A);
         hip_check(hipGetLastError(), "k_mixed_stage");
-        hipLaunchKernelGGL(csl::k_mixed_reduce, dim3(1u), dim3(256), 0, s, h->partials.p, nblk, 1, int(ri), inv2,
-                           inv3, invE, h->recs.p, 1);
+        hipLaunchKernelGGL(csl::k_mixed_reduce, dim3(1u), dim3(256), 0, s, h->partials.p, nullptr, nblk, 1, int(ri),
+                           inv2, inv3, invE, h->recs.p, nullptr, 1);
         hip_check(hipGetLastError(), "k_mixed_reduce");
     };
     hipEvent_t e0, e1;

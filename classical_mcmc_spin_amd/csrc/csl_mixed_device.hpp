@@ -59,16 +59,18 @@ struct MixDev {
 constexpr int kRec = CSL_MIXED_RECORD;
 
 // d_a = f_abc H_b S_c over the 9 non-zero (a<b<c) structure constants
-// (cross_prod_SU3_flat, simple_linear_alg.h:78-169)
+// (cross_prod_SU3_flat, simple_linear_alg.h:78-169).  The fused products are
+// written out, so every kernel rounds a site the same way (the compiler
+// otherwise fuses one or the other product as it sees fit).
 __device__ __forceinline__ void su3_cross(const double* H, const double* S, double* d) {
     constexpr double h = 0.5;
     constexpr double r = 0.8660254037844386;  // sqrt(3)/2
 #pragma unroll
     for (int i = 0; i < 8; ++i) d[i] = 0.0;
     auto tri = [&](int a, int b, int c, double v) {
-        d[a] += v * (H[b] * S[c] - H[c] * S[b]);
-        d[b] += v * (H[c] * S[a] - H[a] * S[c]);
-        d[c] += v * (H[a] * S[b] - H[b] * S[a]);
+        d[a] = fma(v, fma(H[b], S[c], -(H[c] * S[b])), d[a]);
+        d[b] = fma(v, fma(H[c], S[a], -(H[a] * S[c])), d[b]);
+        d[c] = fma(v, fma(H[a], S[b], -(H[b] * S[a])), d[c]);
     };
     tri(0, 1, 2, 1.0);
     tri(0, 3, 6, h);
@@ -79,6 +81,20 @@ __device__ __forceinline__ void su3_cross(const double* H, const double* S, doub
     tri(2, 5, 6, -h);
     tri(3, 4, 7, r);
     tri(5, 6, 7, r);
+}
+
+// dS/dt of an SU(2) site with its Gilbert term (mixed_lattice_md.cpp:570-578)
+__device__ __forceinline__ void ll_mixed_su2(const double* H, const double* S, double alpha, double k[3]) {
+    k[0] = fma(H[1], S[2], -(H[2] * S[1]));
+    k[1] = fma(H[2], S[0], -(H[0] * S[2]));
+    k[2] = fma(H[0], S[1], -(H[1] * S[0]));
+    if (alpha != 0.0) {
+        const double S2 = fma(S[0], S[0], fma(S[1], S[1], S[2] * S[2]));
+        const double SH = fma(S[0], H[0], fma(S[1], H[1], S[2] * H[2]));
+        const double g = (S2 > 0.0) ? alpha / sqrt(S2) : 0.0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) k[d] = fma(g, fma(S[d], SH, -(H[d] * S2)), k[d]);
+    }
 }
 
 __device__ __forceinline__ double envelope(double amp, double t, double tc, double width, double freq) {

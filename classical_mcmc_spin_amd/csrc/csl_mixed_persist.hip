@@ -320,14 +320,8 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
                     for (int d = 0; d < 3; ++d) e = fma(S[d], H[d] - wrow[3 * a + d], e);
                     sums2(slot, j, S);
                 }
-                double k[3] = {H[1] * S[2] - H[2] * S[1], H[2] * S[0] - H[0] * S[2], H[0] * S[1] - H[1] * S[0]};
-                if (M->alpha != 0.0) {  // mixed_lattice_md.cpp:570-578
-                    const double S2 = S[0] * S[0] + S[1] * S[1] + S[2] * S[2];
-                    const double SH = S[0] * H[0] + S[1] * H[1] + S[2] * H[2];
-                    const double g = (S2 > 0.0) ? M->alpha / sqrt(S2) : 0.0;
-#pragma unroll
-                    for (int d = 0; d < 3; ++d) k[d] += g * (S[d] * SH - H[d] * S2);
-                }
+                double k[3];
+                ll_mixed_su2(H, S, M->alpha, k);
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
                     acc2[j][d] = (s == 0 ? S[d] : acc2[j][d]) + bdt * k[d];

@@ -91,16 +91,7 @@ struct Fe {
         }
     }
     __device__ __forceinline__ void rhs(cptr<MixDev> M, int, bool, const double* H, const double* S, double k[3]) const {
-        k[0] = H[1] * S[2] - H[2] * S[1];
-        k[1] = H[2] * S[0] - H[0] * S[2];
-        k[2] = H[0] * S[1] - H[1] * S[0];
-        if (M->alpha != 0.0) {  // mixed_lattice_md.cpp:570-578
-            const double S2 = S[0] * S[0] + S[1] * S[1] + S[2] * S[2];
-            const double SH = S[0] * H[0] + S[1] * H[1] + S[2] * H[2];
-            const double g = (S2 > 0.0) ? M->alpha / sqrt(S2) : 0.0;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) k[d] += g * (S[d] * SH - H[d] * S2);
-        }
+        ll_mixed_su2(H, S, M->alpha, k);
     }
     static __device__ __forceinline__ void load(const Lay& Y, const double* buf, int p, double v[3]) {
         ld3(buf + Y.f + 3 * p, v);
