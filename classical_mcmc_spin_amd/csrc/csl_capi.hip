@@ -74,6 +74,19 @@ struct PartPlan {
     DBuf<int> halo_src, n_halo, nbr;
 };
 
+// Buffers and transform plans of the structure factor.
+struct DqWork {
+    DBuf<double> pos, cin, cf, sqt, phase, out, samples;
+    hipfftHandle p3 = 0, p1 = 0;
+    std::array<size_t, 6> key{};
+    void drop_plans() {
+        if (p3) (void)hipfftDestroy(p3);
+        if (p1) (void)hipfftDestroy(p1);
+        p3 = p1 = 0;
+    }
+    ~DqWork() { drop_plans(); }
+};
+
 struct csl_lattice {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -94,6 +107,7 @@ struct csl_lattice {
     DBuf<double> X, ACC, Y1, Y2, partials, fac, tgrid, rec_mags, rec_energy, rec_states, aux;
     DBuf<double> KS;              // stage derivatives of the generic fixed-step engine [S][3][NP]
     DBuf<double> bt_init, bt_tp, bt_amp, bt_final;
+    DqWork dq;                    // structure factor
     DBuf<double> pp_recs;         // pump-probe records, trajectory by trajectory
     DBuf<int> pp_keep;
     DBuf<double> dp_times;        // Dormand-Prince records: times [B][max_rec]
@@ -135,6 +149,7 @@ struct csl_lattice {
     hipGraphExec_t graph_exec = nullptr;
     std::vector<unsigned char> graph_key;
     ~csl_lattice() {
+        dq.drop_plans();  // before their stream
         if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
         if (stream2) (void)hipStreamDestroy(stream2);
         if (stream) (void)hipStreamDestroy(stream);
@@ -481,7 +496,8 @@ ScratchLayout scratch_layout(size_t n_grid, size_t G, size_t sched_ints, size_t 
 void run_persistent(csl_lattice* h, size_t B, const double* d_init, size_t init_stride,
                     const double* d_tp, const double* d_amp, const std::vector<double>& grid,
                     double dt, size_t si, bool want_energy, bool want_final, const TuneVal& tv,
-                    double* ms_out, const ExtBufs* ext = nullptr) {
+                    double* ms_out, const ExtBufs* ext = nullptr, double* d_samples = nullptr, size_t sample_every = 0,
+                    size_t n_samples = 0) {
     const size_t n_steps = grid.size() - 1;
     const size_t n_rec = records_for(n_steps, si);
     if (n_steps > size_t(std::numeric_limits<int>::max())) fail(CSL_ERR_ARG, "too many steps");
@@ -510,6 +526,9 @@ void run_persistent(csl_lattice* h, size_t B, const double* d_init, size_t init_
     A.save_interval = int(si);
     A.n_rec = int(n_rec);
     A.dt = dt;
+    A.samples = d_samples;
+    A.sample_every = int(sample_every);
+    A.n_samples = int(n_samples);
     csl::LatDev L = h->L;
     if (h->rep_B) {
         if (B != h->rep_B) fail(CSL_ERR_ARG, "batch size differs from the per-replica Hamiltonians set");
@@ -2600,65 +2619,89 @@ int csl_structure_factor(csl_lattice* h, size_t B, const double* init, int init_
         check_finite(init, init_per_replica ? B * nd : nd, "initial state");
         hipStream_t s = h->stream;
         h->bt_init.upload(init, init_per_replica ? B * nd : nd, s);
-        h->X.ensure(B * 3 * size_t(L.NP));
-        hip_check(hipMemsetAsync(h->X.p, 0, B * 3 * size_t(L.NP) * sizeof(double), s), "memset");
-        hip_check(csl::launch_perm_to_soa(L, h->bt_init.p, init_per_replica ? nd : 0, h->X.p, int(B), s), "perm");
-        DBuf<double> pos, cin, cf, sqt, out;
-        pos.upload(positions, h->n_atoms * 3, s);
-        const size_t nbatch3 = B * h->n_atoms * 3;
-        cin.ensure(2 * nbatch3 * Q);
-        cf.ensure(2 * nbatch3 * Q);
-        const size_t R = B * 3 * Q;
-        sqt.ensure(2 * n_t * R);
-        out.ensure(Q * n_t);
-        hipfftHandle p3 = 0, p1 = 0;
-        auto fft_check = [](hipfftResult r, const char* what) {
-            if (r != HIPFFT_SUCCESS) fail(CSL_ERR_HIP, std::string(what) + " failed (hipFFT status " + std::to_string(int(r)) + ")");
-        };
-        struct PlanGuard {
-            hipfftHandle& a;
-            hipfftHandle& b;
-            ~PlanGuard() {
-                if (a) hipfftDestroy(a);
-                if (b) hipfftDestroy(b);
-            }
-        } guard{p3, p1};
-        int dims3[3] = {int(L1), int(L2), int(L3)};
-        fft_check(hipfftCreate(&p3), "hipfftCreate");
-        size_t ws = 0;
-        fft_check(hipfftMakePlanMany(p3, 3, dims3, nullptr, 1, int(Q), nullptr, 1, int(Q), HIPFFT_Z2Z, int(nbatch3), &ws),
-                  "3-D plan");
-        fft_check(hipfftSetStream(p3, s), "hipfftSetStream");
-        int dims1[1] = {int(n_t)};
-        fft_check(hipfftCreate(&p1), "hipfftCreate");
-        fft_check(hipfftMakePlanMany(p1, 1, dims1, dims1, int(R), 1, dims1, int(R), 1, HIPFFT_Z2Z, int(R), &ws),
-                  "time plan");
-        fft_check(hipfftSetStream(p1, s), "hipfftSetStream");
-        auto* cin2 = reinterpret_cast<double2*>(cin.p);
-        auto* cf2 = reinterpret_cast<double2*>(cf.p);
-        auto* sqt2 = reinterpret_cast<double2*>(sqt.p);
-        auto sample = [&](size_t n) {
-            if (n % sample_interval || n / sample_interval >= n_t) return;
-            const size_t ti = n / sample_interval;
-            hip_check(csl::launch_sq_fill(L, h->X.p, int(B), cin2, s), "k_sq_fill");
-            fft_check(hipfftExecZ2Z(p3, reinterpret_cast<hipfftDoubleComplex*>(cin2),
-                                    reinterpret_cast<hipfftDoubleComplex*>(cf2), HIPFFT_FORWARD),
-                      "3-D FFT");
-            hip_check(csl::launch_sq_combine(cf2, int(B), int(h->n_atoms), int(L1), int(L2), int(L3), pos.p,
-                                             sqt2 + ti * R, s),
-                      "k_sq_combine");
-        };
+        if (h->rep_B) fail(CSL_ERR_UNSUPPORTED, "per-replica Hamiltonians need the persistent kernel");
         std::vector<double> zero(2 * B, 0.0);
         h->bt_tp.upload(zero.data(), zero.size(), s);
         h->bt_amp.upload(zero.data(), zero.size(), s);
-        if (h->rep_B) fail(CSL_ERR_UNSUPPORTED, "per-replica Hamiltonians need the persistent kernel");
-        run_stages(h, B, h->bt_tp.p, h->bt_amp.p, false, grid, dt, 1, false, nullptr, sample);
-        fft_check(hipfftExecZ2Z(p1, reinterpret_cast<hipfftDoubleComplex*>(sqt2),
+        const size_t per = B * h->n_atoms * 3;   // grids of one sample
+        const size_t R = B * 3 * Q;
+        // a lattice of one workgroup: the persistent kernel leaves the
+        // samples behind (when they take at most a quarter of the free
+        // memory), and their grids are transformed many samples at a time
+        size_t free_b = 0, total_b = 0;
+        hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+        const bool persistent = !persistent_candidates(h).empty() && n_t * per * Q * sizeof(double) <= free_b / 4 &&
+                                n_steps <= size_t(std::numeric_limits<int>::max());
+        // samples per transform: grids of at most 256 MB
+        const size_t nc = persistent ? std::max<size_t>(1, std::min(n_t, (size_t(256) << 20) / (per * Q * 16))) : 1;
+        DqWork& w = h->dq;
+        w.pos.upload(positions, h->n_atoms * 3, s);
+        w.cin.ensure(2 * nc * per * Q);
+        w.cf.ensure(2 * nc * per * Q);
+        w.sqt.ensure(2 * n_t * R);
+        w.phase.ensure(2 * h->n_atoms * Q);
+        w.out.ensure(Q * n_t);
+        auto fft_check = [](hipfftResult r, const char* what) {
+            if (r != HIPFFT_SUCCESS) fail(CSL_ERR_HIP, std::string(what) + " failed (hipFFT status " + std::to_string(int(r)) + ")");
+        };
+        // plans kept on the handle while the shapes stay (making them takes
+        // longer than a small run)
+        const std::array<size_t, 6> key{L1, L2, L3, nc * per, n_t, R};
+        if (!w.p3 || w.key != key) {
+            w.drop_plans();
+            size_t ws = 0;
+            int dims3[3] = {int(L1), int(L2), int(L3)};
+            fft_check(hipfftCreate(&w.p3), "hipfftCreate");
+            fft_check(hipfftMakePlanMany(w.p3, 3, dims3, nullptr, 1, int(Q), nullptr, 1, int(Q), HIPFFT_Z2Z,
+                                         int(nc * per), &ws),
+                      "3-D plan");
+            fft_check(hipfftSetStream(w.p3, s), "hipfftSetStream");
+            int dims1[1] = {int(n_t)};
+            fft_check(hipfftCreate(&w.p1), "hipfftCreate");
+            fft_check(hipfftMakePlanMany(w.p1, 1, dims1, dims1, int(R), 1, dims1, int(R), 1, HIPFFT_Z2Z, int(R), &ws),
+                      "time plan");
+            fft_check(hipfftSetStream(w.p1, s), "hipfftSetStream");
+            w.key = key;
+        }
+        auto* cin2 = reinterpret_cast<double2*>(w.cin.p);
+        auto* cf2 = reinterpret_cast<double2*>(w.cf.p);
+        auto* sqt2 = reinterpret_cast<double2*>(w.sqt.p);
+        auto* ph2 = reinterpret_cast<double2*>(w.phase.p);
+        hip_check(csl::launch_sq_phase(int(h->n_atoms), int(L1), int(L2), int(L3), w.pos.p, ph2, s), "k_sq_phase");
+        // grids in cin -> S(q, t) of nc samples from ti on
+        auto transform = [&](size_t ti) {
+            fft_check(hipfftExecZ2Z(w.p3, reinterpret_cast<hipfftDoubleComplex*>(cin2),
+                                    reinterpret_cast<hipfftDoubleComplex*>(cf2), HIPFFT_FORWARD),
+                      "3-D FFT");
+            hip_check(csl::launch_sq_combine(cf2, nc * B, int(h->n_atoms), Q, ph2, sqt2 + ti * R, s), "k_sq_combine");
+        };
+        if (persistent) {
+            w.samples.ensure(n_t * per * Q);
+            run_persistent(h, B, h->bt_init.p, init_per_replica ? nd : 0, h->bt_tp.p, h->bt_amp.p, grid, dt, 1, false,
+                           false, pick_persistent(h, B, 0), nullptr, nullptr, w.samples.p, sample_interval, n_t);
+            // the last transform starts early enough to be a full one
+            for (size_t c = 0; c < n_t; c += nc) {
+                const size_t ti = std::min(c, n_t - nc);
+                hip_check(csl::launch_sq_expand(w.samples.p + ti * per * Q, nc * per * Q, cin2, s), "k_sq_expand");
+                transform(ti);
+            }
+        } else {
+            h->X.ensure(B * 3 * size_t(L.NP));
+            hip_check(hipMemsetAsync(h->X.p, 0, B * 3 * size_t(L.NP) * sizeof(double), s), "memset");
+            hip_check(csl::launch_perm_to_soa(L, h->bt_init.p, init_per_replica ? nd : 0, h->X.p, int(B), s), "perm");
+            auto sample = [&](size_t n) {
+                if (n % sample_interval || n / sample_interval >= n_t) return;
+                hip_check(csl::launch_sq_fill(L, h->X.p, int(B), cin2, s), "k_sq_fill");
+                transform(n / sample_interval);
+            };
+            run_stages(h, B, h->bt_tp.p, h->bt_amp.p, false, grid, dt, 1, false, nullptr, sample);
+        }
+        fft_check(hipfftExecZ2Z(w.p1, reinterpret_cast<hipfftDoubleComplex*>(sqt2),
                                 reinterpret_cast<hipfftDoubleComplex*>(sqt2), HIPFFT_FORWARD),
                   "time FFT");
-        hip_check(csl::launch_sq_power(sqt2, int(n_t), int(B), Q, 1.0 / (double(B) * double(h->N) * double(n_t)), out.p, s),
+        hip_check(csl::launch_sq_power(sqt2, int(n_t), int(B), Q, 1.0 / (double(B) * double(h->N) * double(n_t)), w.out.p, s),
                   "k_sq_power");
-        copy_back(sqw, out.p, Q * n_t, s);
+        copy_back(sqw, w.out.p, Q * n_t, s);
         copy_back(mags, h->rec_mags.p, (n_steps + 1) * B * 9, s);
         hip_check(hipStreamSynchronize(s), "structure factor");
     });

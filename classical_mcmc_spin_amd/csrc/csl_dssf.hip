@@ -5,9 +5,11 @@
 //
 // r_i = cell vector (i, j, k) + the atom's position in the cell (in units of
 // the cell's lattice vectors, which are orthonormal for the cubic
-// pyrochlore cell).  Per sample step the spins of every (trajectory, atom,
-// component) are expanded into a complex 3-D grid over the cells, a batched
-// 3-D FFT (hipFFT) gives F_a,atom(q), and k_sq_combine sums the atoms with
+// pyrochlore cell).  Lattices of one workgroup integrate on the persistent
+// kernel, which leaves the samples behind; larger ones on the stage kernels,
+// sample by sample.  The spins of every (trajectory, atom,
+// component) are expanded into a complex 3-D grid over the cells, batched
+// 3-D FFTs (hipFFT) gives F_a,atom(q), and k_sq_combine sums the atoms with
 // their position phases into the S(q, t) buffer; after the run a batched
 // 1-D FFT along t and k_sq_power give S(q, w).  The reference post-processes
 // saved spin snapshots in Python (util/readers_new/reader_pyrochlore.py:150-270).
@@ -33,30 +35,45 @@ __global__ void k_sq_fill(LatDev L, const double* __restrict__ x, int B, double2
     out[id] = make_double2(x[(size_t(b) * 3 + comp) * L.NP + p], 0.0);
 }
 
-// F [B][n_atoms][3][Q] -> S(q, t) slot [B][3][Q]: sum_atom exp(-i q.r_atom) F
-__global__ void k_sq_combine(const double2* __restrict__ F, int B, int n_atoms, int L1, int L2, int L3,
-                             const double* __restrict__ pos, double2* __restrict__ sqt) {
-    const size_t id = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+__global__ void k_sq_expand(const double* __restrict__ v, size_t n, double2* __restrict__ out) {
+    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = make_double2(v[i], 0.0);
+}
+
+// exp(-i q . r_atom) of every wave vector, once per run (each sample's
+// combination evaluated the sines of all atoms again)
+__global__ void k_sq_phase(int n_atoms, int L1, int L2, int L3, const double* __restrict__ pos,
+                           double2* __restrict__ phase) {
     const size_t Q = size_t(L1) * L2 * L3;
-    const size_t total = size_t(B) * 3 * Q;
-    if (id >= total) return;
+    const size_t id = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (id >= Q * n_atoms) return;
     const size_t q = id % Q;
-    const size_t r = id / Q;           // (b, comp)
-    const int comp = int(r % 3);
-    const int b = int(r / 3);
+    const int a = int(id / Q);
     const int h = int(q / (size_t(L2) * L3));
     const int k = int((q / L3) % L2);
     const int l = int(q % L3);
     const double two_pi = 6.283185307179586;
     const double qx = two_pi * h / L1, qy = two_pi * k / L2, qz = two_pi * l / L3;
+    const double ph = -(qx * pos[3 * a] + qy * pos[3 * a + 1] + qz * pos[3 * a + 2]);
+    double s, c;
+    sincos(ph, &s, &c);
+    phase[id] = make_double2(c, s);
+}
+
+// F [B][n_atoms][3][Q] -> S(q, t) [B][3][Q]: sum_atom exp(-i q.r_atom) F
+__global__ void k_sq_combine(const double2* __restrict__ F, size_t B, int n_atoms, size_t Q,
+                             const double2* __restrict__ phase, double2* __restrict__ sqt) {
+    const size_t id = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (id >= B * 3 * Q) return;
+    const size_t q = id % Q;
+    const size_t r = id / Q;           // (b, comp)
+    const size_t comp = r % 3, b = r / 3;
     double re = 0.0, im = 0.0;
     for (int a = 0; a < n_atoms; ++a) {
-        const double ph = -(qx * pos[3 * a] + qy * pos[3 * a + 1] + qz * pos[3 * a + 2]);
-        double s, c;
-        sincos(ph, &s, &c);
-        const double2 f = F[((size_t(b) * n_atoms + a) * 3 + comp) * Q + q];
-        re += c * f.x - s * f.y;
-        im += c * f.y + s * f.x;
+        const double2 f = F[((b * n_atoms + a) * 3 + comp) * Q + q];
+        const double2 p = phase[size_t(a) * Q + q];
+        re += p.x * f.x - p.y * f.y;
+        im += p.x * f.y + p.y * f.x;
     }
     sqt[id] = make_double2(re, im);
 }
@@ -82,11 +99,21 @@ hipError_t launch_sq_fill(const LatDev& L, const double* x, int B, double2* out,
     return hipGetLastError();
 }
 
-hipError_t launch_sq_combine(const double2* F, int B, int n_atoms, int L1, int L2, int L3, const double* pos,
-                             double2* sqt, hipStream_t st) {
-    const size_t total = size_t(B) * 3 * L1 * L2 * L3;
-    hipLaunchKernelGGL(k_sq_combine, dim3(unsigned((total + 255) / 256)), dim3(256), 0, st, F, B, n_atoms, L1, L2,
-                       L3, pos, sqt);
+hipError_t launch_sq_expand(const double* v, size_t n, double2* out, hipStream_t st) {
+    hipLaunchKernelGGL(k_sq_expand, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, v, n, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_sq_phase(int n_atoms, int L1, int L2, int L3, const double* pos, double2* phase, hipStream_t st) {
+    const size_t total = size_t(n_atoms) * L1 * L2 * L3;
+    hipLaunchKernelGGL(k_sq_phase, dim3(unsigned((total + 255) / 256)), dim3(256), 0, st, n_atoms, L1, L2, L3, pos, phase);
+    return hipGetLastError();
+}
+
+hipError_t launch_sq_combine(const double2* F, size_t B, int n_atoms, size_t Q, const double2* phase, double2* sqt,
+                             hipStream_t st) {
+    const size_t total = B * 3 * Q;
+    hipLaunchKernelGGL(k_sq_combine, dim3(unsigned((total + 255) / 256)), dim3(256), 0, st, F, B, n_atoms, Q, phase, sqt);
     return hipGetLastError();
 }
 

@@ -40,12 +40,22 @@ struct PersistArgs {
     double* saved;           // [slots][NP][3] device-order states at the seams
     unsigned* flags;         // [slots], zero before the launch
     unsigned* status;        // set to 1 if a wait for a slot gave up
+    // State samples for the structure factor: the state at every
+    // sample_every-th step start (n_samples of them) as
+    // [n_samples][B][n_atoms][3][n_cells], or sample_every 0
+    double* samples;
+    int sample_every, n_samples;
     // Lattices of different sizes in one launch (kPersistMulti): trajectory b
     // runs on lats[lat_of[b]] and starts from init + init_off[b]
     const LatDev* lats;
     const int* lat_of;
     const size_t* init_off;
 };
+
+// Where trajectory b's sample ti of sublattice `atom` starts (3 n_cells values).
+__device__ __forceinline__ double* sample_row(double* samples, int B, int n_atoms, int n_cells, int ti, int b, int atom) {
+    return samples + ((size_t(ti) * B + b) * n_atoms + atom) * 3 * size_t(n_cells);
+}
 
 // Partitioned persistent batched integration (csl_partition.hip), for
 // lattices whose state does not fit one workgroup's LDS: each trajectory is
@@ -210,8 +220,13 @@ hipError_t launch_quench_check(const double* e, double* e_prev, int* frozen, int
 
 // structure factor (csl_dssf.hip)
 hipError_t launch_sq_fill(const LatDev& L, const double* x, int B, double2* out, hipStream_t st);
-hipError_t launch_sq_combine(const double2* F, int B, int n_atoms, int L1, int L2, int L3, const double* pos,
-                             double2* sqt, hipStream_t st);
+// out[i] = (v[i], 0)
+hipError_t launch_sq_expand(const double* v, size_t n, double2* out, hipStream_t st);
+// phases [n_atoms][Q] of the atoms' positions at the Q wave vectors
+hipError_t launch_sq_phase(int n_atoms, int L1, int L2, int L3, const double* pos, double2* phase, hipStream_t st);
+// B trajectories (of one or of several samples in turn)
+hipError_t launch_sq_combine(const double2* F, size_t B, int n_atoms, size_t Q, const double2* phase, double2* sqt,
+                             hipStream_t st);
 hipError_t launch_sq_power(const double2* sw, int T, int B, size_t Q, double scale, double* out, hipStream_t st);
 
 

@@ -292,6 +292,15 @@ __global__ void __launch_bounds__(persistent_max_block<SPT>()) k_persistent(LatD
         const bool rec = (n % A.save_interval) == 0;
         const int ri = n / A.save_interval;
         if (n + 1 < s_end) write_drive(n + 1);
+        if (A.sample_every && n % A.sample_every == 0 && n / A.sample_every < A.n_samples) {
+#pragma unroll
+            for (int m = 0; m < SPT; ++m)
+                if (act[m]) {
+                    double* row = sample_row(A.samples, A.B, L0.n_atoms, L0.n_cells, n / A.sample_every, b, atm[m]);
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) row[size_t(d) * L0.n_cells + (site(m) - atm[m] * L0.npad)] = x[m][d];
+                }
+        }
         if constexpr (UNROLL) {
             stage(std::integral_constant<int, 0>{}, par, rec, ri);
             stage(std::integral_constant<int, 1>{}, par, rec, ri);

@@ -49,7 +49,7 @@ __device__ __forceinline__ KP kern_args() {
 
 // The waves that own NU units.  The barriers of a workgroup's waves pair up
 // by count, whichever instance a wave runs.
-template <int SPT, int NU, int ZMAX, bool DAMP>
+template <int SPT, int NU, int ZMAX, bool DAMP, bool SAMP>
 __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, int wave, int wstart) {
     const int NP = K.L.NP, n_atoms = K.L.n_atoms, npad = K.L.npad;
     const int T = blockDim.x;
@@ -348,6 +348,12 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
         const int si = K.A.save_interval;
         int ri = (s_begin + si - 1) / si;      // first record at or after s_begin
         int next_rec = ri * si;
+        int smp = 0, next_smp = -1;            // next state sample
+        if constexpr (SAMP) {
+            const int se = K.A.sample_every;
+            smp = (s_begin + se - 1) / se;
+            next_smp = smp < K.A.n_samples ? smp * se : -1;
+        }
         for (int n0 = s_begin, cp = 0; n0 < s_end; n0 += C, cp ^= 1) {
             const int n1 = min(n0 + C, s_end);
             const int ri0 = ri;
@@ -359,6 +365,20 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
                     slot = ri - ri0;
                     ++ri;
                     next_rec += si;
+                }
+                if (SAMP && n == next_smp) {
+                    const KP G = kern_args();
+                    double* row = sample_row(G->A.samples, G->A.B, n_atoms, G->L.n_cells, smp, b, atom);
+#pragma unroll
+                    for (int m = 0; m < NU; ++m) {
+                        const int cell = pbase + m * kWave - atom * npad;
+                        if (cell < G->L.n_cells) {
+#pragma unroll
+                            for (int d = 0; d < 3; ++d) row[size_t(d) * G->L.n_cells + cell] = x[m][d];
+                        }
+                    }
+                    ++smp;
+                    next_smp = smp < G->A.n_samples ? next_smp + G->A.sample_every : -1;
                 }
                 const int q = n + 1 - n0;
                 if (n + 1 < s_end && q < C) write_hin(drv + (cp * C + q) * 6, par ^ 1);
@@ -426,8 +446,9 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
 
 }  // namespace
 
-// SPT: the most units a wave owns; the others own one less.
-template <int SPT, int ZMAX, bool DAMP>
+// SPT: the most units a wave owns; the others own one less.  SAMP: the launch
+// stores state samples (without them the test alone costs 3 % at 24x24).
+template <int SPT, int ZMAX, bool DAMP, bool SAMP>
 __global__ void __launch_bounds__(persistent_max_block<SPT>()) k_trajectory(TrajKernArgs K) {
     extern __shared__ double smem[];
     const int wave = uniform(threadIdx.x >> 6);
@@ -435,15 +456,15 @@ __global__ void __launch_bounds__(persistent_max_block<SPT>()) k_trajectory(Traj
     atom_major_tile(blockDim.x >> 6, K.L.n_atoms, K.L.npad / kWave, wave, wstart, wunits);
     wstart = uniform(wstart);
     wunits = uniform(wunits);
-    if (SPT == 1 || wunits == SPT) run_wave<SPT, SPT, ZMAX, DAMP>(K, smem, wave, wstart);
-    else run_wave<SPT, (SPT > 1 ? SPT - 1 : 1), ZMAX, DAMP>(K, smem, wave, wstart);
+    if (SPT == 1 || wunits == SPT) run_wave<SPT, SPT, ZMAX, DAMP, SAMP>(K, smem, wave, wstart);
+    else run_wave<SPT, (SPT > 1 ? SPT - 1 : 1), ZMAX, DAMP, SAMP>(K, smem, wave, wstart);
 }
 
 namespace {
 
-template <int SPT, int ZMAX, bool DAMP>
+template <int SPT, int ZMAX, bool DAMP, bool SAMP>
 hipError_t launch_t(const TrajKernArgs& K, int block, size_t lds, hipStream_t st, int* occ) {
-    auto kern = k_trajectory<SPT, ZMAX, DAMP>;
+    auto kern = k_trajectory<SPT, ZMAX, DAMP, SAMP>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
@@ -454,8 +475,12 @@ hipError_t launch_t(const TrajKernArgs& K, int block, size_t lds, hipStream_t st
 
 template <int SPT, int ZMAX>
 hipError_t launch_t_damp(const TrajKernArgs& K, int block, size_t lds, hipStream_t st, int* occ) {
-    return K.L.alpha > 0.0 ? launch_t<SPT, ZMAX, true>(K, block, lds, st, occ)
-                           : launch_t<SPT, ZMAX, false>(K, block, lds, st, occ);
+    const bool damp = K.L.alpha > 0.0, samp = K.A.sample_every > 0;
+    if (samp)
+        return damp ? launch_t<SPT, ZMAX, true, true>(K, block, lds, st, occ)
+                    : launch_t<SPT, ZMAX, false, true>(K, block, lds, st, occ);
+    return damp ? launch_t<SPT, ZMAX, true, false>(K, block, lds, st, occ)
+                : launch_t<SPT, ZMAX, false, false>(K, block, lds, st, occ);
 }
 
 }  // namespace

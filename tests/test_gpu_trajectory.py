@@ -94,3 +94,35 @@ def test_pump_probe_rows(n_tau, steps):
     assert np.array_equal(r["M0"], m[:, 0])
     assert np.array_equal(r["M1"], np.swapaxes(m[:, 1:1 + n_tau], 0, 1))
     assert np.array_equal(r["M01"], np.swapaxes(m[:, 1 + n_tau:], 0, 1))
+
+
+@pytest.mark.parametrize("dims,steps,every", [((5, 3, 1), 19, 1), ((13, 5, 1), 24, 8), ((4, 6, 1), 37, 5)])
+@pytest.mark.parametrize("onsite", [0.0, 0.1])
+def test_structure_factor_samples(dims, steps, every, onsite):
+    """Samples left by the persistent kernels (atom-major, and the general
+    one for an onsite matrix) and their batched transforms against numpy on
+    the stage engine's states.  The power sums |S(q, w)|^2 of some thousand
+    rounded terms: 1e-12 relative to the largest."""
+    lat = model.Lattice(_kitaev(Ka=onsite, Kb=-onsite, Kc=0.5 * onsite), *dims)
+    B, n_t = 3, steps // every
+    T1 = (steps + 0.5) * DT
+    init = np.stack([random_state(lat, 40 + b) for b in range(B)])
+    pos = np.array([[0.0, 0.0, 0.0], [0.1, 0.55, 0.0]])
+    print(f"[dssf] {dims} steps {steps} every {every} onsite {onsite}", flush=True)
+    states = []
+    with GPULattice(lat) as gl:
+        r = gl.structure_factor(init, 0.0, T1, DT, every, dims, pos, want_mags=True)
+        for b in range(B):
+            gl.set_spins(init[b])
+            states.append(gl.integrate(0.0, T1, DT, tgrid="boost", engine=1, want_states=True)["states"])
+    S = np.stack(states, 1)[:-1:every][:n_t]                       # [n_t, B, N, 3]
+    F = np.fft.fftn(S.reshape((n_t, B) + dims + (2, 3)), axes=(2, 3, 4))
+    q = np.stack(np.meshgrid(*[2 * np.pi * np.arange(L) / L for L in dims], indexing="ij"), -1)
+    ph = np.exp(-1j * np.einsum("ijkc,ac->ijka", q, pos))
+    sw = np.fft.fft((F * ph[..., None]).sum(-2), axis=0)
+    p = (np.abs(sw) ** 2).sum((1, 5)) / (B * lat.lattice_size * n_t)
+    ref = p.reshape(n_t, -1).T
+    assert r["sqw"].shape == ref.shape
+    assert np.max(np.abs(r["sqw"] - ref)) <= 1e-12 * np.max(ref)
+    m = S.mean(2)
+    assert np.max(np.abs(r["mags"][:-1:every][:n_t, :, 1] - m)) <= 1e-13
