@@ -20,7 +20,7 @@ LIB_NAME = "libcsl_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 
 # (source, object suffix, extra flags)
-HIP_UNITS = [("csl_kernels.hip", "", []), ("csl_capi.hip", "", []), ("csl_mixed.hip", "", []), ("csl_adjoint.hip", "", []),
+HIP_UNITS = [("csl_kernels.hip", "", []), ("csl_capi.hip", "", []), ("csl_mixed.hip", "", []), ("csl_adjoint.hip", "", []), ("csl_adjoint_sweep.hip", "", []),
              ("csl_dssf.hip", "", []), ("csl_spectrum.hip", "", []), ("csl_quench.hip", "", []),
              ("csl_dopri5.hip", "", []), ("csl_partition.hip", "", []), ("csl_mixed_persist.hip", "", []),
              ("csl_mixed_waves.hip", "", [])] + [

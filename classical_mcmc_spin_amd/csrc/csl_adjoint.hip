@@ -23,6 +23,9 @@
 //                every stage of the segment (independent of each other, so
 //                they leave the sequential sweep);
 //   k_adj_final  loss and gradient sums in a fixed order.
+// Lattices with three bonds at every site, per-sublattice fields and up to
+// eight sublattices run k_adj_rows and k_adj_sweep (csl_adjoint_sweep.hip)
+// in place of k_adj_bwd and k_adj_par.
 // The values handed between kernels are exact copies, so every checkpoint
 // spacing gives the same bits.
 //

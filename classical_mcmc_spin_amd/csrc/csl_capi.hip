@@ -127,7 +127,7 @@ struct csl_lattice {
     DBuf<unsigned> part_ver;
     int last_parts = 0, last_groups = 0;
     // adjoint work buffers (stage inputs, field cotangents, checkpoints, ...)
-    DBuf<double> adj_Y, adj_U, adj_ckpt, adj_lam, adj_lossn, adj_part;
+    DBuf<double> adj_Y, adj_U, adj_ckpt, adj_lam, adj_lossn, adj_part, adj_rows;
     hipStream_t stream2 = nullptr;  // second stream of the adjoint (parameter terms)
     int stage_graph = 0;          // batched stage-kernel path replayed from a hipGraph
     int last_grid = 0;
@@ -2377,7 +2377,8 @@ int csl_adjoint_gradient(csl_lattice* h, size_t B, const double* init, int init_
         // checkpoint spacing is asked for); otherwise checkpoints every C
         // steps and one segment of stage inputs, re-integrated per segment.
         const size_t SZ = size_t(3) * L.NP;
-        const size_t per_seg_step = 2 * B * 4 * SZ * sizeof(double);  // Y and U
+        const bool sweep = csl::adjoint_sweep_fits(L);
+        const size_t per_seg_step = (sweep ? 1 : 2) * B * 4 * SZ * sizeof(double);  // Y, and U without the sweep
         size_t free_b = 0, total_b = 0;
         hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
         const size_t budget = std::min<size_t>(free_b / 2, size_t(48) << 30);
@@ -2390,12 +2391,13 @@ int csl_adjoint_gradient(csl_lattice* h, size_t B, const double* init, int init_
         DBuf<double>&d_Y = h->adj_Y, &d_U = h->adj_U, &d_lam = h->adj_lam, &d_lossn = h->adj_lossn,
                      &d_part = h->adj_part, &d_ckpt = h->adj_ckpt;
         d_Y.ensure(B * C * 4 * SZ);
-        d_U.ensure(B * C * 4 * SZ);
+        if (!sweep) d_U.ensure(B * C * 4 * SZ);
         if (!full) d_ckpt.ensure(B * n_seg * SZ);
         d_lam.ensure(B * SZ);
         d_rec.ensure(n_rec * B * 9);
         d_lossn.ensure(B * n_rec);
-        d_part.ensure(B * n_steps * 4 * std::max<size_t>(n_params, 1));
+        d_part.ensure(sweep ? B * csl::adjoint_sweep_doubles(L) : B * n_steps * 4 * std::max<size_t>(n_params, 1));
+        if (sweep) h->adj_rows.ensure(B * n_rec * csl::adjoint_row_doubles(L));
         d_loss.ensure(B);
         d_grad.ensure(B * std::max<size_t>(n_params, 1));
         if (grad_init) d_gi.ensure(B * nd);
@@ -2420,6 +2422,7 @@ int csl_adjoint_gradient(csl_lattice* h, size_t B, const double* init, int init_
         Aa.rec = d_rec.p;
         Aa.loss_n = d_lossn.p;
         Aa.part = d_part.p;
+        Aa.rows = h->adj_rows.p;
         Aa.grad_init = grad_init ? d_gi.p : nullptr;
         Aa.loss = d_loss.p;
         Aa.grad = d_grad.p;
@@ -2452,7 +2455,23 @@ int csl_adjoint_gradient(csl_lattice* h, size_t B, const double* init, int init_
                 ++launches;
             }
         }
-        if (full) {
+        csl::AdjArgs Fin = Aa;
+        if (sweep) {
+            Fin.P = 0;  // the sweep writes the gradient itself
+            hip_check(csl::launch_adjoint_rows(L, Aa, s), "k_adj_rows launch");
+            ++launches;
+        }
+        if (full && sweep) {
+            csl::AdjArgs G = Aa;
+            G.n0 = 0;
+            G.n1 = int(n_steps);
+            G.y0 = 0;
+            G.first = 1;
+            hip_check(csl::launch_adjoint_sweep(L, G, s), "k_adj_sweep launch");
+            hip_check(csl::launch_adjoint_final(Fin, s), "k_adj_final launch");
+            hip_check(hipEventRecord(e1, s), "event record");
+            ++launches;
+        } else if (full) {
             // the backward sweep in segments; the parameter terms of a
             // finished segment run on the second stream (on the CUs the
             // sweep leaves idle) while the sweep continues
@@ -2501,12 +2520,18 @@ int csl_adjoint_gradient(csl_lattice* h, size_t B, const double* init, int init_
                 G.ckpt_interval = 0;
                 G.store_stages = 1;
                 hip_check(csl::launch_adjoint_forward(L, G, s), "k_adj_fwd launch");
+                ++launches;
                 G.first = j == n_seg - 1 ? 1 : 0;
+                if (sweep) {
+                    hip_check(csl::launch_adjoint_sweep(L, G, s), "k_adj_sweep launch");
+                    ++launches;
+                    continue;
+                }
                 hip_check(csl::launch_adjoint_backward(L, G, s), "k_adj_bwd launch");
                 hip_check(csl::launch_adjoint_params(L, G, 2048, s), "k_adj_par launch");
-                launches += 3;
+                launches += 2;
             }
-            hip_check(csl::launch_adjoint_final(Aa, s), "k_adj_final launch");
+            hip_check(csl::launch_adjoint_final(Fin, s), "k_adj_final launch");
             hip_check(hipEventRecord(e1, s), "event record");
         }
         ++launches;

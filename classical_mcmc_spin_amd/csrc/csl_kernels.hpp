@@ -155,7 +155,8 @@ struct AdjArgs {
     int first;                 // the launch holds the last step: lambda starts from dl/dx_N
     double* rec;               // [n_steps+1][B][9] forward records
     double* loss_n;            // [B][n_steps+1] loss term of every record
-    double* part;              // [B][n_steps][4][P] parameter-gradient term of every stage
+    double* part;              // [B][n_steps][4][P] parameter-gradient term of every stage (sweep: thread sums)
+    double* rows;              // sweep: fields and loss cotangents of every step
     double* grad_init;         // [B][N*3] dL/dx_0 (AoS), written by the launch with n0 == 0, or null
     double* loss;              // [B] (final kernel)
     double* grad;              // [B][P] (final kernel)
@@ -171,6 +172,19 @@ hipError_t launch_adjoint_backward(const LatDev& L, const AdjArgs& A, hipStream_
 // the segment's stage slots)
 hipError_t launch_adjoint_params(const LatDev& L, const AdjArgs& A, int blocks_per_traj, hipStream_t st);
 hipError_t launch_adjoint_final(const AdjArgs& A, hipStream_t st);
+
+// The backward sweep that sums the parameter terms itself
+// (csl_adjoint_sweep.hip), for lattices with three bonds at every site,
+// per-sublattice fields and no onsite matrix whose sublattices fit its waves.
+// A.part holds the thread sums handed between segments (adjoint_sweep_doubles
+// per trajectory); the launch with n0 == 0 writes A.grad.  Before it,
+// launch_adjoint_rows turns the records of all steps into A.rows
+// (adjoint_row_doubles per trajectory and record) and the loss terms.
+bool adjoint_sweep_fits(const LatDev& L);
+size_t adjoint_sweep_doubles(const LatDev& L);
+size_t adjoint_row_doubles(const LatDev& L);
+hipError_t launch_adjoint_rows(const LatDev& L, const AdjArgs& A, hipStream_t st);
+hipError_t launch_adjoint_sweep(const LatDev& L, const AdjArgs& A, hipStream_t st);
 
 // Dormand-Prince 5(4) integration (csl_dopri5.hip): one workgroup per trajectory.
 struct Dopri5Args {
