@@ -236,6 +236,11 @@ __global__ void __launch_bounds__(adjoint_max_block<SPT>()) k_adj_fwd(LatDev Lk,
         }
     };
 
+    // padding sites are zero in both buffers (a stage writes the real ones), and so in Y
+    const double none[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int m = 0; m < SPT; ++m)
+        if (tid + m * T < NP) bufB.store(tid + m * T, none);
     // initial state: a checkpoint (SoA, device order) or the initial spins
     if (A.ckpt_src >= 0) {
         const double* src = A.ckpt + (size_t(b) * A.n_ckpt + A.ckpt_src) * SZ;
