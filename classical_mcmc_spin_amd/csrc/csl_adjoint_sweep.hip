@@ -86,14 +86,6 @@ struct Lds2 {
     }
 };
 
-// The values as they are now: products into them cannot be put off past this
-// point (with the bond's operands saved for later).
-template <int D>
-__device__ __forceinline__ void hold(double (&v)[D]) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) asm volatile("" : "+v"(v[d]));
-}
-
 template <int NU, bool DAMP>
 __device__ __forceinline__ void sweep_wave(double* smem, int wave, int wstart) {
     const KP K = kern_args();

@@ -21,6 +21,14 @@ __device__ __forceinline__ int opaque_zero() {
     return z;
 }
 
+// The values as they are now: products into them cannot be put off past this
+// point (with the bond's operands saved for later).
+template <int D>
+__device__ __forceinline__ void hold(double (&v)[D]) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) asm volatile("" : "+v"(v[d]));
+}
+
 __device__ __forceinline__ LatDev refresh(const LatDev& L0) {
     LatDev L = L0;
     const int z = opaque_zero();

@@ -32,8 +32,23 @@
 // directions with scalar loads (translation-invariant tables only).  Records
 // are per-part sums of the observables (reduced over the parts by a second
 // kernel in a fixed order).
+//
+// Where a wave's sites all lie in one sublattice (AM, launch_part_t) a bond's
+// matrix is read once for them and the bonds run one after the other over all
+// of them, a recorded step leaves four sums per wave (S and S.H) instead of
+// ten, and the record is put together after the version is out.  32
+// trajectories of the 16^3 pyrochlore lattice x 256 steps, 16 parts: 26.7 ->
+// 24.4 ms, 11.9 us a stage.
+//
+// What bounds it: the way from one part to the next, 4.4 us of a stage
+// (exports complete, version out, version seen, halo in: four trips to the
+// device's coherence point; 32 and 64 parts, with half and a quarter of the
+// sites, take 6.9 and 5.6 us a stage), then FP64 issue (4.7 us with four
+// waves of 640 VALU instructions per SIMD) and the barriers around the one
+// LDS buffer.
 #include "csl_device.hpp"
 #include "csl_lds.hpp"
+#include "csl_record.hpp"
 
 namespace csl {
 
@@ -79,7 +94,9 @@ __device__ __forceinline__ void part_field(const LatDev& L, const LdsState& Y, i
 
 }  // namespace
 
-template <int SPT, int ZMAX, bool DBUF>
+// AM: a wave's SPT slots of 64 sites follow each other and lie in one
+// sublattice (launch_part_t).
+template <int SPT, int ZMAX, bool DBUF, bool AM>
 __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0, PartArgs A) {
     extern __shared__ double smem[];
     const int T = blockDim.x;
@@ -94,6 +111,7 @@ __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0
     double* drv = smem + 3 * size_t(n_tot);  // [2 parity][3 stage times][2 pulses]
     double* red = drv + 12;                  // [nwaves][10]
     int* ctl = reinterpret_cast<int*>(red + nwaves * 10);  // [0]: a wait gave up
+    double* rot = red + nwaves * 10 + 2;   // AM: [n_atoms][10] frame and staggered sign of a sublattice
 
     // group and part of this workgroup; with xcd_map the P parts of a group
     // sit on one XCD (workgroups are dealt to the 8 XCDs round-robin)
@@ -112,14 +130,15 @@ __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0
     const int NP = L0.NP;
     const int nw = (ZMAX + 1) / 2;
 
-    // own sites: slot q = tid + m*T; sublattice q / cpad (wave-uniform)
+    // own sites: slot q0 + m*qs; sublattice slot / cpad (wave-uniform)
+    const int q0 = AM ? wave * (SPT * kWave) + lane : tid, qs = AM ? kWave : T;
     unsigned nbp[SPT][(ZMAX + 1) / 2];
     int atm[SPT], cnt[SPT];
     unsigned act = 0, expm = 0;
 #pragma unroll
     for (int m = 0; m < SPT; ++m) {
-        const int q = tid + m * T;
-        const int a = uniform((wave * kWave + m * T) / A.cpad);
+        const int q = q0 + m * qs;
+        const int a = uniform((AM ? wave * (SPT * kWave) : wave * kWave + m * T) / A.cpad);
         atm[m] = a;
         cnt[m] = uniform(as_const(L0.cnt_atom)[a]);
         const int c = q - a * A.cpad;
@@ -128,7 +147,7 @@ __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0
 #pragma unroll
         for (int j = 0; j < nw; ++j) nbp[m][j] = A.col[(size_t(part) * nw + j) * A.n_loc + q];
     }
-    auto cell_of = [&](int m) { return part * A.c_per + (tid + m * T - atm[m] * A.cpad); };
+    auto cell_of = [&](int m) { return part * A.c_per + (q0 + m * qs - atm[m] * A.cpad); };
     const int n_halo = A.n_halo[part];
     const int* hsrc = A.halo_src + size_t(part) * A.n_halo_max;
     const int* nbrs = A.nbr + size_t(part) * A.n_nbr_max;
@@ -136,6 +155,15 @@ __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0
     double* exch = A.exch + size_t(grp) * 6 * size_t(NP);
     unsigned v = 0;  // versions this part has published (the same count in every part of the group)
 
+    // where the thread's first halo values come from: read once, a stage's
+    // import then waits for one memory access instead of two
+    constexpr int kHaloRegs = 2;
+    int hreg[kHaloRegs];
+#pragma unroll
+    for (int i = 0; i < kHaloRegs; ++i) hreg[i] = tid + i * T < n_halo ? hsrc[tid + i * T] : 0;
+    if constexpr (AM)
+        for (int i = tid; i < 10 * L0.n_atoms; i += T)
+            rot[i] = i % 10 < 9 ? L0.frames[i / 10 * 9 + i % 10] : L0.afm[i / 10];
     if (tid == 0) ctl[0] = 0;
     __syncthreads();
 
@@ -175,12 +203,21 @@ __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0
     // this XCD's L2 from two stages ago)
     auto import_halo = [&](unsigned want) {
         const double* src = exch + size_t(want & 1u) * 3 * size_t(NP);
-        for (int h = tid; h < n_halo; h += T) {
-            const int d = hsrc[h];
-            const double val[3] = {__hip_atomic_load(src + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                                   __hip_atomic_load(src + NP + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                                   __hip_atomic_load(src + 2 * NP + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
-            Y.store(hb + h, val);
+        auto get = [&](int d, double val[3]) {
+            val[0] = __hip_atomic_load(src + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            val[1] = __hip_atomic_load(src + NP + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            val[2] = __hip_atomic_load(src + 2 * NP + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        double val[kHaloRegs][3];
+#pragma unroll
+        for (int i = 0; i < kHaloRegs; ++i)
+            if (tid + i * T < n_halo) get(hreg[i], val[i]);
+#pragma unroll
+        for (int i = 0; i < kHaloRegs; ++i)
+            if (tid + i * T < n_halo) Y.store(hb + tid + i * T, val[i]);
+        for (int h = tid + kHaloRegs * T; h < n_halo; h += T) {
+            get(hsrc[h], val[0]);
+            Y.store(hb + h, val[0]);
         }
     };
     // the own stage values y of version v+1: LDS, and the exchange buffer
@@ -189,7 +226,7 @@ __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0
     // Exports are agent-scope stores: written through to the device's
     // coherence point, so no release has to write the XCD's L2 back.
     auto put = [&](int m, int buf, const double y[3]) {
-        Y.store(fresh(buf * A.n_loc + tid + m * T), y);
+        Y.store(fresh(buf * A.n_loc + q0 + m * qs), y);
         if ((expm >> m) & 1u) {
             double* dst = exch + size_t((v + 1u) & 1u) * 3 * size_t(NP);
             const int d = fresh(atm[m] * L0.npad + cell_of(m));
@@ -267,6 +304,22 @@ __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0
                 if (lane == kWave - 1) red[wave * 10 + j] = s;
             }
         };
+        // AM: the sums of S and e over the wave's sites, turned into the
+        // sublattice's frame and staggered by record_am
+        auto reduce_am = [&](const double sm[3], double e) { wave_sum4(sm[0], sm[1], sm[2], e, lane, red + wave * 4); };
+        auto record_am = [&](int ri) {
+            if (wave == nwaves - 1 && lane < 10 && (lane < 9 || want_e)) {
+                double s = 0.0;
+                for (int w = 0; w < nwaves; ++w) {
+                    const double* r = red + w * 4;
+                    const double* R = rot + 10 * (w * (SPT * kWave) / A.cpad);
+                    const int d = lane % 3;
+                    const double g = R[3 * d] * r[0] + R[3 * d + 1] * r[1] + R[3 * d + 2] * r[2];
+                    s += lane < 3 ? R[9] * g : (lane < 6 ? r[d] : (lane < 9 ? g : r[3]));
+                }
+                A.part_obs[((size_t(b) * A.n_rec + ri) * A.P + part) * 10 + lane] = s;
+            }
+        };
         // the part's sums of the recorded step ri (after a barrier)
         auto record = [&](int ri) {
             if (wave == 0 && lane < 10 && (lane < 9 || want_e)) {
@@ -317,20 +370,9 @@ __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0
                 else if constexpr (cur == 1) return q + n_loc;
                 else return q < n_loc ? q : q + n_loc;
             };
-            double e[SPT], yn[DBUF ? 1 : SPT][3];
-#pragma unroll
-            for (int m = 0; m < SPT; ++m) {
-                double S[3], H[3];
-                if (s == 0) {
-                    S[0] = x[m][0];
-                    S[1] = x[m][1];
-                    S[2] = x[m][2];
-                } else {
-                    Y.load(fresh(cur * n_loc + tid + m * T), S);
-                }
-                part_field<ZMAX>(L, Y, atm[m], cnt[m], nbp[m], slot, S, H);
-                e[m] = (obs && want_e) ? site_energy(L, atm[m], 0, S, H) : 0.0;
-                if (drive_now) sub_drive(L, atm[m], f1, f2, H);
+            double yn[DBUF ? 1 : SPT][3];
+            // stage values of slot m from its field (drive included)
+            auto advance = [&](int m, const double S[3], const double H[3]) {
                 double k[3];
                 ll_su2_guarded(H, S, alpha, k);
                 double* y = yn[DBUF ? 0 : m];
@@ -342,6 +384,80 @@ __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0
                     y[d] = (s < 3) ? x[m][d] + cdt * k[d] : x[m][d];
                 }
                 if (DBUF) put(m, nxt, y);
+            };
+            if constexpr (AM) {
+                const int atom = atm[0];
+                cptr<double> B = as_const(L.field) + atom * 3;
+                double h0[3] = {-B[0], -B[1], -B[2]}, hb0[3] = {-B[0], -B[1], -B[2]};
+                if (drive_now) {
+                    cptr<double> d0 = as_const(L.fdrive) + atom * 3;
+                    cptr<double> d1 = as_const(L.fdrive) + (L.n_atoms + atom) * 3;
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        const double D = d0[d] * f1 + d1[d] * f2;
+                        h0[d] -= D;
+                        hb0[d] += D;
+                    }
+                }
+                double H[SPT][3];
+#pragma unroll
+                for (int m = 0; m < SPT; ++m)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) H[m][d] = h0[d];
+#pragma unroll
+                for (int k = 0; k < ZMAX; ++k) {
+                    cptr<double> J = as_const(L.mats) + (atom * ZMAX + k) * 9 + opaque_zero();
+#pragma unroll
+                    for (int m = 0; m < SPT; ++m) {
+                        const int q = int((unsigned(fresh(int(nbp[m][k >> 1]))) >> (16 * (k & 1))) & 0xffffu);
+                        double Sp[3];
+                        Y.load(slot(q), Sp);
+                        add_bond_fused(J, Sp, H[m]);
+                        hold(H[m]);
+                    }
+                }
+                double sm[3] = {0.0, 0.0, 0.0}, e = 0.0;
+#pragma unroll
+                for (int m = 0; m < SPT; ++m) {
+                    double S[3];
+                    if (s == 0) {
+#pragma unroll
+                        for (int d = 0; d < 3; ++d) S[d] = x[m][d];
+                        if (obs) {
+#pragma unroll
+                            for (int d = 0; d < 3; ++d) {
+                                sm[d] += S[d];
+                                e = fma(S[d], 0.5 * (H[m][d] + hb0[d]), e);
+                            }
+                        }
+                    } else {
+                        Y.load(fresh(cur * n_loc + q0 + m * qs), S);
+                    }
+                    advance(m, S, H[m]);
+                }
+                if (obs) reduce_am(sm, e);
+                if (!DBUF) __syncthreads();
+                publish(DBUF ? nullptr : yn);
+                // red[] is complete since publish's barrier and not written
+                // again before the next step's barriers
+                if (obs) record_am(ri);
+                return true;
+            }
+            double e[SPT];
+#pragma unroll
+            for (int m = 0; m < SPT; ++m) {
+                double S[3], H[3];
+                if (s == 0) {
+                    S[0] = x[m][0];
+                    S[1] = x[m][1];
+                    S[2] = x[m][2];
+                } else {
+                    Y.load(fresh(cur * n_loc + q0 + m * qs), S);
+                }
+                part_field<ZMAX>(L, Y, atm[m], cnt[m], nbp[m], slot, S, H);
+                e[m] = (obs && want_e) ? site_energy(L, atm[m], 0, S, H) : 0.0;
+                if (drive_now) sub_drive(L, atm[m], f1, f2, H);
+                advance(m, S, H);
             }
             // stage 0: x still holds the state at t_n (the record's state)
             if (obs) reduce_obs(L, e);
@@ -378,10 +494,22 @@ __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0
                                  x[m], H);
                 e[m] = want_e ? site_energy(L, atm[m], 0, x[m], H) : 0.0;
             }
-            reduce_obs(L, e);
+            if constexpr (AM) {
+                double sm[3] = {0.0, 0.0, 0.0}, es = 0.0;
+#pragma unroll
+                for (int m = 0; m < SPT; ++m) {
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) sm[d] += x[m][d];
+                    es += e[m];
+                }
+                reduce_am(sm, es);
+            } else {
+                reduce_obs(L, e);
+            }
         }
         __syncthreads();
-        record(A.n_rec - 1);
+        if constexpr (AM) record_am(A.n_rec - 1);
+        else record(A.n_rec - 1);
         if (A.final_states) {
             double* out = A.final_states + size_t(b) * L0.N * 3;
 #pragma unroll
@@ -418,15 +546,29 @@ __global__ void __launch_bounds__(256) k_part_reduce(const double* __restrict__ 
 
 namespace {
 
-template <int SPT, int ZMAX, bool DBUF>
-hipError_t launch_part_t(const LatDev& L, const PartArgs& A, int block, size_t lds, hipStream_t st, int* occ) {
-    auto kern = k_partitioned<SPT, ZMAX, DBUF>;
+template <int SPT, int ZMAX, bool DBUF, bool AM>
+hipError_t launch_part_am(const LatDev& L, const PartArgs& A, int block, size_t lds, hipStream_t st, int* occ) {
+    auto kern = k_partitioned<SPT, ZMAX, DBUF, AM>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
     if (occ) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, kern, block, lds);
     hipLaunchKernelGGL(kern, dim3(unsigned(A.groups * A.P)), dim3(block), lds, st, L, A);
     return hipGetLastError();
+}
+
+// Whole waves in one sublattice (the bond matrices are then read once for
+// the wave's SPT sites a lane, not once a site), on lattices whose field is
+// per sublattice without an onsite matrix and whose sites all have ZMAX
+// bonds, where the sublattices' frames fit beside the state in LDS.
+template <int SPT, int ZMAX, bool DBUF>
+hipError_t launch_part_t(const LatDev& L, const PartArgs& A, int block, size_t lds, hipStream_t st, int* occ) {
+    if constexpr (ZMAX <= 6) {
+        const size_t lds_am = lds + 10 * sizeof(double) * size_t(L.n_atoms);
+        if (A.cpad % (SPT * kWave) == 0 && L.zmax == ZMAX && L.full_coord && !L.has_onsite && lds_am <= kLdsBytes)
+            return launch_part_am<SPT, ZMAX, DBUF, true>(L, A, block, lds_am, st, occ);
+    }
+    return launch_part_am<SPT, ZMAX, DBUF, false>(L, A, block, lds, st, occ);
 }
 
 template <int SPT, bool DBUF>
