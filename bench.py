@@ -220,7 +220,7 @@ def bench_2dcs(args):
 
     site_steps = B * N * N_STEPS
     flops_launch = site_steps * (FLOPS_Z3 + FLOPS_DRIVE)
-    roof = fp64_roofline("k_persistent", flops_launch, kms,
+    roof = fp64_roofline("k_trajectory", flops_launch, kms,
                          algorithmic_flops_per_site_step=FLOPS_Z3 + FLOPS_DRIVE,
                          hbm_algorithmic_frac=site_steps * BYTES_PER_SITE_STEP / (kms * 1e-3) / HBM_PEAK)
     roof["traffic"] = profile_number("traffic_k_persistent_2dcs_36x36.txt", "traffic_bytes_per_launch")
@@ -593,7 +593,7 @@ def bench_adjoint(args):
                    "sites": N, "starts": ADJ_B, "rk4_steps": ADJ_STEPS, "parameters": 5, "alpha": 0.02},
         "kernel_ms": kms,
         "max_rel_err_vs_oracle_tangent_linear": err,
-        "roofline": fp64_roofline("k_adj_fwd + k_adj_bwd + k_adj_par", ADJ_B * N * ADJ_STEPS * ADJ_FLOPS_PER_SITE_STEP,
+        "roofline": fp64_roofline("k_adj_fwd + k_adj_sweep", ADJ_B * N * ADJ_STEPS * ADJ_FLOPS_PER_SITE_STEP,
                                   kms, algorithmic_flops_per_site_step=ADJ_FLOPS_PER_SITE_STEP,
                                   note=f"forward and backward sweeps: one workgroup per start ({ADJ_B} of the 256 CUs); "
                                        "parameter terms on the other CUs, overlapped with the sweep"),
