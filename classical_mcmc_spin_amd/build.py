@@ -19,12 +19,13 @@ ROOT = os.path.dirname(HERE)
 LIB_NAME = "libcsl_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 
-# (source, object suffix, extra flags)
-HIP_UNITS = [("csl_kernels.hip", "", []), ("csl_capi.hip", "", []), ("csl_mixed.hip", "", []), ("csl_adjoint.hip", "", []), ("csl_adjoint_sweep.hip", "", []),
-             ("csl_dssf.hip", "", []), ("csl_spectrum.hip", "", []), ("csl_quench.hip", "", []),
-             ("csl_dopri5.hip", "", []), ("csl_partition.hip", "", []), ("csl_mixed_persist.hip", "", []),
-             ("csl_mixed_waves.hip", "", [])] + [
-    (src, f"_spt{n}", [f"-DCSL_SPT={n}"]) for src in ("csl_persistent.hip", "csl_trajectory.hip") for n in (1, 2, 3, 4, 6)]
+# (source, object suffix, extra flags); the units that compile longest first
+HIP_UNITS = [(src, f"_spt{n}", [f"-DCSL_SPT={n}"])
+             for src in ("csl_persistent.hip", "csl_trajectory.hip") for n in (6, 4, 3, 2, 1)]
+HIP_UNITS = HIP_UNITS[:5] + [("csl_dopri5.hip", "", []), ("csl_partition.hip", "", [])] + HIP_UNITS[5:] + [
+    ("csl_kernels.hip", "", []), ("csl_capi.hip", "", []), ("csl_mixed.hip", "", []), ("csl_adjoint.hip", "", []),
+    ("csl_adjoint_sweep.hip", "", []), ("csl_dssf.hip", "", []), ("csl_spectrum.hip", "", []),
+    ("csl_quench.hip", "", []), ("csl_mixed_persist.hip", "", []), ("csl_mixed_waves.hip", "", [])]
 CXX_UNITS = ["gpu_api_shim.cpp", "mixed_gpu_api_shim.cpp"]
 
 HIPCC_FLAGS = [
