@@ -27,6 +27,7 @@
 #include "csl_internal.hpp"
 #include "csl_kernels.hpp"
 #include "csl_mixed_lds.hpp"
+#include "csl_mixed_pack.hpp"
 #include "csl_tableau.hpp"
 
 namespace csl {
@@ -2198,18 +2199,14 @@ int csl_mixed_create(size_t A2, size_t A3, size_t n_cells, const double* field2,
                     pk.resize((pk.size() + 255) / 256 * 256);
                     return at;
                 };
-                auto partners = [&](const EllHost& e, int NP, int Z, int npart) {
-                    std::vector<unsigned short> q(size_t(NP) * Z);
-                    for (int p = 0; p < NP; ++p)
-                        for (int k = 0; k < Z; ++k)
-                            q[size_t(p) * Z + k] = static_cast<unsigned short>(
-                                k < e.cnt[p] ? e.col[size_t(k) * NP + p] : std::min(p, npart - 1));
+                auto partners = [&](const EllHost& e, int NP, int Z) {
+                    const auto q = cslh::packed_partners(e.col.data(), e.cnt.data(), NP, Z, npad);
                     return put(q.data(), q.size() * sizeof(unsigned short));
                 };
-                const size_t o22 = partners(e22, M.NP2, csl::kMixZ22, M.NP2);
-                const size_t o23 = partners(e23, M.NP2, csl::kMixZ23, M.NP3);
-                const size_t o32 = partners(e32, M.NP3, csl::kMixZ32, M.NP2);
-                const size_t o33 = partners(e33, M.NP3, csl::kMixZ33, M.NP3);
+                const size_t o22 = partners(e22, M.NP2, csl::kMixZ22);
+                const size_t o23 = partners(e23, M.NP2, csl::kMixZ23);
+                const size_t o32 = partners(e32, M.NP3, csl::kMixZ32);
+                const size_t o33 = partners(e33, M.NP3, csl::kMixZ33);
                 const size_t oj = put(P.mats.data(), P.mats.size() * sizeof(double));
                 const size_t oo = put(P.off32.data(), P.off32.size() * sizeof(int));
                 h->ppack.upload(pk.data(), pk.size(), s);

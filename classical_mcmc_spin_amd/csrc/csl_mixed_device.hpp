@@ -39,8 +39,8 @@ struct MixDev {
     double gamma[8];
     int has_bloch;
     // partner indices of the persistent kernels, 16 bits each, one load per
-    // site and bond kind ([NP2] kinds 22 and 23, [NP3] kinds 32 and 33); a
-    // padding slot's partners are itself.  Null when a table does not fit.
+    // site and bond kind ([NP2] kinds 22 and 23, [NP3] kinds 32 and 33; unused
+    // slots: csl_mixed_pack.hpp).  Null when a table does not fit.
     const uint4* __restrict__ q22;
     const uint4* __restrict__ q23;
     const uint4* __restrict__ q32;

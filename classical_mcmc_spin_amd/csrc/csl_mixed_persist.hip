@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
         if (P.wait >= 0) mix_wait_seam(K.A, P.wait, tid);
         __syncthreads();  // the previous piece is done with LDS and G
         // initial state: the stage values of stage 0; padding lanes hold
-        // zeros and gather themselves, so their derivative is zero
+        // zeros and gather padding, so their derivative is zero
 #pragma unroll
         for (int j = 0; j < SPT; ++j) {
             const int p = p0 + j * kWave;

@@ -202,7 +202,7 @@ __device__ __forceinline__ void run_unit(const MixKernArgs& K, double* smem, con
         const bool drive = K.A.tp != nullptr;
         if (P.wait >= 0) mix_wait_seam(K.A, P.wait, tid);
         __syncthreads();  // the previous piece is done with the LDS
-        // padding lanes hold zeros and gather themselves: their derivative is zero
+        // padding lanes hold zeros and gather padding: their derivative is zero
         double x[D], acc[D], y[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) x[d] = real ? X[size_t(d) * NP + p] : 0.0;

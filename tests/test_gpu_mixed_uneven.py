@@ -1,0 +1,69 @@
+"""Mixed lattices whose species have different numbers of sublattices: the
+packed partner tables of the tangent run (their unused slots on the host:
+test_mixed_pack.py).
+
+Tolerances: runs against the oracle as in test_gpu_mixed_shapes.py (some 100
+roundings a step and component, 1e-12 for up to 9 steps of unit vectors); the
+tangent records against central differences of the oracle's runs at scales
+1 +- 1e-5 (truncation 1e-10, rounding 1e-16 / 1e-5 a record) to 1e-6 of their
+largest, as in test_gpu_mixed_grad.py.
+"""
+import numpy as np
+import pytest
+
+from classical_mcmc_spin_amd import gpu_mixed as GM
+from classical_mcmc_spin_amd import mixed_model as mm
+from classical_mcmc_spin_amd import seeding
+from classical_mcmc_spin_amd.model import UnitCell
+
+pytestmark = pytest.mark.gpu
+
+DT = 0.005
+
+
+def uneven_cell(A2, A3, tt=False, seed=7):
+    """A2 SU(2) and A3 SU(3) sublattices, fields and onsite terms of both;
+    four SU(2) bonds a sublattice, two mixed bonds a SU(2) sublattice, and with
+    tt SU(3)-SU(3) bonds of the first sublattice."""
+    g = np.random.default_rng(seed)
+    fe, tm = UnitCell(3, A2), UnitCell(8, A3)
+    sym = lambda n, s: (lambda m: s * (m + m.T))(g.normal(size=(n, n)))
+    for a in range(A2):
+        fe.set_field(0.2 * g.normal(size=3), a)
+        fe.set_onsite_interaction(sym(3, 0.05), a)
+        for o in ((0, 0, 0), (0, 0, 1)):
+            fe.set_bilinear_interaction(0.3 * g.normal(size=(3, 3)), a, (a + 1) % A2, o)
+    fe.set_afm_sublattice_signs(np.where(np.arange(A2) % 2, -1.0, 1.0))
+    for a in range(A3):
+        tm.set_field(0.3 * g.normal(size=8), a)
+        tm.set_onsite_interaction(sym(8, 0.05), a)
+    if tt:
+        tm.set_bilinear_interaction(0.1 * g.normal(size=(8, 8)), 0, A3 - 1, (0, 0, 1))
+    muc = mm.MixedUnitCell(fe, tm)
+    for a in range(A2):
+        for o in ((0, 0, 0), (0, 1, 0)):
+            muc.set_mixed_bilinear(0.2 * g.normal(size=(3, 8)), a, a % A3, o)
+    return muc
+
+
+@pytest.mark.parametrize("A2,A3,dims,tt", [(4, 2, (3, 2, 2), False), (2, 3, (5, 3, 5), True), (6, 1, (1, 5, 2), False)])
+def test_tangent_with_uneven_sublattices(oracle, A2, A3, dims, tt):
+    muc = uneven_cell(A2, A3, tt)
+    ml = mm.MixedLattice(muc, *dims)
+    init = ml.flat_state(seeding.random_spins(ml.N2, 3), mm.random_su3_states(ml.N3, 4))
+    n = 12
+    T1 = (n + 0.5) * DT
+    w = np.r_[np.ones(33), 0.0]
+    run = lambda s: oracle.MixedOracle(mm.scale_fe_tm(muc, s), *dims).integrate_md(init, 0.0, T1, DT)["records"]
+    ref = run(1.0)
+    h = 1e-5
+    fd = (run(1.0 + h) - run(1.0 - h)) / (2.0 * h)
+    target = ref + 0.01
+    with GM.GPUMixedLattice(ml) as gm:
+        g = gm.scale_gradient(init, [[0.0, 0.0]], target, w, None, 0.0, T1, DT, want_records=True)
+    assert np.max(np.abs(g["records"][:, 0] - ref)) <= 1e-12
+    tr = g["trecords"][:, 0]
+    assert np.max(np.abs(tr[:, :33] - fd[:, :33])) <= 1e-6 * np.max(np.abs(fd[:, :33]))
+    grad = 2.0 * np.sum(w * (ref - target) * tr)
+    # 33 n products of records within 1e-12 and these tangents, summed in another order
+    assert abs(g["grad"][0] - grad) <= 1e-10 * np.sum(np.abs(w * (ref - target) * tr))
