@@ -25,6 +25,7 @@
 #include "../../include/csl_gpu.h"
 #include "csl_host.hpp"
 #include "csl_kernels.hpp"
+#include "csl_plan_pair.hpp"
 #include "csl_tableau.hpp"
 
 // Scratch of csl_integrate_batched_noalloc: one region per GPU, in the code
@@ -74,17 +75,12 @@ struct PartPlan {
     DBuf<int> halo_src, n_halo, nbr;
 };
 
-// Buffers and transform plans of the structure factor.
+// Buffers and transform plans (a: the 3-D one, b: along time) of the
+// structure factor.
+inline void drop_fft_plan(hipfftHandle p) { (void)hipfftDestroy(p); }
 struct DqWork {
     DBuf<double> pos, cin, cf, sqt, phase, out, samples;
-    hipfftHandle p3 = 0, p1 = 0;
-    std::array<size_t, 6> key{};
-    void drop_plans() {
-        if (p3) (void)hipfftDestroy(p3);
-        if (p1) (void)hipfftDestroy(p1);
-        p3 = p1 = 0;
-    }
-    ~DqWork() { drop_plans(); }
+    cslh::PlanPair<hipfftHandle, std::array<size_t, 6>, drop_fft_plan> plans;
 };
 
 struct csl_lattice {
@@ -149,7 +145,7 @@ struct csl_lattice {
     hipGraphExec_t graph_exec = nullptr;
     std::vector<unsigned char> graph_key;
     ~csl_lattice() {
-        dq.drop_plans();  // before their stream
+        dq.plans.drop();  // before their stream
         if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
         if (stream2) (void)hipStreamDestroy(stream2);
         if (stream) (void)hipStreamDestroy(stream);
@@ -2671,23 +2667,20 @@ int csl_structure_factor(csl_lattice* h, size_t B, const double* init, int init_
         };
         // plans kept on the handle while the shapes stay (making them takes
         // longer than a small run)
-        const std::array<size_t, 6> key{L1, L2, L3, nc * per, n_t, R};
-        if (!w.p3 || w.key != key) {
-            w.drop_plans();
+        w.plans.use({L1, L2, L3, nc * per, n_t, R}, [&](hipfftHandle& p3, hipfftHandle& p1) {
             size_t ws = 0;
             int dims3[3] = {int(L1), int(L2), int(L3)};
-            fft_check(hipfftCreate(&w.p3), "hipfftCreate");
-            fft_check(hipfftMakePlanMany(w.p3, 3, dims3, nullptr, 1, int(Q), nullptr, 1, int(Q), HIPFFT_Z2Z,
+            fft_check(hipfftCreate(&p3), "hipfftCreate");
+            fft_check(hipfftMakePlanMany(p3, 3, dims3, nullptr, 1, int(Q), nullptr, 1, int(Q), HIPFFT_Z2Z,
                                          int(nc * per), &ws),
                       "3-D plan");
-            fft_check(hipfftSetStream(w.p3, s), "hipfftSetStream");
+            fft_check(hipfftSetStream(p3, s), "hipfftSetStream");
             int dims1[1] = {int(n_t)};
-            fft_check(hipfftCreate(&w.p1), "hipfftCreate");
-            fft_check(hipfftMakePlanMany(w.p1, 1, dims1, dims1, int(R), 1, dims1, int(R), 1, HIPFFT_Z2Z, int(R), &ws),
+            fft_check(hipfftCreate(&p1), "hipfftCreate");
+            fft_check(hipfftMakePlanMany(p1, 1, dims1, dims1, int(R), 1, dims1, int(R), 1, HIPFFT_Z2Z, int(R), &ws),
                       "time plan");
-            fft_check(hipfftSetStream(w.p1, s), "hipfftSetStream");
-            w.key = key;
-        }
+            fft_check(hipfftSetStream(p1, s), "hipfftSetStream");
+        });
         auto* cin2 = reinterpret_cast<double2*>(w.cin.p);
         auto* cf2 = reinterpret_cast<double2*>(w.cf.p);
         auto* sqt2 = reinterpret_cast<double2*>(w.sqt.p);
@@ -2695,7 +2688,7 @@ int csl_structure_factor(csl_lattice* h, size_t B, const double* init, int init_
         hip_check(csl::launch_sq_phase(int(h->n_atoms), int(L1), int(L2), int(L3), w.pos.p, ph2, s), "k_sq_phase");
         // grids in cin -> S(q, t) of nc samples from ti on
         auto transform = [&](size_t ti) {
-            fft_check(hipfftExecZ2Z(w.p3, reinterpret_cast<hipfftDoubleComplex*>(cin2),
+            fft_check(hipfftExecZ2Z(w.plans.a, reinterpret_cast<hipfftDoubleComplex*>(cin2),
                                     reinterpret_cast<hipfftDoubleComplex*>(cf2), HIPFFT_FORWARD),
                       "3-D FFT");
             hip_check(csl::launch_sq_combine(cf2, nc * B, int(h->n_atoms), Q, ph2, sqt2 + ti * R, s), "k_sq_combine");
@@ -2721,7 +2714,7 @@ int csl_structure_factor(csl_lattice* h, size_t B, const double* init, int init_
             };
             run_stages(h, B, h->bt_tp.p, h->bt_amp.p, false, grid, dt, 1, false, nullptr, sample);
         }
-        fft_check(hipfftExecZ2Z(w.p1, reinterpret_cast<hipfftDoubleComplex*>(sqt2),
+        fft_check(hipfftExecZ2Z(w.plans.b, reinterpret_cast<hipfftDoubleComplex*>(sqt2),
                                 reinterpret_cast<hipfftDoubleComplex*>(sqt2), HIPFFT_FORWARD),
                   "time FFT");
         hip_check(csl::launch_sq_power(sqt2, int(n_t), int(B), Q, 1.0 / (double(B) * double(h->N) * double(n_t)), w.out.p, s),
