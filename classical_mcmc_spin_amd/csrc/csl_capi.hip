@@ -23,6 +23,7 @@
 #include <hipfft/hipfft.h>
 
 #include "../../include/csl_gpu.h"
+#include "csl_dssf_route.hpp"
 #include "csl_host.hpp"
 #include "csl_kernels.hpp"
 #include "csl_plan_pair.hpp"
@@ -81,7 +82,21 @@ inline void drop_fft_plan(hipfftHandle p) { (void)hipfftDestroy(p); }
 struct DqWork {
     DBuf<double> pos, cin, cf, sqt, phase, out, samples;
     cslh::PlanPair<hipfftHandle, std::array<size_t, 6>, drop_fft_plan> plans;
+    size_t work = 0;   // bytes of the plans' work areas
+    size_t bytes() const {
+        return work + sizeof(double) * (pos.n + cin.n + cf.n + sqt.n + phase.n + out.n + samples.n);
+    }
+    void release() {
+        for (DBuf<double>* d : {&pos, &cin, &cf, &sqt, &phase, &out, &samples}) d->release();
+        plans.drop();
+        work = 0;
+    }
 };
+// What a structure-factor call leaves on its handle for the next one (3 % of
+// the card); a call that needs more gives everything back, and pays 19 ms for
+// making it again: 24x24, 64 trajectories x 800 samples (3.3 GB) take 11.8 ms
+// with it kept and 30.6 without, 16 x 200 (0.6 GB) 1.3 and 10.
+constexpr size_t kDqKept = size_t(8) << 30;
 
 struct csl_lattice {
     int device = 0;
@@ -2647,15 +2662,23 @@ int csl_structure_factor(csl_lattice* h, size_t B, const double* init, int init_
         const size_t per = B * h->n_atoms * 3;   // grids of one sample
         const size_t R = B * 3 * Q;
         // a lattice of one workgroup: the persistent kernel leaves the
-        // samples behind (when they take at most a quarter of the free
-        // memory), and their grids are transformed many samples at a time
+        // samples behind, and their grids are transformed many at a time
+        DqWork& w = h->dq;
+        struct Keep {
+            DqWork& w;
+            bool done = false;
+            ~Keep() {
+                if (!done || w.bytes() > kDqKept) w.release();
+            }
+        } keep{w};
         size_t free_b = 0, total_b = 0;
         hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-        const bool persistent = !persistent_candidates(h).empty() && n_t * per * Q * sizeof(double) <= free_b / 4 &&
-                                n_steps <= size_t(std::numeric_limits<int>::max());
-        // samples per transform: grids of at most 256 MB
-        const size_t nc = persistent ? std::max<size_t>(1, std::min(n_t, (size_t(256) << 20) / (per * Q * 16))) : 1;
-        DqWork& w = h->dq;
+        const bool one_workgroup =
+            !persistent_candidates(h).empty() && n_steps <= size_t(std::numeric_limits<int>::max());
+        const cslh::DssfRoute route = cslh::dssf_route(one_workgroup, n_t, per * Q, R, free_b, w.bytes());
+        const bool persistent = route.persistent;
+        const size_t nc = route.nc;
+        if (!persistent) w.samples.release();
         w.pos.upload(positions, h->n_atoms * 3, s);
         w.cin.ensure(2 * nc * per * Q);
         w.cf.ensure(2 * nc * per * Q);
@@ -2667,18 +2690,22 @@ int csl_structure_factor(csl_lattice* h, size_t B, const double* init, int init_
         };
         // plans kept on the handle while the shapes stay (making them takes
         // longer than a small run)
-        w.plans.use({L1, L2, L3, nc * per, n_t, R}, [&](hipfftHandle& p3, hipfftHandle& p1) {
+        const size_t nfft = nc * per;
+        w.plans.use({L1, L2, L3, nfft, n_t, R}, [&](hipfftHandle& p3, hipfftHandle& p1) {
             size_t ws = 0;
+            w.work = 0;
             int dims3[3] = {int(L1), int(L2), int(L3)};
             fft_check(hipfftCreate(&p3), "hipfftCreate");
             fft_check(hipfftMakePlanMany(p3, 3, dims3, nullptr, 1, int(Q), nullptr, 1, int(Q), HIPFFT_Z2Z,
-                                         int(nc * per), &ws),
+                                         int(nfft), &ws),
                       "3-D plan");
+            w.work += ws;
             fft_check(hipfftSetStream(p3, s), "hipfftSetStream");
             int dims1[1] = {int(n_t)};
             fft_check(hipfftCreate(&p1), "hipfftCreate");
             fft_check(hipfftMakePlanMany(p1, 1, dims1, dims1, int(R), 1, dims1, int(R), 1, HIPFFT_Z2Z, int(R), &ws),
                       "time plan");
+            w.work += ws;
             fft_check(hipfftSetStream(p1, s), "hipfftSetStream");
         });
         auto* cin2 = reinterpret_cast<double2*>(w.cin.p);
@@ -2722,6 +2749,7 @@ int csl_structure_factor(csl_lattice* h, size_t B, const double* init, int init_
         copy_back(sqw, w.out.p, Q * n_t, s);
         copy_back(mags, h->rec_mags.p, (n_steps + 1) * B * 9, s);
         hip_check(hipStreamSynchronize(s), "structure factor");
+        keep.done = true;
     });
 }
 

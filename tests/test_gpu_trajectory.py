@@ -126,3 +126,33 @@ def test_structure_factor_samples(dims, steps, every, onsite):
     assert np.max(np.abs(r["sqw"] - ref)) <= 1e-12 * np.max(ref)
     m = S.mean(2)
     assert np.max(np.abs(r["mags"][:-1:every][:n_t, :, 1] - m)) <= 1e-13
+
+
+@pytest.mark.parametrize("B,n_t,kept", [(4, 30, True), (128, 1200, False)])
+def test_structure_factor_buffers(B, n_t, kept):
+    """A call repeated on its handle gives the same bits, also with a call of
+    another shape between; buffers of up to 8 GB stay on the handle, larger
+    ones (samples and S(q, t) 4.2 GB each here) are given back."""
+    import torch
+    lat = model.Lattice(_kitaev(), 24, 24, 1)
+    init = np.stack([random_state(lat, b) for b in range(B)])
+    pos = np.array([[0.0, 0.0, 0.0], [0.1, 0.55, 0.0]])
+
+    def used():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return total - free
+
+    with GPULattice(lat) as gl:
+        run = lambda n: gl.structure_factor(init, 0.0, (n + 0.5) * DT, DT, 1, (24, 24, 1), pos)["sqw"]
+        gl.integrate_batched(init, np.zeros((B, 2)), np.zeros((B, 2)), 0.0, (n_t + 0.5) * DT, DT, tgrid="boost")
+        before = used()
+        first = run(n_t)
+        held = used() - before
+        print(f"[dssf buffers] B {B} samples {n_t}: {held / 2**20:.0f} MB stay", flush=True)
+        samples = 8 * n_t * B * lat.lattice_size * 3
+        assert (held >= samples) if kept else (held < 64 << 20)
+        second = run(n_t)
+        run(n_t // 2)
+        third = run(n_t)
+    assert np.array_equal(first, second) and np.array_equal(first, third)
