@@ -305,9 +305,10 @@ class GPULattice:
         fi = f64(field_in).reshape(self.A, 3)
         n_tau_max = int(abs((tau_end - tau_start) / tau_step)) + 2
         ns, _ = self.count_records(T0, T1, T_step, 1, "boost")
-        # the observer gate drops the start sample, so an RK4 run has ns
-        # records and its rows need no padding
-        max_rec = max(ns, 1) if method == "rk4" else ns + 1
+        # the observer gate (_gate) drops the start sample of all but the
+        # finest grids, so an RK4 run's rows need no padding
+        start = len(_gate([T0], T0, T1, T_step))
+        max_rec = max(ns + start, 1) if method == "rk4" else ns + 1
         times = np.empty(max_rec)
         M0 = np.empty(max_rec * 9)
         M1 = np.empty(n_tau_max * max_rec * 9)

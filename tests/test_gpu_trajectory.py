@@ -96,6 +96,20 @@ def test_pump_probe_rows(n_tau, steps):
     assert np.array_equal(r["M01"], np.swapaxes(m[:, 1 + n_tau:], 0, 1))
 
 
+@pytest.mark.parametrize("step,steps,kept", [(1e-10, 4, 5), (1.0000001e-10, 4, 4), (2.5e-11, 7, 8)])
+def test_pump_probe_keeps_the_start_of_fine_grids(step, steps, kept):
+    """The observer gate passes a sample less than 1e-10 short of a step after
+    the last one: the start sample too where the step is that fine."""
+    lat = model.Lattice(_kitaev(), 3, 2, 1)
+    f = np.zeros((2, 3))
+    f[:, 0] = 1.0
+    with GPULattice(lat) as gl:
+        r = gl.pump_probe(random_state(lat, 3), f, 0.5, 0.1, 0.0, 0.0, 0.02, 0.02, 0.0, (steps + 0.5) * step, step)
+    assert r["M0"].shape == (kept, 3, 3) and r["M1"].shape[:2] == r["M01"].shape[:2] == (2, kept)
+    t = step * np.arange(steps + 1)
+    assert np.array_equal(r["times"], t[steps + 1 - kept:])
+
+
 @pytest.mark.parametrize("dims,steps,every", [((5, 3, 1), 19, 1), ((13, 5, 1), 24, 8), ((4, 6, 1), 37, 5)])
 @pytest.mark.parametrize("onsite", [0.0, 0.1])
 def test_structure_factor_samples(dims, steps, every, onsite):
