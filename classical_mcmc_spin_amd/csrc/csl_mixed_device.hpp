@@ -142,8 +142,6 @@ struct MixPersistShape {
     bool waves;  // one unit of 64 sites of one species per wave (csl_mixed_waves.hip)
 };
 MixPersistShape mixed_persist_shape(const MixDev& M, bool tt);
-// glds: SU(3) components 6, 7 of the stage values in LDS too
-size_t mixed_persist_lds_bytes(const MixDev& M, int block, bool glds);
 // The one-unit-per-wave kernel: its LDS, and the launcher (arguments as
 // launch_mixed_persist).
 size_t mixed_waves_lds_bytes(const MixDev& M);

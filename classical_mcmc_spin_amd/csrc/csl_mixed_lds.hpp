@@ -72,18 +72,28 @@ struct MixTables {
     int rows;      // 3 A2 + 8 A3
 };
 
-// cst and the undriven rows (B of the SU(2) sublattices first)
+// B, d0, d1 of field component i (the SU(2) sublattices' first).
+struct MixRow {
+    double B, d0, d1;
+};
+__device__ __forceinline__ MixRow mix_row(cptr<MixDev> M, int i) {
+    const int n2 = 3 * M->A2, n3 = 8 * M->A3;
+    const bool f = i < n2;
+    const int j = f ? i : i - n2;
+    return {f ? M->field2[j] : M->field3[j], f ? M->fdrive2[j] : M->fdrive3[j],
+            f ? M->fdrive2[n2 + j] : M->fdrive3[n3 + j]};
+}
+
+// cst and the undriven rows
 __device__ __forceinline__ void mix_fill_tables(cptr<MixDev> M, const MixTables& Q, int tid, int T) {
-    const int n2 = 3 * M->A2, n3 = 8 * M->A3, R = Q.rows;
+    const int R = Q.rows;
     for (int i = tid; i < R; i += T) {
-        const bool f = i < n2;
-        const int j = f ? i : i - n2;
-        const double B = f ? M->field2[j] : M->field3[j];
-        Q.cst[3 * i] = B;
-        Q.cst[3 * i + 1] = f ? M->fdrive2[j] : M->fdrive3[j];
-        Q.cst[3 * i + 2] = f ? M->fdrive2[n2 + j] : M->fdrive3[n3 + j];
+        const MixRow r = mix_row(M, i);
+        Q.cst[3 * i] = r.B;
+        Q.cst[3 * i + 1] = r.d0;
+        Q.cst[3 * i + 2] = r.d1;
         for (int par = 0; par < 2; ++par)  // without a drive the rows stay -B (and -B + 2B)
-            for (int st = 0; st < 4; ++st) Q.hin[(par * 4 + st) * R + i] = st < 3 ? -B : B;
+            for (int st = 0; st < 4; ++st) Q.hin[(par * 4 + st) * R + i] = st < 3 ? -r.B : r.B;
     }
 }
 
@@ -115,6 +125,19 @@ __device__ __forceinline__ void mix_write_hin(const MixTables& Q, const double* 
         const int st = i / R, r = i - st * R, q = st == 3 ? 0 : st, s3 = r < n2 ? 0 : 2;
         const double D = Q.cst[3 * r + 1] * f[q * 4 + s3] + Q.cst[3 * r + 2] * f[q * 4 + s3 + 1];
         Q.hin[par * 4 * R + i] = st == 3 ? Q.cst[3 * r] - D : -Q.cst[3 * r] - D;
+    }
+}
+
+// One row st of the one set of rows of the tight layout (csl_mixed_lay.hpp):
+// -(B + drive) at the st-th stage time, st 3 the first plus 2B; f null: no drive.
+__device__ __forceinline__ void mix_write_row(cptr<MixDev> M, const MixTables& Q, const double* f, int st, int n2, int tid,
+                                              int T) {
+    const int q = st == 3 ? 0 : st;
+    for (int i = tid; i < Q.rows; i += T) {
+        const MixRow r = mix_row(M, i);
+        const int s3 = i < n2 ? 0 : 2;
+        const double D = f ? r.d0 * f[q * 4 + s3] + r.d1 * f[q * 4 + s3 + 1] : 0.0;
+        Q.hin[st * Q.rows + i] = st == 3 ? r.B - D : -r.B - D;
     }
 }
 

@@ -28,7 +28,8 @@
 //
 // Field rows, pulse envelopes and records are handled as in
 // csl_trajectory.hip: rows of -(B + drive) from LDS, envelopes of two steps
-// at a time, records from the waves' sums of S and S.H, two at a time.  With
+// at a time, records from the waves' sums of S and S.H, two at a time; lattices
+// with many sublattices keep smaller tables (TIGHT, csl_mixed_lay.hpp).  With
 // every record's 33 wave sums in shuffles, an envelope evaluation per wave
 // and stage, one 4-byte partner load per bond and one 8-byte access per
 // component a stage of the 8x8x8 cell took 36.8 us; it takes 28 (a third of
@@ -36,38 +37,14 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "csl_mixed_lay.hpp"
 #include "csl_mixed_lds.hpp"
 
 namespace csl {
 
 namespace {
 
-constexpr int kChunk = 2;   // steps whose records and envelopes go together
-
-// LDS layout (in doubles)
-struct Lay {
-    int t, t2, f;            // SU(3) [NP3][6] (and [NP3][2] with GLDS), SU(2) [NP2][3]
-    int cst, hin, drv, red;
-    int rows, n2, n3, rec;   // units of each species, doubles per record
-    int total;
-    __host__ __device__ Lay(int NP2, int NP3, int A2, int A3, int nwaves, bool glds) {
-        t = 0;
-        t2 = 6 * NP3;
-        f = t2 + (glds ? 2 * NP3 : 0);
-        rows = 3 * A2 + 8 * A3;
-        cst = f + 3 * NP2;
-        cst += cst & 1;
-        hin = cst + 3 * rows;
-        drv = hin + 8 * rows;
-        red = drv + 2 * kChunk * 12;
-        n2 = NP2 / kWave;
-        n3 = NP3 / kWave;
-        // a record: SU(2) units x 4, SU(3) units x 8 (twice with signed
-        // sums), one energy sum per wave
-        rec = 4 * n2 + ((A3 & 1) ? 16 : 8) * n3 + 4 * nwaves;
-        total = red + kChunk * rec;
-    }
-};
+using Lay = MixPersistLay;
 
 template <int Z22, int ZM, bool GLDS>
 struct Field {
@@ -191,7 +168,7 @@ struct Field {
 
 }  // namespace
 
-template <int SPT, int T, int Z22, int ZM, bool TT, bool GLDS>
+template <int SPT, int T, int Z22, int ZM, bool TT, bool GLDS, bool TIGHT>
 __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
     extern __shared__ double smem[];
     constexpr int nwaves = T / kWave;
@@ -201,7 +178,8 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
     const int lane = tid & (kWave - 1);
     const int wave = uniform(tid >> 6);
     const int NP2 = M0->NP2, NP3 = M0->NP3, A2 = M0->A2, A3 = M0->A3, npad = M0->npad, n_cells = M0->n_cells;
-    const Lay Y(NP2, NP3, A2, A3, nwaves, GLDS);
+    const Lay Y(NP2, NP3, A2, A3, nwaves, GLDS, TIGHT);
+    constexpr int kChunk = TIGHT ? 1 : 2;
     const MixTables Q{smem + Y.cst, smem + Y.hin, smem + Y.drv, smem + Y.red, Y.rows};
     const int R = Y.rows;
     double2* const Gw = GLDS ? nullptr : reinterpret_cast<double2*>(K.A.G) + size_t(blockIdx.x) * 2 * size_t(NP3);
@@ -244,14 +222,34 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
                 else Gw[p] = make_double2(v[6], v[7]);
             }
         }
-        mix_fill_tables(M0, Q, tid, T);
+        if constexpr (TIGHT)
+            for (int st = 0; st < 4; ++st) mix_write_row(M0, Q, nullptr, st, 3 * A2, tid, T);
+        else
+            mix_fill_tables(M0, Q, tid, T);
         __syncthreads();
         auto write_drive = [&](int n0, int cp) {
             if (drive && wave == nwaves - 1) mix_write_drive(Q, b, n0, s_end, cp, kChunk, lane);
         };
         auto write_hin = [&](const double* f, int par) {
-            if (drive) mix_write_hin(Q, f, par, 3 * A2, tid, T);
+            if (!drive) return;
+            if constexpr (TIGHT)
+                for (int st = 0; st < 4; ++st) mix_write_row(M0, Q, f, st, 3 * A2, tid, T);
+            else
+                mix_write_hin(Q, f, par, 3 * A2, tid, T);
         };
+        // TIGHT: the rows of the step before are replaced one by one as they
+        // have been read: 0 and 3 by stage 0, 1 by stage 2, 2 by stage 3 (its
+        // successor is written in stage 1 of its own step)
+        auto replace_rows = [&](int s, const double* f, const double* f_next, bool more) {
+            if (!drive) return;
+            if (s == 1) mix_write_row(M0, Q, f, 2, 3 * A2, tid, T);
+            if (s == 2 && more) {
+                mix_write_row(M0, Q, f_next, 0, 3 * A2, tid, T);
+                mix_write_row(M0, Q, f_next, 3, 3 * A2, tid, T);
+            }
+            if (s == 3 && more) mix_write_row(M0, Q, f_next, 1, 3 * A2, tid, T);
+        };
+        auto field_b = [&](int i) { return TIGHT ? mix_row(M0, i).B : Q.cst[3 * i]; };
         write_drive(s_begin, 0);
         lds_barrier();
         write_hin(Q.drv, 0);
@@ -297,8 +295,9 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
         auto stage = [&](int s, int par, int slot) __attribute__((always_inline)) {
             const double cdt = s == 2 ? dt : 0.5 * dt;
             const double bdt = (s == 0 || s == 3) ? (1.0 / 6.0) * dt : (1.0 / 3.0) * dt;
-            const double* hrow = Q.hin + (par * 4 + (s == 0 ? 0 : (s == 3 ? 2 : 1))) * R;
-            const double* wrow = Q.hin + (par * 4 + 3) * R;
+            const int set = TIGHT ? 0 : par * 4;
+            const double* hrow = Q.hin + (set + (s == 0 ? 0 : (s == 3 ? 2 : 1))) * R;
+            const double* wrow = Q.hin + (set + 3) * R;
             const Field<Z22, ZM, GLDS> F{Mg, smem, Y, GLDS ? nullptr : Gw + (s & 1) * NP3};
             double2* const Gn = GLDS ? nullptr : Gw + (1 - (s & 1)) * NP3;
             double e = 0.0;
@@ -446,7 +445,9 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
                     // rows of the next step: this parity's were last read a
                     // step ago; the next chunk's envelopes are complete since
                     // stage 0
-                    if (s == 2 && n + 1 < s_end)
+                    if constexpr (TIGHT)
+                        replace_rows(s, Q.drv + cp * 12, Q.drv + (cp ^ 1) * 12, n + 1 < s_end);
+                    else if (s == 2 && n + 1 < s_end)
                         write_hin(q < kChunk ? Q.drv + (cp * kChunk + q) * 12 : Q.drv + (cp ^ 1) * kChunk * 12, par ^ 1);
                     stage(s, par, s == 0 ? slot : -1);
                     if (s == 0 && n + 1 == n1 && ri > ri0) publish(ri0, ri - ri0);
@@ -473,20 +474,20 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
                 double S[3], H[3];
                 ld3(smem + Y.f + 3 * p, S);
 #pragma unroll
-                for (int d = 0; d < 3; ++d) H[d] = -Q.cst[3 * (3 * a + d)];
+                for (int d = 0; d < 3; ++d) H[d] = -field_b(3 * a + d);
                 F.fe(a, p, S, H);
 #pragma unroll
-                for (int d = 0; d < 3; ++d) e = fma(S[d], H[d] - Q.cst[3 * (3 * a + d)], e);
+                for (int d = 0; d < 3; ++d) e = fma(S[d], H[d] - field_b(3 * a + d), e);
                 sums2(0, j, S);
             }
 #pragma unroll 1
             for (int j = 0; j < m3; ++j) {
                 const int p = p0 + j * kWave, a = atom(j);
-                const double* c3 = Q.cst + 3 * (3 * A2 + 8 * a);
+                const int c3 = 3 * A2 + 8 * a;
                 double S[8], H[8];
                 F.tm(p, S);
 #pragma unroll
-                for (int d = 0; d < 8; ++d) H[d] = -c3[3 * d];
+                for (int d = 0; d < 8; ++d) H[d] = -field_b(c3 + d);
                 F.template tm_bonds<TT>(a, p, H);
                 if (M0->has_onsite3) {
                     const cptr<double> A3m = as_const(M0->onsite3) + a * 64;
@@ -496,7 +497,7 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
                         for (int c = 0; c < 8; ++c) H[d] = fma(A3m[d * 8 + c], S[c], H[d]);
                 }
 #pragma unroll
-                for (int d = 0; d < 8; ++d) e = fma(S[d], H[d] - c3[3 * d], e);
+                for (int d = 0; d < 8; ++d) e = fma(S[d], H[d] - field_b(c3 + d), e);
                 sums3(0, j, S);
             }
             sum_e(0, e);
@@ -508,9 +509,10 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
 
 namespace {
 
-template <int SPT, int T, int Z22, int ZM, bool TT, bool GLDS>
-hipError_t launch_mp(const MixDev* M, const MixPersistArgs& A, int grid, size_t lds, hipStream_t st, int* occ) {
-    auto kern = k_mixed_persist<SPT, T, Z22, ZM, TT, GLDS>;
+template <int SPT, int T, int Z22, int ZM, bool TT, bool GLDS, bool TIGHT>
+hipError_t launch_mp(const MixDev* M, const MixPersistArgs& A, int grid, const Lay& Y, hipStream_t st, int* occ) {
+    auto kern = k_mixed_persist<SPT, T, Z22, ZM, TT, GLDS, TIGHT>;
+    const size_t lds = sizeof(double) * size_t(Y.total);
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
@@ -520,14 +522,21 @@ hipError_t launch_mp(const MixDev* M, const MixPersistArgs& A, int grid, size_t 
     return hipGetLastError();
 }
 
+Lay persist_lay(const MixDev& M, int block, bool glds) {
+    return mix_persist_lay(M.NP2, M.NP3, M.A2, M.A3, block / kWave, glds);
+}
+
 // components 6 and 7 in LDS where they fit: always up to 1024 sites of each
 // species (two units per wave of 512 threads, one of 1024)
 template <int SPT, int T, int Z22, int ZM, bool TT>
 hipError_t launch_mp_g(const MixDev& Mh, const MixDev* M, const MixPersistArgs& A, int grid, hipStream_t st, int* occ) {
-    const size_t in_lds = mixed_persist_lds_bytes(Mh, T, true);
-    if (in_lds <= 160 * 1024) return launch_mp<SPT, T, Z22, ZM, TT, true>(M, A, grid, in_lds, st, occ);
-    if constexpr (SPT * T > 1024)
-        return launch_mp<SPT, T, Z22, ZM, TT, false>(M, A, grid, mixed_persist_lds_bytes(Mh, T, false), st, occ);
+    const Lay in_lds(Mh.NP2, Mh.NP3, Mh.A2, Mh.A3, T / kWave, true, false);
+    if (in_lds.total <= kMixLdsDoubles) return launch_mp<SPT, T, Z22, ZM, TT, true, false>(M, A, grid, in_lds, st, occ);
+    if constexpr (SPT * T > 1024) {
+        const Lay Y = persist_lay(Mh, T, false);
+        return Y.tight ? launch_mp<SPT, T, Z22, ZM, TT, false, true>(M, A, grid, Y, st, occ)
+                       : launch_mp<SPT, T, Z22, ZM, TT, false, false>(M, A, grid, Y, st, occ);
+    }
     return hipErrorInvalidValue;
 }
 
@@ -560,12 +569,8 @@ MixPersistShape mixed_persist_shape(const MixDev& M, bool tt) {
         const int spt = (np + 511) / 512;
         if (spt <= 4) sh = {512, spt, true, false};
     }
-    if (sh.block && mixed_persist_lds_bytes(M, sh.block, false) > 160 * 1024) sh = {0, 0, tt, false};
+    if (sh.block && persist_lay(M, sh.block, false).total > kMixLdsDoubles) sh = {0, 0, tt, false};
     return sh;
-}
-
-size_t mixed_persist_lds_bytes(const MixDev& M, int block, bool glds) {
-    return sizeof(double) * size_t(Lay(M.NP2, M.NP3, M.A2, M.A3, block / kWave, glds).total);
 }
 
 hipError_t launch_mixed_persist(const MixDev& Mh, const MixDev* M, const MixPersistArgs& A, const MixPersistShape& sh,

@@ -67,3 +67,35 @@ def test_tangent_with_uneven_sublattices(oracle, A2, A3, dims, tt):
     grad = 2.0 * np.sum(w * (ref - target) * tr)
     # 33 n products of records within 1e-12 and these tangents, summed in another order
     assert abs(g["grad"][0] - grad) <= 1e-10 * np.sum(np.abs(w * (ref - target) * tr))
+
+
+@pytest.mark.parametrize("A2,A3,dims,tt,steps,every", [
+    (16, 16, (8, 4, 4), True, 5, 1),      # 128 cells: 170 KB with the roomy tables
+    (16, 16, (5, 5, 5), False, 4, 3),
+    (32, 31, (4, 4, 4), False, 3, 1),     # 64 cells, the most sublattices; odd
+    (32, 31, (1, 9, 7), True, 2, 2),
+])
+def test_many_sublattices_stay_persistent(oracle, A2, A3, dims, tt, steps, every):
+    """Lattices of 2048 sites of each species whose field rows leave no room
+    for two steps' worth: driven, three trajectories, against the oracle."""
+    muc = uneven_cell(A2, A3, tt)
+    ml = mm.MixedLattice(muc, *dims)
+    init = ml.flat_state(seeding.random_spins(ml.N2, 3), mm.random_su3_states(ml.N3, 4))
+    g = np.random.default_rng(1)
+    f2, f3 = g.normal(size=(A2, 3)), g.normal(size=(A3, 8))
+    tp = np.array([[0.0, 0.0], [0.01, 0.015], [0.0, 0.02]])
+    sc = np.array([[0.0, 0.0], [1.0, 0.5], [0.0, 1.0]])
+    T1 = (steps + 0.5) * DT
+    print(f"[mixed] {A2} + {A3} sublattices of {dims}", flush=True)
+    with GM.GPUMixedLattice(ml) as gm:
+        GM._set_pulses(gm, f2, f2, f3, f3, 0.0, 0.0, 0.5, 0.02, 3.0, 0.4, 0.03, 0.0)
+        r = gm.integrate_batched(init, tp, sc, 0.0, T1, DT, save_interval=every, want_final=True)
+        assert gm.last_path()["persistent"]
+    keep = sorted(set(range(0, steps, every)) | {steps})
+    for b in range(3):
+        o = oracle.MixedOracle(muc, *dims)
+        o.set_pulse(2, f2 * sc[b, 0], tp[b, 0], f2 * sc[b, 1], tp[b, 1], 0.5, 0.02, 3.0)
+        o.set_pulse(3, f3 * sc[b, 0], tp[b, 0], f3 * sc[b, 1], tp[b, 1], 0.4, 0.03, 0.0)
+        ref = o.integrate_md(init, 0.0, T1, DT)
+        assert np.max(np.abs(r["records"][:, b] - ref["records"][keep])) <= 1e-12
+        assert np.max(np.abs(r["final"][b] - ref["final"])) <= 1e-12
