@@ -101,7 +101,7 @@ __device__ __forceinline__ void sweep_wave(double* smem, int wave, int wstart) {
     const double* const mats = K->L.mats + size_t(b) * K->A.mats_stride + atom * kZ * 9;
     const int n0 = K->A.n0, n1 = K->A.n1;  // stage slots q = 4 n + s of these steps
     const double* const Yb = K->A.Y + (size_t(b) * K->A.seg_len - K->A.y0) * 4 * SZ;
-    const double* const rows = K->A.rows + (size_t(b) * (K->A.n_steps + 1) * n_atoms + atom) * kRow;
+    const double* const rows = K->A.rows + ((size_t(b) * (K->A.seg_len + 1) - K->A.y0) * n_atoms + atom) * kRow;
 
     const int pbase = atom * npad + wstart * kWave + lane;
     int nb[NU][kZ];
@@ -409,16 +409,16 @@ __device__ __forceinline__ void sweep_wave(double* smem, int wave, int wstart) {
 
 }  // namespace
 
-// What the sweep needs of a step besides its states, a thread per (trajectory,
-// step, sublattice): -(B + drive) at the step's three stage times and
+// What the sweep needs of a step of its segment besides the states, a thread
+// per (trajectory, step, sublattice): -(B + drive) at the step's three stage times and
 // d l_n / d x_n, so that the sequential sweep reads three uniform values a
 // stage; and the loss term of the record.
 __global__ void __launch_bounds__(256) k_adj_rows(LatDev L, AdjArgs A) {
-    const size_t n_rec = size_t(A.n_steps) + 1, i = size_t(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= n_rec * A.B * L.n_atoms) return;
+    const size_t n_rec = size_t(A.n_steps) + 1, n_seg = size_t(A.n1 - A.n0) + 1, i = size_t(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= n_seg * A.B * L.n_atoms) return;
     const int atom = int(i % L.n_atoms);
-    const size_t n = i / L.n_atoms % n_rec, b = i / L.n_atoms / n_rec;
-    double* out = A.rows + i * kRow;
+    const size_t n = A.n0 + i / L.n_atoms % n_seg, b = i / L.n_atoms / n_seg;
+    double* out = A.rows + ((b * (A.seg_len + 1) + n - A.y0) * L.n_atoms + atom) * kRow;
     const double* B = L.field + b * A.field_stride + atom * 3;
     for (int sg = 0; sg < 3; ++sg) {
         double f[2] = {0.0, 0.0};
@@ -514,7 +514,7 @@ bool adjoint_sweep_fits(const LatDev& L) { return sweep_shape(L).block > 0; }
 size_t adjoint_row_doubles(const LatDev& L) { return size_t(L.n_atoms) * kRow; }
 
 hipError_t launch_adjoint_rows(const LatDev& L, const AdjArgs& A, hipStream_t st) {
-    const size_t n = (size_t(A.n_steps) + 1) * A.B * L.n_atoms;
+    const size_t n = (size_t(A.n1 - A.n0) + 1) * A.B * L.n_atoms;
     hipLaunchKernelGGL(k_adj_rows, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, L, A);
     return hipGetLastError();
 }

@@ -2408,7 +2408,7 @@ int csl_adjoint_gradient(csl_lattice* h, size_t B, const double* init, int init_
         d_rec.ensure(n_rec * B * 9);
         d_lossn.ensure(B * n_rec);
         d_part.ensure(sweep ? B * csl::adjoint_sweep_doubles(L) : B * n_steps * 4 * std::max<size_t>(n_params, 1));
-        if (sweep) h->adj_rows.ensure(B * n_rec * csl::adjoint_row_doubles(L));
+        if (sweep) h->adj_rows.ensure(B * (C + 1) * csl::adjoint_row_doubles(L));
         d_loss.ensure(B);
         d_grad.ensure(B * std::max<size_t>(n_params, 1));
         if (grad_init) d_gi.ensure(B * nd);
@@ -2467,21 +2467,18 @@ int csl_adjoint_gradient(csl_lattice* h, size_t B, const double* init, int init_
             }
         }
         csl::AdjArgs Fin = Aa;
-        if (sweep) {
-            Fin.P = 0;  // the sweep writes the gradient itself
-            hip_check(csl::launch_adjoint_rows(L, Aa, s), "k_adj_rows launch");
-            ++launches;
-        }
+        if (sweep) Fin.P = 0;  // the sweep writes the gradient itself
         if (full && sweep) {
             csl::AdjArgs G = Aa;
             G.n0 = 0;
             G.n1 = int(n_steps);
             G.y0 = 0;
             G.first = 1;
+            hip_check(csl::launch_adjoint_rows(L, G, s), "k_adj_rows launch");
             hip_check(csl::launch_adjoint_sweep(L, G, s), "k_adj_sweep launch");
             hip_check(csl::launch_adjoint_final(Fin, s), "k_adj_final launch");
             hip_check(hipEventRecord(e1, s), "event record");
-            ++launches;
+            launches += 2;
         } else if (full) {
             // the backward sweep in segments; the parameter terms of a
             // finished segment run on the second stream (on the CUs the
@@ -2534,8 +2531,9 @@ int csl_adjoint_gradient(csl_lattice* h, size_t B, const double* init, int init_
                 ++launches;
                 G.first = j == n_seg - 1 ? 1 : 0;
                 if (sweep) {
+                    hip_check(csl::launch_adjoint_rows(L, G, s), "k_adj_rows launch");
                     hip_check(csl::launch_adjoint_sweep(L, G, s), "k_adj_sweep launch");
-                    ++launches;
+                    launches += 2;
                     continue;
                 }
                 hip_check(csl::launch_adjoint_backward(L, G, s), "k_adj_bwd launch");

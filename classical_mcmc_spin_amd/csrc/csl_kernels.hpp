@@ -156,7 +156,7 @@ struct AdjArgs {
     double* rec;               // [n_steps+1][B][9] forward records
     double* loss_n;            // [B][n_steps+1] loss term of every record
     double* part;              // [B][n_steps][4][P] parameter-gradient term of every stage (sweep: thread sums)
-    double* rows;              // sweep: fields and loss cotangents of every step
+    double* rows;              // sweep: fields and loss cotangents of a segment's steps [B][seg_len + 1]
     double* grad_init;         // [B][N*3] dL/dx_0 (AoS), written by the launch with n0 == 0, or null
     double* loss;              // [B] (final kernel)
     double* grad;              // [B][P] (final kernel)
@@ -177,8 +177,8 @@ hipError_t launch_adjoint_final(const AdjArgs& A, hipStream_t st);
 // (csl_adjoint_sweep.hip), for lattices with three bonds at every site,
 // per-sublattice fields and no onsite matrix whose sublattices fit its waves.
 // A.part holds the thread sums handed between segments (adjoint_sweep_doubles
-// per trajectory); the launch with n0 == 0 writes A.grad.  Before it,
-// launch_adjoint_rows turns the records of all steps into A.rows
+// per trajectory); the launch with n0 == 0 writes A.grad.  Before each,
+// launch_adjoint_rows turns the records n0 .. n1 of its segment into A.rows
 // (adjoint_row_doubles per trajectory and record) and the loss terms.
 bool adjoint_sweep_fits(const LatDev& L);
 size_t adjoint_sweep_doubles(const LatDev& L);

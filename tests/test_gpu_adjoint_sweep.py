@@ -43,3 +43,28 @@ def test_sweep_shapes(po, L1, L2, alpha):  # noqa: F811
         lo, g = _oracle_grad(po, th[b], L1, L2, init, T0, T1, dt, target, alpha, pulse)
         assert abs(outs[0][0][b] - lo) <= 1e-10 * abs(lo)
         assert np.abs(outs[0][1][b] - g).max() <= 1e-10 * np.abs(g).max()
+
+
+def test_checkpointed_memory(po):  # noqa: F811
+    """With checkpoints a run keeps buffers of one segment: beside the records
+    and their loss terms (10 doubles a start and step) and drive factors (6),
+    nothing grows with the number of steps but the checkpoints."""
+    import torch
+    L1, L2, n, dt, ck, B = 6, 6, 4000, 0.002, 64, 64
+    pulse = (0.5, 0.5, 0.0, 0.2)
+    init, T0, T1, target = _setup(po, L1, L2, n, dt, 0.02, pulse)
+    th = np.tile(THETA_STAR * 1.05, (B, 1))
+    fit = AD.KitaevFit(L1, L2, init, target, T0, T1, dt, pulse=pulse, alpha=0.02, weights=W, ckpt_interval=ck)
+    try:
+        torch.cuda.synchronize()
+        free0, _ = torch.cuda.mem_get_info()
+        fit(th)
+        torch.cuda.synchronize()
+        free1, _ = torch.cuda.mem_get_info()
+    finally:
+        fit.close()
+    site = 3 * 2 * 64 * 8   # one padded state
+    need = B * (ck * 4 * site + (n // ck + 1) * site + n * 16 * 8)
+    print(f"[adjoint memory] {(free0 - free1) / 2**20:.0f} MB, buffers that scale {need / 2**20:.0f} MB", flush=True)
+    # and under 25 MB of tables, inputs and rounding to pages of 2 MB
+    assert free0 - free1 <= need + (25 << 20)
