@@ -85,7 +85,13 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
 
     const int pbase = atom * npad + wstart * kWave + lane;
     double x[NU][3], acc[NU][3], y[NU][3];
-    int nb[NU][ZMAX];
+    // Twelve bonds and three sites a thread or more: partners two to a word,
+    // and a stage's own value read back from LDS, or 470 bytes a lane spill
+    // (600 trajectories of 36x36 x 200 steps: 11.3 -> 8.3 ms a call; at two
+    // sites and fewer unpacking costs 7 %).
+    constexpr bool kPack = ZMAX > 6 && SPT > 2;
+    constexpr int kWords = kPack ? (ZMAX + 1) / 2 : ZMAX;
+    unsigned nb[NU][kWords];
 #pragma unroll
     for (int m = 0; m < NU; ++m) {
         // padding lanes (no cell) hold a zero spin and gather themselves:
@@ -93,8 +99,18 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
         const int p = pbase + m * kWave;
         const bool real = p - atom * npad < K.L.n_cells;
 #pragma unroll
-        for (int k = 0; k < ZMAX; ++k) nb[m][k] = real ? K.L.col[size_t(k) * NP + p] : p;
+        for (int k = 0; k < kWords; ++k) nb[m][k] = 0;
+#pragma unroll
+        for (int k = 0; k < ZMAX; ++k) {
+            const unsigned q = real ? K.L.col[size_t(k) * NP + p] : p;
+            if constexpr (kPack) nb[m][k >> 1] |= q << (16 * (k & 1));
+            else nb[m][k] = q;
+        }
     }
+    auto nbr = [&](int m, int k) {
+        if constexpr (kPack) return int((unsigned(fresh(int(nb[m][k >> 1]))) >> (16 * (k & 1))) & 0xffffu);
+        else return int(nb[m][k]);
+    };
     const double dt = K.A.dt;
     const double b16 = (1.0 / 6.0) * dt, b13 = (1.0 / 3.0) * dt, hdt = 0.5 * dt;
 
@@ -272,7 +288,7 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
                 }
                 double S[NU][3];
 #pragma unroll
-                for (int m = 0; m < NU; ++m) lds_ld(cur, nb[m][0], S[m]);
+                for (int m = 0; m < NU; ++m) lds_ld(cur, nbr(m, 0), S[m]);
 #pragma unroll
                 for (int k = 0; k < ZMAX; ++k) {
 #pragma unroll
@@ -281,7 +297,7 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
                         for (int e = 0; e < 3; ++e)
 #pragma unroll
                             for (int d = 0; d < 3; ++d) H[m][d] = fma(Jh[k * 9 + d * 3 + e], S[m][e], H[m][d]);
-                        if (k + 1 < ZMAX) lds_ld(cur, nb[m][k + 1], S[m]);
+                        if (k + 1 < ZMAX) lds_ld(cur, nbr(m, k + 1), S[m]);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
@@ -297,13 +313,22 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
 #pragma unroll
                     for (int m = 0; m < NU; ++m) {
                         double S[3];
-                        lds_ld(cur, nb[m][k], S);
+                        lds_ld(cur, nbr(m, k), S);
 #pragma unroll
                         for (int e = 0; e < 3; ++e)
 #pragma unroll
                             for (int d = 0; d < 3; ++d) H[m][d] = fma(J[d * 3 + e], S[e], H[m][d]);
                     }
                 }
+            }
+            // damped: a unit's root and division make a branch, into which the
+            // compiler puts off the field's products and the updates of the
+            // other units with all their operands: 300 to 2600 bytes a lane of
+            // spills, and 24x24 with twelve bonds 64 x 200 steps 4.3 ms
+            // against 2.0 with the field and each unit's update held
+            if constexpr (DAMP) {
+#pragma unroll
+                for (int m = 0; m < NU; ++m) hold(H[m]);
             }
             if (s == 0 && slot >= 0) {
                 // e = sum S.H - (hin + 2B).S with the driven H: the undriven
@@ -322,7 +347,9 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
             }
 #pragma unroll
             for (int m = 0; m < NU; ++m) {
-                const double* Sm = s == 0 ? x[m] : y[m];
+                double own[3];
+                if constexpr (kPack && s > 0) lds_ld(cur, fresh(pbase + m * kWave), own);
+                const double* Sm = s == 0 ? x[m] : (kPack ? own : y[m]);
                 double k[3];
                 if constexpr (DAMP) {
                     ll_su2_guarded(H[m], Sm, K.L.alpha, k);
@@ -337,6 +364,14 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
                     else if (s < 3) acc[m][d] = acc[m][d] + bdt * k[d];
                     else x[m][d] = acc[m][d] + bdt * k[d];
                     if (s < 3) y[m][d] = x[m][d] + cdt * k[d];
+                }
+                if constexpr (DAMP) {
+                    if constexpr (s < 3) {
+                        hold(acc[m]);
+                        hold(y[m]);
+                    } else {
+                        hold(x[m]);
+                    }
                 }
                 lds_st(nxt, pbase + m * kWave, s < 3 ? y[m] : x[m]);
             }
@@ -415,7 +450,7 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
 #pragma unroll
                 for (int k = 0; k < ZMAX; ++k) {
                     double S[3];
-                    lds_ld(0, nb[m][k], S);
+                    lds_ld(0, nbr(m, k), S);
                     add_bond_fused(as_const(mats) + (atom * ZMAX + k) * 9, S, H);
                 }
 #pragma unroll

@@ -67,6 +67,37 @@ def test_trajectory_edges(oracle, name, steps, every, alpha):
         assert np.max(np.abs(r["final"][b] - ref["final"].reshape(-1, 3))) <= TOL
 
 
+@pytest.mark.parametrize("dims,shapes", [((23, 25, 1), {2, 3}), ((36, 28, 1), {2, 3, 4, 6}), ((31, 39, 1), {3, 4})])
+@pytest.mark.parametrize("alpha", [0.0, 0.03])
+def test_twelve_bonds_every_sites_per_thread(oracle, dims, shapes, alpha):
+    """Twelve bonds a site, damped and not, at every atom-major launch shape of
+    the lattice (from three sites a thread on the partners are packed)."""
+    uc = _kitaev(J2_A=0.1, J2_B=-0.07, J3=0.05)
+    lat = model.Lattice(uc, *dims)
+    s = random_state(lat, 78)
+    steps = 9
+    T1 = (steps + 0.5) * DT
+    o = oracle.OracleLattice(uc, *dims)
+    o.set_alpha(alpha)
+    ref = o.integrate_md(s.reshape(-1), 0.0, T1, DT)
+    seen = set()
+    with GPULattice(lat) as gl:
+        gl.set_damping(alpha)
+        for c in gl.launch_candidates():
+            if not c["atom_major"]:
+                continue
+            gl.set_launch_config(2, c["block"], c["sites_per_thread"], c["flags"])
+            print(f"[twelve] {dims} alpha {alpha} {c}", flush=True)
+            r = gl.integrate_batched(s, np.zeros((2, 2)), np.zeros((2, 2)), 0.0, T1, DT, tgrid="boost", want_final=True)
+            assert gl.last_launch_config()["atom_major"]
+            seen.add(c["sites_per_thread"])
+            for b in range(2):
+                assert np.max(np.abs(r["mags"][:, b] - ref["mags"])) <= TOL
+                assert np.max(np.abs(r["energy"][:, b] - ref["energy"])) <= TOL
+                assert np.max(np.abs(r["final"][b] - ref["final"].reshape(-1, 3))) <= TOL
+    assert shapes <= seen
+
+
 @pytest.mark.parametrize("n_tau,steps", [(1, 1), (7, 15), (8, 16), (17, 33)])
 def test_pump_probe_rows(n_tau, steps):
     """Trajectory-major pump-probe records (tiles of 16 records x 16
