@@ -1697,8 +1697,10 @@ void run_mixed(csl_mixed* h, size_t B, const double* d_tp, const double* d_tp3, 
     hip_check(hipEventCreate(&e1), "event");
     size_t launches = 0;
     const dim3 grid_dim{unsigned(nblk), unsigned(B), 1u};
-    // tangent runs: the padded tables where the lattice has them
-    const int padded = h->M.jpad ? h->M.jz22 * 10 + h->M.jzm : 0;
+    // tangent runs: the padded tables where the lattice has them and every
+    // slot names a site (their stage values are in device memory, without a
+    // record of zeros)
+    const int padded = h->M.jpad && !h->M.bondless ? h->M.jz22 * 10 + h->M.jzm : 0;
     auto* const tl_kernel = padded == 64   ? csl::k_mixed_stage<true, 6, 4>
                             : padded == 68 ? csl::k_mixed_stage<true, 6, 8>
                             : padded == 84 ? csl::k_mixed_stage<true, 8, 4>
@@ -1952,7 +1954,7 @@ bool run_mixed_persist(csl_mixed* h, size_t B, const double* d_tp, const double*
         A.status = h->pflags.p + grid_wg;
     }
     h->recs.ensure(n_rec * B * CSL_MIXED_RECORD);
-    h->pG.ensure(grid_wg * 4 * size_t(h->M.NP3));
+    h->pG.ensure(grid_wg * 4 * size_t(h->M.NP3 + 1));
     h->ptgrid.upload(grid.data(), grid.size(), s);
     A.b0 = 0;
     A.B = int(B);
@@ -2199,14 +2201,14 @@ int csl_mixed_create(size_t A2, size_t A3, size_t n_cells, const double* field2,
                     pk.resize((pk.size() + 255) / 256 * 256);
                     return at;
                 };
-                auto partners = [&](const EllHost& e, int NP, int Z) {
-                    const auto q = cslh::packed_partners(e.col.data(), e.cnt.data(), NP, Z, npad);
+                auto partners = [&](const EllHost& e, int NP, int Z, int npart) {
+                    const auto q = cslh::packed_partners(e.col.data(), e.cnt.data(), NP, Z, npart);
                     return put(q.data(), q.size() * sizeof(unsigned short));
                 };
-                const size_t o22 = partners(e22, M.NP2, csl::kMixZ22);
-                const size_t o23 = partners(e23, M.NP2, csl::kMixZ23);
-                const size_t o32 = partners(e32, M.NP3, csl::kMixZ32);
-                const size_t o33 = partners(e33, M.NP3, csl::kMixZ33);
+                const size_t o22 = partners(e22, M.NP2, csl::kMixZ22, M.NP2);
+                const size_t o23 = partners(e23, M.NP2, csl::kMixZ23, M.NP3);
+                const size_t o32 = partners(e32, M.NP3, csl::kMixZ32, M.NP2);
+                const size_t o33 = partners(e33, M.NP3, csl::kMixZ33, M.NP3);
                 const size_t oj = put(P.mats.data(), P.mats.size() * sizeof(double));
                 const size_t oo = put(P.off32.data(), P.off32.size() * sizeof(int));
                 h->ppack.upload(pk.data(), pk.size(), s);
@@ -2217,6 +2219,8 @@ int csl_mixed_create(size_t A2, size_t A3, size_t n_cells, const double* field2,
                 M.jpad = reinterpret_cast<const double*>(h->ppack.p + oj);
                 M.j32pad = reinterpret_cast<const int*>(h->ppack.p + oo);
                 M.j22off = P.j22off;
+                for (const EllHost* e : {&e22, &e23, &e32})
+                    for (int c : e->cnt_atom) M.bondless |= c == 0;
                 M.jz22 = P.z22;
                 M.jzm = P.zm;
             }

@@ -54,6 +54,7 @@ struct MixDev {
     const double* __restrict__ jpad;
     const int* __restrict__ j32pad;
     int j22off, jz22, jzm;
+    int bondless;  // a sublattice has no bonds of kind 22, 23 or 32 (its packed partners name the record of zeros)
 };
 
 constexpr int kRec = CSL_MIXED_RECORD;
@@ -112,7 +113,7 @@ struct MixPersistArgs {
     double dt;
     const double* tgrid;       // [n_steps + 1] step start times
     double* X;                 // [B_rec][3 NP2 + 8 NP3] SoA states: initial in, final out; x during the run
-    double* G;                 // [grid][2 parities][NP3][2] SU(3) components 6, 7 of the stage values
+    double* G;                 // [grid][2 parities][NP3 + 1][2] SU(3) components 6, 7 of the stage values
     const double* tp;          // [B_rec][2] SU(2) pulse centres, or null: no drive
     const double* tp3;         // [B_rec][2] SU(3) pulse centres
     const double* scale;       // [B_rec][2] pulse scales, or null (1)

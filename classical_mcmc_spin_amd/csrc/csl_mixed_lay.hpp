@@ -10,7 +10,9 @@ constexpr int kMixLdsDoubles = 160 * 1024 / 8;
 struct MixPersistLay {
     int chunk = 2;                           // steps whose records and envelopes go together
     bool tight = false;
-    int t = 0, t2 = 0, f = 0;                // SU(3) [NP3][6] (and [NP3][2] with GLDS), SU(2) [NP2][3]
+    // SU(3) [NP3 + 1][6] (and [NP3 + 1][2] with GLDS), SU(2) [NP2 + 1][3]; the
+    // last record of each is zero (csl_mixed_pack.hpp)
+    int t = 0, t2 = 0, f = 0;
     int cst = 0, hin = 0, drv = 0, red = 0;  // per-sublattice B, d0, d1; field rows; envelopes; record sums
     int rows = 0, n2 = 0, n3 = 0, rec = 0;   // field components; units of each species; doubles per record
     int total = 0;
@@ -23,10 +25,10 @@ struct MixPersistLay {
     // on the stage kernels.
     constexpr MixPersistLay(int NP2, int NP3, int A2, int A3, int nwaves, bool glds, bool tight_) : tight(tight_) {
         chunk = tight ? 1 : 2;
-        t2 = 6 * NP3;
-        f = t2 + (glds ? 2 * NP3 : 0);
+        t2 = 6 * (NP3 + 1);
+        f = t2 + (glds ? 2 * (NP3 + 1) : 0);
         rows = 3 * A2 + 8 * A3;
-        cst = f + 3 * NP2;
+        cst = f + 3 * (NP2 + 1);
         cst += cst & 1;
         hin = cst + (tight ? 0 : 3 * rows);
         drv = hin + (tight ? 4 : 8) * rows;

@@ -182,7 +182,8 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
     constexpr int kChunk = TIGHT ? 1 : 2;
     const MixTables Q{smem + Y.cst, smem + Y.hin, smem + Y.drv, smem + Y.red, Y.rows};
     const int R = Y.rows;
-    double2* const Gw = GLDS ? nullptr : reinterpret_cast<double2*>(K.A.G) + size_t(blockIdx.x) * 2 * size_t(NP3);
+    const int GS = NP3 + 1;                          // a parity of components 6, 7 in global memory
+    double2* const Gw = GLDS ? nullptr : reinterpret_cast<double2*>(K.A.G) + size_t(blockIdx.x) * 2 * size_t(GS);
     const size_t SZ = 3 * size_t(NP2) + 8 * size_t(NP3);
     const size_t o3 = 3 * size_t(NP2);
     const double dt = K.A.dt;
@@ -200,7 +201,13 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
         if (P.wait >= 0) mix_wait_seam(K.A, P.wait, tid);
         __syncthreads();  // the previous piece is done with LDS and G
         // initial state: the stage values of stage 0; padding lanes hold
-        // zeros and gather padding, so their derivative is zero
+        // zeros and gather zeros, so their derivative is zero
+        if (tid < 6) smem[Y.t + 6 * NP3 + tid] = 0.0;
+        if (tid < 3) smem[Y.f + 3 * NP2 + tid] = 0.0;
+        if (tid < 2) {
+            if constexpr (GLDS) smem[Y.t2 + 2 * NP3 + tid] = 0.0;
+            else Gw[tid * GS + NP3] = make_double2(0.0, 0.0);
+        }
 #pragma unroll
         for (int j = 0; j < SPT; ++j) {
             const int p = p0 + j * kWave;
@@ -298,8 +305,8 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
             const int set = TIGHT ? 0 : par * 4;
             const double* hrow = Q.hin + (set + (s == 0 ? 0 : (s == 3 ? 2 : 1))) * R;
             const double* wrow = Q.hin + (set + 3) * R;
-            const Field<Z22, ZM, GLDS> F{Mg, smem, Y, GLDS ? nullptr : Gw + (s & 1) * NP3};
-            double2* const Gn = GLDS ? nullptr : Gw + (1 - (s & 1)) * NP3;
+            const Field<Z22, ZM, GLDS> F{Mg, smem, Y, GLDS ? nullptr : Gw + (s & 1) * GS};
+            double2* const Gn = GLDS ? nullptr : Gw + (1 - (s & 1)) * GS;
             double e = 0.0;
             double y2[SPT][3];
             auto fe_unit = [&](int j) __attribute__((always_inline)) {

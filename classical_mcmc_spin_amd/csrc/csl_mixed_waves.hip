@@ -29,16 +29,19 @@ constexpr int kChunk = 4;   // steps whose records and envelopes go together
 
 // LDS layout (in doubles)
 struct Lay {
-    int f, t, t2;            // stage values of one buffer: SU(2) [NP2][3], SU(3) [NP3][6] and [NP3][2]
+    // stage values of one buffer: SU(2) [NP2 + 1][3], SU(3) [NP3 + 1][6] and
+    // [NP3 + 1][2]; the last record of each is zero (csl_mixed_pack.hpp)
+    int f, t, t2;
     int buf;                 // size of a buffer
     int cst, hin, drv, red;  // per-sublattice B, d0, d1; field rows; envelopes; record sums
     int rows, width;         // 3 A2 + 8 A3; sums per unit and record
     int total;
     __host__ __device__ Lay(int NP2, int NP3, int A2, int A3, int nwaves) {
         t = 0;
-        t2 = 6 * NP3;
-        f = 8 * NP3;
-        buf = 8 * NP3 + 3 * NP2;
+        t2 = 6 * (NP3 + 1);
+        f = 8 * (NP3 + 1);
+        buf = f + 3 * (NP2 + 1);
+        buf += buf & 1;
         rows = 3 * A2 + 8 * A3;
         width = (A3 & 1) ? 20 : 12;
         cst = 2 * buf;
@@ -202,7 +205,12 @@ __device__ __forceinline__ void run_unit(const MixKernArgs& K, double* smem, con
         const bool drive = K.A.tp != nullptr;
         if (P.wait >= 0) mix_wait_seam(K.A, P.wait, tid);
         __syncthreads();  // the previous piece is done with the LDS
-        // padding lanes hold zeros and gather padding: their derivative is zero
+        // padding lanes hold zeros and gather zeros: their derivative is zero
+        if (tid < 22) {
+            double* b0 = smem + tid / 11 * Y.buf;
+            const int i = tid % 11;
+            b0[i < 6 ? Y.t + 6 * NP3 + i : (i < 8 ? Y.t2 + 2 * NP3 + i - 6 : Y.f + 3 * NP2 + i - 8)] = 0.0;
+        }
         double x[D], acc[D], y[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) x[d] = real ? X[size_t(d) * NP + p] : 0.0;

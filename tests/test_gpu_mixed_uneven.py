@@ -99,3 +99,40 @@ def test_many_sublattices_stay_persistent(oracle, A2, A3, dims, tt, steps, every
         ref = o.integrate_md(init, 0.0, T1, DT)
         assert np.max(np.abs(r["records"][:, b] - ref["records"][keep])) <= 1e-12
         assert np.max(np.abs(r["final"][b] - ref["final"])) <= 1e-12
+
+
+@pytest.mark.parametrize("dims", [(2, 2, 2), (3, 3, 3), (7, 7, 5), (8, 8, 8)])
+@pytest.mark.parametrize("coupled", [False, True])
+def test_an_overflow_stays_where_the_bonds_lead(dims, coupled):
+    """SU(3) sites that overflow (values of 1e200 at the start) leave alone what
+    no bond ties to them: the SU(2) species without mixed bonds, or with them
+    the SU(3) sublattice that has none.  The same states to the last bit as
+    beside ordinary spins, in the batch and in the tangent run's forward one."""
+    muc = uneven_cell(4, 3)
+    # mixed bonds to the first two SU(3) sublattices, or none
+    muc.bilinear_SU2_SU3 = [b for b in muc.bilinear_SU2_SU3 if b.partner < 2] if coupled else []
+    ml = mm.MixedLattice(muc, *dims)
+    s2, s3 = seeding.random_spins(ml.N2, 3), mm.random_su3_states(ml.N3, 4)
+    huge = s3.copy()
+    wild = np.arange(ml.N3) % 3 != 2 if coupled else np.ones(ml.N3, bool)
+    huge[wild] *= 1e200
+    n = 3
+    T1 = (n + 0.5) * DT
+    out = []
+    with GM.GPUMixedLattice(ml) as gm:
+        for x in (s3, huge):
+            init = ml.flat_state(s2, x)
+            r = gm.integrate_batched(init, [[0.0, 0.0]], None, 0.0, T1, DT, want_final=True)
+            assert gm.last_path()["persistent"]
+            g = gm.scale_gradient(init, [[0.0, 0.0]], np.zeros((n + 1, 34)), np.r_[np.ones(33), 0.0], None, 0.0, T1,
+                                  DT, want_records=True)
+            out.append((ml.split_state(r["final"][0]), r["records"][:, 0], g["records"][:, 0], g["trecords"][:, 0]))
+    (a2, a3), (b2, b3) = out[0][0], out[1][0]
+    assert not np.all(np.isfinite(b3))
+    if coupled:
+        assert np.array_equal(a3[~wild], b3[~wild])
+    else:
+        assert np.array_equal(a2, b2)
+        for q in (1, 2):
+            assert np.array_equal(out[0][q][:, :9], out[1][q][:, :9])
+        assert np.all(out[1][3][:, :9] == 0.0)

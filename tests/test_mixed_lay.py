@@ -22,7 +22,7 @@ int main() {
                     if (Y.total * 8 > 160 * 1024 && ++bad < 5)
                         std::printf("%d + %d sublattices of %d: %d bytes\\n", A2, A3, npad, Y.total * 8);
                     const int at[] = {Y.t, Y.t2, Y.f, Y.cst, Y.hin, Y.drv, Y.red, Y.total};
-                    const int size[] = {6 * A3 * npad, 0, 3 * A2 * npad, Y.tight ? 0 : 3 * Y.rows,
+                    const int size[] = {6 * A3 * npad + 6, 0, 3 * A2 * npad + 3, Y.tight ? 0 : 3 * Y.rows,
                                         (Y.tight ? 4 : 8) * Y.rows, 24 * Y.chunk, Y.chunk * Y.rec};
                     for (int i = 0; i < 7; ++i)
                         if (at[i] + size[i] > at[i + 1]) ++bad, std::printf("part %d overlaps\\n", i);
