@@ -113,6 +113,7 @@ SIGNATURES = {
     "csl_mixed_last_kernel_ms": (_i, [_vp, _pd, _psz]),
     "csl_mixed_set_persistent": (_i, [_vp, _i]),
     "csl_mixed_last_path": (_i, [_vp, _pi, _pi, _psz, _pd]),
+    "csl_mixed_last_variant": (_i, [_vp, _pi]),
 }
 
 

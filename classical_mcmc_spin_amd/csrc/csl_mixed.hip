@@ -1574,7 +1574,7 @@ struct csl_mixed {
     // persistent batched kernel: 0 when the lattice qualifies, -1 stage
     // kernels, n > 0 at most n co-resident workgroups
     int persist_mode = 0;
-    int last_persist = 0, last_persist_grid = 0;
+    int last_persist = 0, last_persist_grid = 0, last_variant = 0;
     size_t last_split = 0;  // trajectories the persistent kernel ran in two pieces
     double last_persist_ms = 0.0;  // the persistent launch alone
     DBuf<double> pG, ptgrid;
@@ -1994,6 +1994,7 @@ bool run_mixed_persist(csl_mixed* h, size_t B, const double* d_tp, const double*
     h->last_persist_ms = ms;
     h->last_launches = 1;
     h->last_persist = 1;
+    h->last_variant = csl::mixed_persist_variant(h->M, shape);
     h->last_persist_grid = int(grid_wg);
     h->last_split = n_split;
     return true;
@@ -2027,6 +2028,7 @@ bool run_mixed_coop_batch(csl_mixed* h, size_t B, const double* d_tp, const doub
     h->last_persist_ms = ms;
     h->last_launches = 1;
     h->last_persist = 2;
+    h->last_variant = 0;
     h->last_persist_grid = int(B) * (blocks_of(h->M.NP2) + blocks_of(h->M.NP3));
     h->last_split = 0;
     return true;
@@ -2529,6 +2531,7 @@ int csl_mixed_integrate_batched(csl_mixed* h, size_t B, const double* init, int 
         hip_check(hipMemsetAsync(h->X.p, 0, B * h->sz() * sizeof(double), s), "memset");
         to_soa(h, h->init.p, init_per_replica ? nf : 0, h->X.p, B);
         h->last_persist = 0;
+        h->last_variant = 0;
         h->last_persist_grid = 0;
         h->last_split = 0;
         h->last_persist_ms = 0.0;
@@ -2842,6 +2845,13 @@ int csl_mixed_last_path(csl_mixed* h, int* persistent, int* workgroups, size_t* 
         if (workgroups) *workgroups = h->last_persist_grid;
         if (split) *split = h->last_split;
         if (kernel_ms) *kernel_ms = h->last_persist ? h->last_persist_ms : 0.0;
+    });
+}
+
+int csl_mixed_last_variant(csl_mixed* h, int* variant) {
+    return guarded([&] {
+        check_mixed(h);
+        if (variant) *variant = h->last_variant;
     });
 }
 

@@ -143,6 +143,8 @@ struct MixPersistShape {
     bool waves;  // one unit of 64 sites of one species per wave (csl_mixed_waves.hip)
 };
 MixPersistShape mixed_persist_shape(const MixDev& M, bool tt);
+// Its variant, CSL_MIXED_VARIANT_* bits.
+int mixed_persist_variant(const MixDev& M, const MixPersistShape& shape);
 // The one-unit-per-wave kernel: its LDS, and the launcher (arguments as
 // launch_mixed_persist).
 size_t mixed_waves_lds_bytes(const MixDev& M);

@@ -533,11 +533,13 @@ Lay persist_lay(const MixDev& M, int block, bool glds) {
     return mix_persist_lay(M.NP2, M.NP3, M.A2, M.A3, block / kWave, glds);
 }
 
-// components 6 and 7 in LDS where they fit: always up to 1024 sites of each
-// species (two units per wave of 512 threads, one of 1024)
+// Components 6 and 7 in LDS where they fit: always up to 1024 sites of each
+// species (two units per wave of 512 threads, one of 1024).
+Lay glds_lay(const MixDev& M, int block) { return Lay(M.NP2, M.NP3, M.A2, M.A3, block / kWave, true, false); }
+
 template <int SPT, int T, int Z22, int ZM, bool TT>
 hipError_t launch_mp_g(const MixDev& Mh, const MixDev* M, const MixPersistArgs& A, int grid, hipStream_t st, int* occ) {
-    const Lay in_lds(Mh.NP2, Mh.NP3, Mh.A2, Mh.A3, T / kWave, true, false);
+    const Lay in_lds = glds_lay(Mh, T);
     if (in_lds.total <= kMixLdsDoubles) return launch_mp<SPT, T, Z22, ZM, TT, true, false>(M, A, grid, in_lds, st, occ);
     if constexpr (SPT * T > 1024) {
         const Lay Y = persist_lay(Mh, T, false);
@@ -562,7 +564,7 @@ hipError_t launch_mp_z(const MixDev& Mh, const MixDev* M, const MixPersistArgs& 
 // Without SU(3)-SU(3) bonds: 1024 threads (4 waves per SIMD) and up to two
 // units of each species per wave — the SU(3) sites update in place, so a
 // thread holds only its accumulators and its SU(2) sites' next values.  With
-// them: 512 threads and up to four units (the SU(3) next values are held
+// them: 512 threads and two to four units (the SU(3) next values are held
 // too).  Lattices of at most 16 units (both species together) whose stage
 // values fit LDS twice take the one-unit-per-wave kernel.
 MixPersistShape mixed_persist_shape(const MixDev& M, bool tt) {
@@ -580,6 +582,14 @@ MixPersistShape mixed_persist_shape(const MixDev& M, bool tt) {
     return sh;
 }
 
+int mixed_persist_variant(const MixDev& M, const MixPersistShape& sh) {
+    if (!sh.block) return 0;
+    if (sh.waves) return CSL_MIXED_VARIANT_PERSISTENT | CSL_MIXED_VARIANT_UNIT_WAVES;
+    if (glds_lay(M, sh.block).total <= kMixLdsDoubles) return CSL_MIXED_VARIANT_PERSISTENT;
+    return CSL_MIXED_VARIANT_PERSISTENT | CSL_MIXED_VARIANT_GLOBAL_67 |
+           (persist_lay(M, sh.block, false).tight ? CSL_MIXED_VARIANT_TIGHT : 0);
+}
+
 hipError_t launch_mixed_persist(const MixDev& Mh, const MixDev* M, const MixPersistArgs& A, const MixPersistShape& sh,
                                 int grid, hipStream_t st, int* occ) {
     if (!sh.tt && sh.block == 1024) {
@@ -588,7 +598,6 @@ hipError_t launch_mixed_persist(const MixDev& Mh, const MixDev* M, const MixPers
     }
     if (sh.tt && sh.block == 512 && Mh.jz22 == 8 && Mh.jzm == 8) {
         switch (sh.spt) {
-            case 1: return launch_mp_g<1, 512, 8, 8, true>(Mh, M, A, grid, st, occ);
             case 2: return launch_mp_g<2, 512, 8, 8, true>(Mh, M, A, grid, st, occ);
             case 3: return launch_mp_g<3, 512, 8, 8, true>(Mh, M, A, grid, st, occ);
             case 4: return launch_mp_g<4, 512, 8, 8, true>(Mh, M, A, grid, st, occ);

@@ -142,12 +142,17 @@ class GPUMixedLattice:
     def last_path(self):
         """csl_mixed_last_path of the last integrate_batched:
         {"persistent": bool, "cooperative": bool, "workgroups": int, "split": int,
-        "kernel_ms": float} (split: trajectories run in two pieces by two
-        workgroups; kernel_ms: the persistent or cooperative launch)."""
+        "kernel_ms": float, "unit_waves": bool, "global_67": bool, "tight":
+        bool} (split: trajectories run in two pieces by two workgroups;
+        kernel_ms: the persistent or cooperative launch; the last three: the
+        variant of the persistent kernel, csl_mixed_last_variant)."""
         p, w, t, ms = C.c_int(), C.c_int(), C.c_size_t(), C.c_double()
         check(lib().csl_mixed_last_path(self.h, C.byref(p), C.byref(w), C.byref(t), C.byref(ms)))
+        v = C.c_int()
+        check(lib().csl_mixed_last_variant(self.h, C.byref(v)))
         return {"persistent": p.value == 1, "cooperative": p.value == 2, "workgroups": w.value,
-                "split": t.value, "kernel_ms": ms.value}
+                "split": t.value, "kernel_ms": ms.value, "unit_waves": bool(v.value & 2),
+                "global_67": bool(v.value & 4), "tight": bool(v.value & 8)}
 
     def normalize(self, len2=1.0, len3=1.0):
         check(lib().csl_mixed_normalize(self.h, len2, len3))

@@ -195,6 +195,17 @@ int csl_mixed_set_persistent(csl_mixed* h, int mode);
  * counterpart in the reference. */
 int csl_mixed_last_path(csl_mixed* h, int* persistent, int* workgroups, size_t* split, double* kernel_ms);
 
+/* Variant of the persistent kernel of the last csl_mixed_integrate_batched
+ * (0 where another path ran): bit 0 persistent, bit 1 one unit of 64 sites of
+ * one species per wave, bit 2 SU(3) components 6 and 7 in device memory, bit 3
+ * the tight tables of lattices with many sublattices.  No counterpart in the
+ * reference. */
+#define CSL_MIXED_VARIANT_PERSISTENT 1
+#define CSL_MIXED_VARIANT_UNIT_WAVES 2
+#define CSL_MIXED_VARIANT_GLOBAL_67 4
+#define CSL_MIXED_VARIANT_TIGHT 8
+int csl_mixed_last_variant(csl_mixed* h, int* variant);
+
 /* With enable != 0, csl_mixed_integrate_batched issues its launch sequence
  * (4 stage launches and one record reduction per step) from a hipGraph
  * captured on the first call and replayed by later calls with the same

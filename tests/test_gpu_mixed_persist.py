@@ -1,7 +1,9 @@
-"""GPU parity of the persistent batched kernel of the mixed SU(2) + SU(3)
-lattice (k_mixed_persist: one workgroup integrates one trajectory over the
-whole time grid, stage values in LDS plus two SU(3) components in global
-memory, x in the trajectory's state slot).
+"""GPU parity of the persistent batched kernels of the mixed SU(2) + SU(3)
+lattice: one workgroup integrates one trajectory over the whole time grid.
+The rich cells here (up to 3x2x2) run k_mixed_waves, one unit of 64 sites per
+wave; the 8x8x8 lattice k_mixed_persist, stage values in LDS plus two SU(3)
+components in global memory, x in the trajectory's state slot.  Every variant
+of the latter: test_gpu_mixed_variants.py.
 
 Bar: records and final states against the mixed oracle <= 1e-10 over <= 300
 steps with every term of the Hamiltonian, Gilbert and Bloch damping and both
