@@ -101,7 +101,7 @@ __device__ __forceinline__ void sweep_wave(double* smem, int wave, int wstart) {
     const double* const mats = K->L.mats + size_t(b) * K->A.mats_stride + atom * kZ * 9;
     const int n0 = K->A.n0, n1 = K->A.n1;  // stage slots q = 4 n + s of these steps
     const double* const Yb = K->A.Y + (size_t(b) * K->A.seg_len - K->A.y0) * 4 * SZ;
-    const double* const rows = K->A.rows + ((size_t(b) * (K->A.seg_len + 1) - K->A.y0) * n_atoms + atom) * kRow;
+    const double* const rows = K->A.rows + (size_t(b) * (K->A.seg_len + 1) * n_atoms + atom) * kRow;
 
     const int pbase = atom * npad + wstart * kWave + lane;
     int nb[NU][kZ];
@@ -418,7 +418,7 @@ __global__ void __launch_bounds__(256) k_adj_rows(LatDev L, AdjArgs A) {
     if (i >= n_seg * A.B * L.n_atoms) return;
     const int atom = int(i % L.n_atoms);
     const size_t n = A.n0 + i / L.n_atoms % n_seg, b = i / L.n_atoms / n_seg;
-    double* out = A.rows + ((b * (A.seg_len + 1) + n - A.y0) * L.n_atoms + atom) * kRow;
+    double* out = A.rows + ((b * (A.seg_len + 1) + n) * L.n_atoms + atom) * kRow;
     const double* B = L.field + b * A.field_stride + atom * 3;
     for (int sg = 0; sg < 3; ++sg) {
         double f[2] = {0.0, 0.0};

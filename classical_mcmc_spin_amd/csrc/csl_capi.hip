@@ -2531,6 +2531,7 @@ int csl_adjoint_gradient(csl_lattice* h, size_t B, const double* init, int init_
                 ++launches;
                 G.first = j == n_seg - 1 ? 1 : 0;
                 if (sweep) {
+                    G.rows = h->adj_rows.p - size_t(G.y0) * csl::adjoint_row_doubles(L);
                     hip_check(csl::launch_adjoint_rows(L, G, s), "k_adj_rows launch");
                     hip_check(csl::launch_adjoint_sweep(L, G, s), "k_adj_sweep launch");
                     launches += 2;

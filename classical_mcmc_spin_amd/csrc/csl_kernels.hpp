@@ -156,7 +156,8 @@ struct AdjArgs {
     double* rec;               // [n_steps+1][B][9] forward records
     double* loss_n;            // [B][n_steps+1] loss term of every record
     double* part;              // [B][n_steps][4][P] parameter-gradient term of every stage (sweep: thread sums)
-    double* rows;              // sweep: fields and loss cotangents of a segment's steps [B][seg_len + 1]
+    double* rows;              // sweep: fields and loss cotangents of a segment's steps, step n of trajectory b at
+                               // row b * (seg_len + 1) + n (the pointer is where step 0 would be)
     double* grad_init;         // [B][N*3] dL/dx_0 (AoS), written by the launch with n0 == 0, or null
     double* loss;              // [B] (final kernel)
     double* grad;              // [B][P] (final kernel)
