@@ -91,7 +91,7 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
     // sites and fewer unpacking costs 7 %).
     constexpr bool kPack = ZMAX > 6 && SPT > 2;
     constexpr int kWords = kPack ? (ZMAX + 1) / 2 : ZMAX;
-    unsigned nb[NU][kWords];
+    int nb[NU][kWords];
 #pragma unroll
     for (int m = 0; m < NU; ++m) {
         // padding lanes (no cell) hold a zero spin and gather themselves:
@@ -99,17 +99,15 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
         const int p = pbase + m * kWave;
         const bool real = p - atom * npad < K.L.n_cells;
 #pragma unroll
-        for (int k = 0; k < kWords; ++k) nb[m][k] = 0;
-#pragma unroll
         for (int k = 0; k < ZMAX; ++k) {
-            const unsigned q = real ? K.L.col[size_t(k) * NP + p] : p;
-            if constexpr (kPack) nb[m][k >> 1] |= q << (16 * (k & 1));
-            else nb[m][k] = q;
+            const int q = real ? K.L.col[size_t(k) * NP + p] : p;
+            if constexpr (!kPack) nb[m][k] = q;
+            else nb[m][k >> 1] = k & 1 ? nb[m][k >> 1] | q << 16 : q;
         }
     }
     auto nbr = [&](int m, int k) {
-        if constexpr (kPack) return int((unsigned(fresh(int(nb[m][k >> 1]))) >> (16 * (k & 1))) & 0xffffu);
-        else return int(nb[m][k]);
+        if constexpr (kPack) return int((unsigned(fresh(nb[m][k >> 1])) >> (16 * (k & 1))) & 0xffffu);
+        else return nb[m][k];
     };
     const double dt = K.A.dt;
     const double b16 = (1.0 / 6.0) * dt, b13 = (1.0 / 3.0) * dt, hdt = 0.5 * dt;
