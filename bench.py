@@ -223,9 +223,10 @@ def bench_2dcs(args):
     roof = fp64_roofline("k_trajectory", flops_launch, kms,
                          algorithmic_flops_per_site_step=FLOPS_Z3 + FLOPS_DRIVE,
                          hbm_algorithmic_frac=site_steps * BYTES_PER_SITE_STEP / (kms * 1e-3) / HBM_PEAK)
-    roof["traffic"] = profile_number("traffic_k_persistent_2dcs_36x36.txt", "traffic_bytes_per_launch")
+    counters = "counters_k_trajectory_2dcs_36x36.txt"
+    roof["traffic"] = profile_number(counters, "traffic_bytes_per_launch")
     for key in ("valu_issue_frac", "lds_busy_frac"):
-        v = profile_number("counters_k_persistent_2dcs_36x36.txt", key)
+        v = profile_number(counters, key)
         if v is not None:
             roof[key] = v
     line = {
@@ -461,7 +462,7 @@ def bench_pyrochlore(args):
     site_steps = PYRO_B * N * PYRO_STEPS
     roof = fp64_roofline("k_partitioned", site_steps * FLOPS_Z6, kms, algorithmic_flops_per_site_step=FLOPS_Z6,
                          hbm_algorithmic_bytes_per_launch=site_steps * BYTES_PER_SITE_STEP)
-    roof["traffic"] = profile_number("traffic_k_partitioned_pyrochlore_16x16x16.txt", "traffic_bytes_per_launch")
+    roof["traffic"] = profile_number("counters_k_partitioned_pyrochlore_16x16x16.txt", "traffic_bytes_per_launch")
     stage_roof = hbm_roofline("k_stage", PYRO_B * N * BYTES_PER_SITE_STEP / 4, kms_st)  # one RK stage of every site
     stage_roof["traffic"] = profile_number("traffic_l2_k_stage_pyrochlore_16x16x16.txt", "traffic_bytes_per_launch")
     out = {
@@ -493,13 +494,14 @@ def bench_pyrochlore(args):
 
 ADJ_L, ADJ_STEPS, ADJ_B, ADJ_B_FULL = 24, 2000, 32, 256
 # Algorithmic FP64 flops per site-step of one gradient (z = 3, Gilbert
-# damping, pulse drive, 5 parameters): forward RK4 with records 465 (its
-# stage inputs are kept, so nothing is integrated twice), transposed step
-# 2119 (per stage: field at the stage input 69, H x S and the Gilbert factor
-# 16, the cotangent map w, u 24, the direct term 46, the transposed bond
-# gather 54, five parameter derivatives u . (sum dJ S - dB) 310,
-# combinations 10; plus the loss term 3).
-ADJ_FLOPS_PER_SITE_STEP = 465 + 2119
+# damping, pulse drive): forward RK4 with records 465 (its stage inputs are
+# kept, so nothing is integrated twice), transposed step 1107 (per stage: field
+# at the stage input 69, H x S and the Gilbert factor 16, the cotangent map w,
+# u 24, the direct term 46, the transposed bond gather 54, the sums of u (x) S
+# of three bonds and of u 57, which are contracted with the parameters'
+# matrices once at the end, combinations 10; plus the loss term 3).  The
+# sweep's counters give 1099 executed.
+ADJ_FLOPS_PER_SITE_STEP = 465 + 1107
 # mixed TmFeO3 cell, per (SU(2) + SU(3)) site pair and RK4 step: SU(2) site
 # 2A S 18, 6 SU(2) bonds 108, 8 SU(3) bonds 384, drive 12, H x S 9, update 12
 # = 543; SU(3) site 8 SU(2) bonds 384, drive 32, f_abc 108, update 32 = 556
@@ -595,8 +597,8 @@ def bench_adjoint(args):
         "max_rel_err_vs_oracle_tangent_linear": err,
         "roofline": fp64_roofline("k_adj_fwd + k_adj_sweep", ADJ_B * N * ADJ_STEPS * ADJ_FLOPS_PER_SITE_STEP,
                                   kms, algorithmic_flops_per_site_step=ADJ_FLOPS_PER_SITE_STEP,
-                                  note=f"forward and backward sweeps: one workgroup per start ({ADJ_B} of the 256 CUs); "
-                                       "parameter terms on the other CUs, overlapped with the sweep"),
+                                  note=f"forward and backward sweeps: one workgroup per start ({ADJ_B} of the 256 CUs), "
+                                       "the parameter terms summed in the sweep"),
         "starts_256": {"gradients_per_s": ADJ_B_FULL / el_full, "kernel_ms": kms_full,
                        "fp64_frac": ADJ_B_FULL * N * ADJ_STEPS * ADJ_FLOPS_PER_SITE_STEP / (kms_full * 1e-3)
                        / FP64_PEAK},
@@ -710,7 +712,7 @@ def bench_mixed(args):
     n_sites = ml.N2 + ml.N3
     roof = fp64_roofline("k_mixed_persist", MIX_FLOPS_PAIR_STEP * ml.N2 * B * MIX_STEPS, kms,
                          algorithmic_flops_per_pair_step=MIX_FLOPS_PAIR_STEP, trajectories_in_launch=B)
-    roof["traffic"] = profile_number("traffic_k_mixed_persist_tmfeo3_8x8x8.txt", "traffic_bytes_per_launch")
+    roof["traffic"] = profile_number("counters_k_mixed_persist_tmfeo3_8x8x8.txt", "traffic_bytes_per_launch")
     bytes_stage = B * (ml.N2 * 3 + ml.N3 * 8) * 2 * 8   # one stage: read + write of every component
     stage_roof = hbm_roofline("k_mixed_stage", bytes_stage, kms_st)
     stage_roof["traffic"] = profile_number("traffic_l2_k_mixed_stage_tmfeo3_8x8x8.txt", "traffic_bytes_per_launch")

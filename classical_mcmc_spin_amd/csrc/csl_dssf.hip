@@ -7,9 +7,9 @@
 // the cell's lattice vectors, which are orthonormal for the cubic
 // pyrochlore cell).  Lattices of one workgroup integrate on the persistent
 // kernel, which leaves the samples behind; larger ones on the stage kernels,
-// sample by sample.  The spins of every (trajectory, atom,
+// sample by sample (csl_dssf_route.hpp).  The spins of every (trajectory, atom,
 // component) are expanded into a complex 3-D grid over the cells, batched
-// 3-D FFTs (hipFFT) gives F_a,atom(q), and k_sq_combine sums the atoms with
+// 3-D FFTs (hipFFT) give F_a,atom(q), and k_sq_combine sums the atoms with
 // their position phases into the S(q, t) buffer; after the run a batched
 // 1-D FFT along t and k_sq_power give S(q, w).  The reference post-processes
 // saved spin snapshots in Python (util/readers_new/reader_pyrochlore.py:150-270).

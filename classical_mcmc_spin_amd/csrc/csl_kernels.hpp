@@ -280,9 +280,9 @@ constexpr int kPersistMulti = 4;         // per-trajectory lattices (PersistArgs
 // shape (reported by csl_persistent_candidates; the launcher applies the same
 // rule): FIELD_ONLY for double-buffered, stage-unrolled shapes of lattices
 // with translation-invariant tables, per-sublattice fields, no onsite matrix
-// and full coordination; ATOM_MAJOR in addition when the block tiles the
-// sublattices (npad = waves_per_atom * 64 * SPT, block = n_atoms *
-// waves_per_atom * 64).
+// and full coordination; ATOM_MAJOR in addition when every wave of the block
+// lies in one sublattice and owns spt or spt - 1 of its units of 64 cells
+// (atom_major_tile) and the tables fit LDS: those shapes run k_trajectory.
 constexpr int kVariantFieldOnly = 1;
 constexpr int kVariantAtomMajor = 2;
 constexpr int kVariantPartitioned = 4;  // reported for launches of the partitioned kernel

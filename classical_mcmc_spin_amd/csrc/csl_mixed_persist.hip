@@ -32,8 +32,9 @@
 // with many sublattices keep smaller tables (TIGHT, csl_mixed_lay.hpp).  With
 // every record's 33 wave sums in shuffles, an envelope evaluation per wave
 // and stage, one 4-byte partner load per bond and one 8-byte access per
-// component a stage of the 8x8x8 cell took 36.8 us; it takes 28 (a third of
-// the cycles issue FP64 work; x from global memory costs 3.6 of them).
+// component a stage of the 8x8x8 cell took 36.8 us; it takes 27 (0.28 of the
+// SIMD cycles issue FP64 work, 0.42 anything; x from global memory costs 3.6
+// us; 5.4 TB/s of x, components 6 and 7 and partner words leave the L2s).
 #include <algorithm>
 #include <type_traits>
 
