@@ -190,7 +190,9 @@ __global__ void __launch_bounds__(dopri5_max_block<SPT>()) k_dopri5(LatDev Lk, D
     // factors f1, f2 (zero when the drive is off); with obs, the observable
     // partials of that state go to red[] (all lanes of every wave must take
     // part).
-    auto rhs = [&](const LdsState& cur, double f1, double f2, double (&k)[SPT][3], bool obs)
+    // late (FIELD_ONLY): a state that may be recorded; its drive comes after
+    // the energy (a driven field would round at the drive's size).
+    auto rhs = [&](const LdsState& cur, double f1, double f2, double (&k)[SPT][3], bool obs, bool late)
                    __attribute__((always_inline)) {
         const LatDev L = refresh(L0);
         // LDS indices offset by an opaque zero: the address arithmetic is
@@ -199,15 +201,15 @@ __global__ void __launch_bounds__(dopri5_max_block<SPT>()) k_dopri5(LatDev Lk, D
         const int zz = opaque_zero();
         if constexpr (FIELD_ONLY) {
             cptr<double> B = as_const(L.field) + atom_w * 3;
-            double h0[3] = {-B[0], -B[1], -B[2]}, hb[3] = {-B[0], -B[1], -B[2]};
+            const double hb[3] = {-B[0], -B[1], -B[2]};
+            double h0[3] = {hb[0], hb[1], hb[2]}, D[3] = {0.0, 0.0, 0.0};
             if (drive_on && (f1 != 0.0 || f2 != 0.0)) {
                 cptr<double> d0 = as_const(L.fdrive) + atom_w * 3;
                 cptr<double> d1 = as_const(L.fdrive) + (L.n_atoms + atom_w) * 3;
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
-                    const double D = d0[d] * f1 + d1[d] * f2;
-                    h0[d] -= D;
-                    hb[d] += D;
+                    D[d] = d0[d] * f1 + d1[d] * f2;
+                    if (!late) h0[d] -= D[d];
                 }
             }
             double H[SPT][3];
@@ -237,6 +239,10 @@ __global__ void __launch_bounds__(dopri5_max_block<SPT>()) k_dopri5(LatDev Lk, D
                         sm[d] += S[d];
                         e = fma(S[d], 0.5 * (H[m][d] + hb[d]), e);
                     }
+                }
+                if (late) {
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) H[m][d] -= D[d];
                 }
                 ll_su2_guarded(H[m], S, alpha, k[m]);
             }
@@ -334,7 +340,7 @@ __global__ void __launch_bounds__(dopri5_max_block<SPT>()) k_dopri5(LatDev Lk, D
             for (int d = 0; d < 3; ++d) y[m][d] = x[m][d] + h * kA21 * k1[m][d];
         store_stage(bufB, y);
         __syncthreads();
-        rhs(bufB, f(0, 0), f(0, 1), k2, false);
+        rhs(bufB, f(0, 0), f(0, 1), k2, false, false);
         // stage 3
 #pragma unroll
         for (int m = 0; m < SPT; ++m)
@@ -342,7 +348,7 @@ __global__ void __launch_bounds__(dopri5_max_block<SPT>()) k_dopri5(LatDev Lk, D
             for (int d = 0; d < 3; ++d) y[m][d] = x[m][d] + h * (kA31 * k1[m][d] + kA32 * k2[m][d]);
         store_stage(bufA, y);
         __syncthreads();
-        rhs(bufA, f(1, 0), f(1, 1), k3, false);
+        rhs(bufA, f(1, 0), f(1, 1), k3, false, false);
         // stage 4
 #pragma unroll
         for (int m = 0; m < SPT; ++m)
@@ -351,7 +357,7 @@ __global__ void __launch_bounds__(dopri5_max_block<SPT>()) k_dopri5(LatDev Lk, D
                 y[m][d] = x[m][d] + h * (kA41 * k1[m][d] + kA42 * k2[m][d] + kA43 * k3[m][d]);
         store_stage(bufB, y);
         __syncthreads();
-        rhs(bufB, f(2, 0), f(2, 1), k4, false);
+        rhs(bufB, f(2, 0), f(2, 1), k4, false, false);
         // stage 5
 #pragma unroll
         for (int m = 0; m < SPT; ++m)
@@ -360,7 +366,7 @@ __global__ void __launch_bounds__(dopri5_max_block<SPT>()) k_dopri5(LatDev Lk, D
                 y[m][d] = x[m][d] + h * (kA51 * k1[m][d] + kA52 * k2[m][d] + kA53 * k3[m][d] + kA54 * k4[m][d]);
         store_stage(bufA, y);
         __syncthreads();
-        rhs(bufA, f(3, 0), f(3, 1), k5, false);
+        rhs(bufA, f(3, 0), f(3, 1), k5, false, false);
         // stage 6 (k6 lives in y's registers after the store)
 #pragma unroll
         for (int m = 0; m < SPT; ++m)
@@ -371,7 +377,7 @@ __global__ void __launch_bounds__(dopri5_max_block<SPT>()) k_dopri5(LatDev Lk, D
         store_stage(bufB, y);
         __syncthreads();
         double k6[SPT][3];
-        rhs(bufB, f(4, 0), f(4, 1), k6, false);
+        rhs(bufB, f(4, 0), f(4, 1), k6, false, false);
         // candidate and the error weights without k7
         double ep[SPT][3];
 #pragma unroll
@@ -384,7 +390,7 @@ __global__ void __launch_bounds__(dopri5_max_block<SPT>()) k_dopri5(LatDev Lk, D
             }
         store_stage(bufA, xn);
         __syncthreads();
-        rhs(bufA, f(5, 0), f(5, 1), k7, obs);
+        rhs(bufA, f(5, 0), f(5, 1), k7, obs, true);
         double e = 0.0;
         if (control != 0) {
             const double ah = fabs(h);
@@ -450,7 +456,7 @@ __global__ void __launch_bounds__(dopri5_max_block<SPT>()) k_dopri5(LatDev Lk, D
         if (need_eval) {
             const bool ob = eobs && (obs_calls % si) == 0;
             const double fl = drive_on && lane < 2 ? lane_drive(te) : 0.0;
-            rhs(bufA, drive_on ? readlane_f64(fl, 0) : 0.0, drive_on ? readlane_f64(fl, 1) : 0.0, k1, ob);
+            rhs(bufA, drive_on ? readlane_f64(fl, 0) : 0.0, drive_on ? readlane_f64(fl, 1) : 0.0, k1, ob, true);
             __syncthreads();
             if (ob) publish(saved++, te);
             if (eobs) ++obs_calls;

@@ -66,7 +66,7 @@ __device__ __forceinline__ void end_bond(double (&H)[D]) {
 // at a time.
 struct MixTables {
     double* cst;   // [rows][3]: B, d0, d1 of every field component
-    double* hin;   // [2 step parity][4][rows]: -(B + drive) at the three stage times, and the first plus 2B
+    double* hin;   // [2 step parity][4][rows]: the drive at the step's start, -(B + drive) at its middle and end, -B
     double* drv;   // [2 chunk parity][chunk][3 stage times][2 species][2 pulses]
     double* red;   // record sums
     int rows;      // 3 A2 + 8 A3
@@ -92,8 +92,8 @@ __device__ __forceinline__ void mix_fill_tables(cptr<MixDev> M, const MixTables&
         Q.cst[3 * i] = r.B;
         Q.cst[3 * i + 1] = r.d0;
         Q.cst[3 * i + 2] = r.d1;
-        for (int par = 0; par < 2; ++par)  // without a drive the rows stay -B (and -B + 2B)
-            for (int st = 0; st < 4; ++st) Q.hin[(par * 4 + st) * R + i] = st < 3 ? -r.B : r.B;
+        for (int par = 0; par < 2; ++par)  // without a drive the rows stay 0 and -B
+            for (int st = 0; st < 4; ++st) Q.hin[(par * 4 + st) * R + i] = st ? -r.B : 0.0;
     }
 }
 
@@ -118,26 +118,25 @@ __device__ __forceinline__ void mix_write_drive(const MixTables& Q, int b, int n
     Q.drv[cp * 12 * chunk + lane] = v;
 }
 
-// Field rows of the step whose envelopes are f[0..11].
+// Field rows 0 to 2 of the step whose envelopes are f[0..11].
 __device__ __forceinline__ void mix_write_hin(const MixTables& Q, const double* f, int par, int n2, int tid, int T) {
     const int R = Q.rows;
-    for (int i = tid; i < 4 * R; i += T) {
-        const int st = i / R, r = i - st * R, q = st == 3 ? 0 : st, s3 = r < n2 ? 0 : 2;
-        const double D = Q.cst[3 * r + 1] * f[q * 4 + s3] + Q.cst[3 * r + 2] * f[q * 4 + s3 + 1];
-        Q.hin[par * 4 * R + i] = st == 3 ? Q.cst[3 * r] - D : -Q.cst[3 * r] - D;
+    for (int i = tid; i < 3 * R; i += T) {
+        const int st = i / R, r = i - st * R, s3 = r < n2 ? 0 : 2;
+        const double D = Q.cst[3 * r + 1] * f[st * 4 + s3] + Q.cst[3 * r + 2] * f[st * 4 + s3 + 1];
+        Q.hin[par * 4 * R + i] = st ? -Q.cst[3 * r] - D : D;
     }
 }
 
-// One row st of the one set of rows of the tight layout (csl_mixed_lay.hpp):
-// -(B + drive) at the st-th stage time, st 3 the first plus 2B; f null: no drive.
+// One row st of the one set of rows of the tight layout (csl_mixed_lay.hpp);
+// f null: no drive.
 __device__ __forceinline__ void mix_write_row(cptr<MixDev> M, const MixTables& Q, const double* f, int st, int n2, int tid,
                                               int T) {
-    const int q = st == 3 ? 0 : st;
     for (int i = tid; i < Q.rows; i += T) {
         const MixRow r = mix_row(M, i);
         const int s3 = i < n2 ? 0 : 2;
-        const double D = f ? r.d0 * f[q * 4 + s3] + r.d1 * f[q * 4 + s3 + 1] : 0.0;
-        Q.hin[st * Q.rows + i] = st == 3 ? r.B - D : -r.B - D;
+        const double D = f && st < 3 ? r.d0 * f[st * 4 + s3] + r.d1 * f[st * 4 + s3 + 1] : 0.0;
+        Q.hin[st * Q.rows + i] = st ? -r.B - D : D;
     }
 }
 

@@ -27,7 +27,7 @@
 // a stage of the 8x8x8 cell).
 //
 // Field rows, pulse envelopes and records are handled as in
-// csl_trajectory.hip: rows of -(B + drive) from LDS, envelopes of two steps
+// csl_trajectory.hip: field rows from LDS, envelopes of two steps
 // at a time, records from the waves' sums of S and S.H, two at a time; lattices
 // with many sublattices keep smaller tables (TIGHT, csl_mixed_lay.hpp).  With
 // every record's 33 wave sums in shuffles, an envelope evaluation per wave
@@ -241,20 +241,17 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
         auto write_hin = [&](const double* f, int par) {
             if (!drive) return;
             if constexpr (TIGHT)
-                for (int st = 0; st < 4; ++st) mix_write_row(M0, Q, f, st, 3 * A2, tid, T);
+                for (int st = 0; st < 3; ++st) mix_write_row(M0, Q, f, st, 3 * A2, tid, T);
             else
                 mix_write_hin(Q, f, par, 3 * A2, tid, T);
         };
         // TIGHT: the rows of the step before are replaced one by one as they
-        // have been read: 0 and 3 by stage 0, 1 by stage 2, 2 by stage 3 (its
+        // have been read: 0 by stage 0, 1 by stage 2, 2 by stage 3 (its
         // successor is written in stage 1 of its own step)
         auto replace_rows = [&](int s, const double* f, const double* f_next, bool more) {
             if (!drive) return;
             if (s == 1) mix_write_row(M0, Q, f, 2, 3 * A2, tid, T);
-            if (s == 2 && more) {
-                mix_write_row(M0, Q, f_next, 0, 3 * A2, tid, T);
-                mix_write_row(M0, Q, f_next, 3, 3 * A2, tid, T);
-            }
+            if (s == 2 && more) mix_write_row(M0, Q, f_next, 0, 3 * A2, tid, T);
             if (s == 3 && more) mix_write_row(M0, Q, f_next, 1, 3 * A2, tid, T);
         };
         auto field_b = [&](int i) { return TIGHT ? mix_row(M0, i).B : Q.cst[3 * i]; };
@@ -304,8 +301,8 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
             const double cdt = s == 2 ? dt : 0.5 * dt;
             const double bdt = (s == 0 || s == 3) ? (1.0 / 6.0) * dt : (1.0 / 3.0) * dt;
             const int set = TIGHT ? 0 : par * 4;
-            const double* hrow = Q.hin + (set + (s == 0 ? 0 : (s == 3 ? 2 : 1))) * R;
-            const double* wrow = Q.hin + (set + 3) * R;
+            const double* hrow = Q.hin + (set + (s == 0 ? 3 : (s == 3 ? 2 : 1))) * R;
+            const double* drow = Q.hin + set * R;   // stage 0: the drive, after the record's undriven energy
             const Field<Z22, ZM, GLDS> F{Mg, smem, Y, GLDS ? nullptr : Gw + (s & 1) * GS};
             double2* const Gn = GLDS ? nullptr : Gw + (1 - (s & 1)) * GS;
             double e = 0.0;
@@ -324,8 +321,12 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
                 F.fe(a, p, S, H);
                 if (slot >= 0) {
 #pragma unroll
-                    for (int d = 0; d < 3; ++d) e = fma(S[d], H[d] - wrow[3 * a + d], e);
+                    for (int d = 0; d < 3; ++d) e = fma(S[d], H[d] + hrow[3 * a + d], e);
                     sums2(slot, j, S);
+                }
+                if (s == 0) {
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) H[d] -= drow[3 * a + d];
                 }
                 double k[3];
                 ll_mixed_su2(H, S, M->alpha, k);
@@ -361,10 +362,14 @@ __global__ void __launch_bounds__(T) k_mixed_persist(MixKernArgs K) {
                         for (int c = 0; c < 8; ++c) H[d] = fma(A3m[d * 8 + c], S[c], H[d]);
                 }
                 if (slot >= 0) {
-                    const double* w = wrow + 3 * A2 + 8 * a;
 #pragma unroll
-                    for (int d = 0; d < 8; ++d) e = fma(S[d], H[d] - w[d], e);
+                    for (int d = 0; d < 8; ++d) e = fma(S[d], H[d] + hr[d], e);
                     sums3(slot, j, S);
+                }
+                if (s == 0) {
+                    const double* dr = drow + 3 * A2 + 8 * a;
+#pragma unroll
+                    for (int d = 0; d < 8; ++d) H[d] -= dr[d];
                 }
                 double k[8];
                 su3_cross(H, S, k);

@@ -263,7 +263,7 @@ __device__ __forceinline__ void run_unit(const MixKernArgs& K, double* smem, con
 
         auto stage = [&](auto s_, int par, int slot) {
             constexpr int s = decltype(s_)::value;
-            constexpr int st = s == 0 ? 0 : (s == 3 ? 2 : 1);
+            constexpr int st = s == 0 ? 3 : (s == 3 ? 2 : 1);
             const double cdt = s == 2 ? dt : 0.5 * dt;
             const double bdt = (s == 0 || s == 3) ? b16 : b13;
             const cptr<MixDev> M = as_const(Mg) + opaque_zero();
@@ -276,12 +276,17 @@ __device__ __forceinline__ void run_unit(const MixKernArgs& K, double* smem, con
             for (int d = 0; d < D; ++d) H[d] = h[d];
             sp.field(M, Y, cur, a, p, S, H);
             if (s == 0 && slot >= 0) {
-                // S.(H - (hin + 2B)) = S.(H_undriven - B): twice the energy
-                const double* w = Q.hin + (par * 4 + 3) * R + row0;
+                // S.(H - B) of the undriven field: twice the energy
                 double e = 0.0;
 #pragma unroll
-                for (int d = 0; d < D; ++d) e = fma(S[d], H[d] - w[d], e);
+                for (int d = 0; d < D; ++d) e = fma(S[d], H[d] + h[d], e);
                 reduce_obs(slot, S, e);
+            }
+            if constexpr (s == 0) {
+                // the drive after the record (a driven field would round at the drive's size)
+                const double* dr = Q.hin + par * 4 * R + row0;
+#pragma unroll
+                for (int d = 0; d < D; ++d) H[d] -= dr[d];
             }
             double k[D];
             sp.rhs(M, p, real, H, S, k);

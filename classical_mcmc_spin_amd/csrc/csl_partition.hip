@@ -388,17 +388,11 @@ __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0
             if constexpr (AM) {
                 const int atom = atm[0];
                 cptr<double> B = as_const(L.field) + atom * 3;
-                double h0[3] = {-B[0], -B[1], -B[2]}, hb0[3] = {-B[0], -B[1], -B[2]};
-                if (drive_now) {
-                    cptr<double> d0 = as_const(L.fdrive) + atom * 3;
-                    cptr<double> d1 = as_const(L.fdrive) + (L.n_atoms + atom) * 3;
-#pragma unroll
-                    for (int d = 0; d < 3; ++d) {
-                        const double D = d0[d] * f1 + d1[d] * f2;
-                        h0[d] -= D;
-                        hb0[d] += D;
-                    }
-                }
+                const double hb0[3] = {-B[0], -B[1], -B[2]};
+                double h0[3] = {hb0[0], hb0[1], hb0[2]};
+                // stage 0 takes the drive after the record's energy (a driven
+                // field would round at the drive's size)
+                if (s > 0 && drive_now) sub_drive(L, atom, f1, f2, h0);
                 double H[SPT][3];
 #pragma unroll
                 for (int m = 0; m < SPT; ++m)
@@ -430,6 +424,7 @@ __global__ void __launch_bounds__(part_max_block<SPT>()) k_partitioned(LatDev L0
                                 e = fma(S[d], 0.5 * (H[m][d] + hb0[d]), e);
                             }
                         }
+                        if (drive_now) sub_drive(L, atom, f1, f2, H[m]);
                     } else {
                         Y.load(fresh(cur * n_loc + q0 + m * qs), S);
                     }

@@ -13,7 +13,7 @@
 // one gather, the field, the update, one store and one barrier.
 //
 // Everything that is not one of those four things is taken out of the stage:
-//   * the field's constant part -(B + drive) of the three stage times comes
+//   * the field's constant part -(B + drive) of the stage times comes
 //     from a small LDS table (one row per sublattice), written one step
 //     ahead by the first waves; the pulse envelopes themselves are evaluated
 //     for a chunk of steps at once, one lane per (step, stage time, pulse);
@@ -66,8 +66,8 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
     // at 36x36), then the small tables
     double* const coef = smem + 6 * NP;          // [n_atoms][10][4] record weights of a wave's sums
     double* const cst = coef + 40 * n_atoms;     // [n_atoms][3][3]: B, d0, d1 of each component
-    double* const hin = cst + 9 * n_atoms;       // [2 step parity][4][n_atoms][3]: -(B + drive) at the three
-                                                 // stage times, and that of the first plus 2B
+    double* const hin = cst + 9 * n_atoms;       // [2 step parity][4][n_atoms][3]: the drive at the step's start,
+                                                 // -(B + drive) at its middle and end, -B
     double* const drv = hin + 24 * n_atoms;      // [2 chunk parity][C][6] pulse envelopes
     double* const red = drv + 12 * C;            // [C][nwaves][4] record sums of the waves
     auto lds_ld = [&](int which, int q, double S[3]) {
@@ -168,20 +168,21 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
             cst[3 * i] = field[i];
             cst[3 * i + 1] = K.L.fdrive[i];
             cst[3 * i + 2] = K.L.fdrive[3 * n_atoms + i];
-            for (int par = 0; par < 2; ++par)  // without a drive the rows stay -B (and -B + 2B)
-                for (int st = 0; st < 4; ++st) hin[(par * 4 + st) * 3 * n_atoms + i] = st < 3 ? -field[i] : field[i];
+            for (int par = 0; par < 2; ++par)  // without a drive the rows stay 0 and -B
+                for (int st = 0; st < 4; ++st) hin[(par * 4 + st) * 3 * n_atoms + i] = st ? -field[i] : 0.0;
         }
         for (int i = tid; i < 40 * n_atoms; i += T) {
             // out[j] = sum over waves of coef[atom][j] . (Sx, Sy, Sz, e):
-            // staggered, local and global magnetisation, energy
+            // staggered, local and global magnetisation, energy: e = S.H with
+            // the undriven H = -B + sum J S, so 1/2 (e - B.S)
             const int a = i / 40, j = (i / 4) % 10, e = i & 3;
             const int d = j % 3;
             double v = 0.0;
             if (e < 3 && j < 9) {
                 v = j < 3 ? K.L.afm[a] * K.L.frames[a * 9 + d * 3 + e]
                           : (j < 6 ? (d == e ? 1.0 : 0.0) : K.L.frames[a * 9 + d * 3 + e]);
-            } else if (e == 3 && j == 9) {
-                v = 0.5;
+            } else if (j == 9) {
+                v = e == 3 ? 0.5 : -0.5 * field[3 * a + e];
             }
             coef[i] = v;
         }
@@ -207,12 +208,11 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
         };
         // hin rows of the step whose envelopes are drv[f .. f+5]
         auto write_hin = [&](const double* f, int par) {
-            if (drive_on && tid < 12 * n_atoms) {
+            if (drive_on && tid < 9 * n_atoms) {
                 const int st = tid / (3 * n_atoms), i = tid - st * 3 * n_atoms;
                 const double B = cst[3 * i], d0 = cst[3 * i + 1], d1 = cst[3 * i + 2];
-                const int q = st == 3 ? 0 : st;
-                const double D = d0 * f[2 * q] + d1 * f[2 * q + 1];
-                hin[par * 12 * n_atoms + tid] = st == 3 ? B - D : -B - D;
+                const double D = d0 * f[2 * st] + d1 * f[2 * st + 1];
+                hin[par * 12 * n_atoms + tid] = st ? -B - D : D;
             }
         };
         write_drive(s_begin, 0);
@@ -264,12 +264,20 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
         auto stage = [&](auto s_, int par, int slot) {
             constexpr int s = decltype(s_)::value;
             constexpr int cur = s & 1, nxt = 1 - (s & 1);
-            constexpr int st = s == 0 ? 0 : (s == 3 ? 2 : 1);
+            constexpr int st = s == 0 ? 3 : (s == 3 ? 2 : 1);
             const double cdt = (s == 2) ? dt : hdt;
             const double bdt = (s == 0 || s == 3) ? b16 : b13;
             const double* h0 = hin + ((par * 4 + st) * n_atoms + atom) * 3;
             double H[NU][3];
             const double hx = h0[0], hy = h0[1], hz = h0[2];
+            // the drive of stage 0, read before the bonds where registers
+            // allow (24x24 2.5 % slower otherwise; 36x36 1.5 % with it)
+            double D[3] = {0.0, 0.0, 0.0};
+            auto load_drive = [&] {
+#pragma unroll
+                for (int d = 0; d < 3; ++d) D[d] = hin[(par * 4 * n_atoms + atom) * 3 + d];
+            };
+            if constexpr (s == 0 && kAhead) load_drive();
 #pragma unroll
             for (int m = 0; m < NU; ++m) {
                 H[m][0] = hx;
@@ -329,19 +337,25 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
                 for (int m = 0; m < NU; ++m) hold(H[m]);
             }
             if (s == 0 && slot >= 0) {
-                // e = sum S.H - (hin + 2B).S with the driven H: the undriven
-                // field's energy 1/2 S.(H - B) twice over
-                const double* w = hin + ((par * 4 + 3) * n_atoms + atom) * 3;
                 double sm[3] = {0.0, 0.0, 0.0}, e = 0.0;
 #pragma unroll
                 for (int m = 0; m < NU; ++m) {
 #pragma unroll
                     for (int d = 0; d < 3; ++d) {
                         sm[d] += x[m][d];
-                        e = fma(x[m][d], H[m][d] - w[d], e);
+                        e = fma(x[m][d], H[m][d], e);
                     }
                 }
                 reduce_obs(slot, sm, e);
+            }
+            if constexpr (s == 0) {
+                // the record's energy is the undriven field's: the drive comes
+                // after it (a driven field would round at the drive's size)
+                if constexpr (!kAhead) load_drive();
+#pragma unroll
+                for (int m = 0; m < NU; ++m)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) H[m][d] -= D[d];
             }
 #pragma unroll
             for (int m = 0; m < NU; ++m) {
@@ -454,7 +468,7 @@ __device__ __forceinline__ void run_wave(const TrajKernArgs& K, double* smem, in
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
                     sm[d] += x[m][d];
-                    e = fma(x[m][d], H[d] - field[atom * 3 + d], e);
+                    e = fma(x[m][d], H[d], e);
                 }
             }
             reduce_obs(0, sm, e);
